@@ -968,9 +968,103 @@ typedef uint32_t KzCandMask;
 typedef uint64_t KzCandMask;
 #endif
 
+// Coverage of a triangle relative to the square being drawn, in 32 bits
+// whatever the triangle's size: a sample at (dx, dy) sixteenths of a pixel
+// from the square's origin is inside iff a[k] * dx + b[k] * dy >= k[k] for
+// the edges E01, E12, E20 (interior-positive; k is the top-left threshold
+// less the edge's value at the origin). Vertices lie within the guard band
+// (|a|, |b| < 2^18) and dx, dy < 2^10, so the left side stays under 2^29 and
+// k clamped to +-2^30 decides the same. The raster is bound by instruction
+// issue, and 64-bit edge products per candidate pixel were most of it where
+// triangles are large: raster of 40,400 triangles around a camera (23 M
+// fragments) 1246 -> 1036 us, of 1,024 large ones at 256^2 204 -> 170, of
+// 4 M in 4,096 meshes 203 -> 194, of 8 M at 4K and four samples 1254 -> 1229;
+// a 1080p grid of 2 px triangles stays at 63.
+struct KzTileCov {
+    int32_t a[3], b[3], k[3];
+};
+
+// `narrow` (wave-uniform): every triangle that can have fragments here has
+// short edges and a pixel box that meets the square, so its values at the
+// origin fit 32 bits; the other lanes' wrap and are not used.
+__device__ __forceinline__ KzTileCov kz_tile_cov(const KzTri &t, int32_t X0, int32_t Y0, bool narrow) {
+    KzTileCov c;
+    const bool flip = t.S < 0;
+    c.a[0] = flip ? t.d1y : -t.d1y;
+    c.b[0] = flip ? -t.d1x : t.d1x;
+    c.a[2] = flip ? -t.d2y : t.d2y;
+    c.b[2] = flip ? t.d2x : -t.d2x;
+    c.a[1] = -c.a[0] - c.a[2];
+    c.b[1] = -c.b[0] - c.b[2];
+    const int32_t rx = X0 * 16 - t.x0, ry = Y0 * 16 - t.y0;
+    int32_t th[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) th[i] = (c.a[i] > 0 || (c.a[i] == 0 && c.b[i] > 0)) ? 0 : 1;
+    if (narrow) {
+        const uint32_t e0 = (uint32_t)__mul24(c.a[0], rx) + (uint32_t)__mul24(c.b[0], ry);
+        const uint32_t e2 = (uint32_t)__mul24(c.a[2], rx) + (uint32_t)__mul24(c.b[2], ry);
+        const uint32_t s = flip ? 0u - (uint32_t)(uint64_t)t.S : (uint32_t)(uint64_t)t.S;
+        c.k[0] = (int32_t)((uint32_t)th[0] - e0);
+        c.k[1] = (int32_t)((uint32_t)th[1] - (s - e0 - e2));
+        c.k[2] = (int32_t)((uint32_t)th[2] - e2);
+        return c;
+    }
+    const int64_t e0 = (int64_t)c.a[0] * rx + (int64_t)c.b[0] * ry;
+    const int64_t e2 = (int64_t)c.a[2] * rx + (int64_t)c.b[2] * ry;
+    const int64_t e[3] = {e0, (flip ? -t.S : t.S) - e0 - e2, e2};
+    const int64_t lim = 1 << 30;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int64_t k = th[i] - e[i];
+        c.k[i] = (int32_t)(k < -lim ? -lim : k > lim ? lim : k);
+    }
+    return c;
+}
+
+// the walk (KzWalk) of a box of width `width` whose first pixel is (px, py)
+// from the square's origin
+__device__ __forceinline__ void kz_tile_walk_init(KzWalk &w, const KzTileCov &c, int32_t px, int32_t py,
+                                                  int32_t width) {
+    const int32_t dx = px * 16 + kz_sample_x[0], dy = py * 16 + kz_sample_y[0];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        w.e[k] = (int32_t)((uint32_t)__mul24(c.a[k], dx) + (uint32_t)__mul24(c.b[k], dy) - (uint32_t)c.k[k]);
+        w.ax[k] = (int32_t)((uint32_t)c.a[k] << 4);
+        w.wy[k] = (int32_t)(((uint32_t)c.b[k] - (uint32_t)__mul24(width - 1, c.a[k])) << 4);
+#pragma unroll
+        for (int s = 0; s < KZ_SAMPLES; ++s)
+            w.o[k][s] =
+                __mul24(c.a[k], kz_sample_x[s] - kz_sample_x[0]) + __mul24(c.b[k], kz_sample_y[s] - kz_sample_y[0]);
+    }
+}
+
+// sample mask of the pixel (px, py) from the square's origin
+__device__ __forceinline__ uint32_t kz_tile_mask(const KzTileCov &c, int32_t px, int32_t py) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int s = 0; s < KZ_SAMPLES; ++s) {
+        const int32_t dx = px * 16 + kz_sample_x[s], dy = py * 16 + kz_sample_y[s];
+        int32_t v = 0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) v |= __mul24(c.a[k], dx) + __mul24(c.b[k], dy) - c.k[k];
+        m |= (v >= 0 ? 1u : 0u) << s;
+    }
+    return m;
+}
+
+__device__ __forceinline__ KzTileCov kz_tile_cov_of(const KzTileCov &c, uint32_t lane) {
+    KzTileCov o;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        o.a[k] = kz_readlane_i(c.a[k], lane);
+        o.b[k] = kz_readlane_i(c.b[k], lane);
+        o.k[k] = kz_readlane_i(c.k[k], lane);
+    }
+    return o;
+}
+
 struct KzLaneTri {
     KzTri t;
-    KzCov c;
     float a0[KZ_NVA], da1[KZ_NVA], da2[KZ_NVA];
     int32_t cx0, cy0, cx1, cy1;  // bbox ∩ tile
     bool live;
@@ -1015,15 +1109,40 @@ __device__ __forceinline__ void kz_ahead_indices(KzAhead &a, const KzFrame &f) {
     kz_triangle_indices(f, a.g, a.draw, a.idx);
 }
 
+// The fragment shader at a pixel centre whose edge values (E01, E20, E12 as
+// floats) are e01, e20, e12. Returns whether the fragment is kept; col is
+// clamped to [0, 1].
+__device__ __forceinline__ bool kz_shade(const KzFrame &f, int32_t px, int32_t py, float e01, float e20, float e12,
+                                         float invS, float z0, float dz1, float dz2, float iw0, float iw1, float iw2,
+                                         const float a0[KZ_NVA], const float da1[KZ_NVA], const float da2[KZ_NVA],
+                                         float col[4]) {
+    const float l0 = e12 * invS, l1 = e20 * invS, l2 = e01 * invS;
+    const float q = ((l0 * iw0) + (l1 * iw1)) + (l2 * iw2);
+    const float rq = 1.0f / q;
+    const float b1 = (l1 * iw1) * rq, b2 = (l2 * iw2) * rq;
+    float vary[KZ_NVA];
+#pragma unroll
+    for (int i = 0; i < KZ_NV; ++i) vary[i] = (a0[i] + b1 * da1[i]) + b2 * da2[i];
+    const float zc = fminf(fmaxf((z0 + l1 * dz1) + l2 * dz2, f.z_lo), f.z_hi);
+    const float frag_coord[4] = {(float)px + 0.5f, (float)py + 0.5f, zc, q};
+    const bool kept = kz_fragment(f, vary, frag_coord, col);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) col[c] = kz_clamp01(col[c]);
+    return kept;
+}
+
 // Resolves the fragment queue s_frag[0, total) of the batch held by the
 // wave's lanes (L), 64 fragments at a time: depth test and write, varyings,
 // fragment shader and blend, in primitive order per pixel. NARROW: every
-// triangle of the batch has short edges (32-bit edge values).
+// triangle of the batch has short edges (32-bit edge values; one copy for
+// both cases, with the test at run time, took 4 us more of a 1080p grid's
+// 63 us). A round none of whose fragments can pass the depth test ends
+// before the varyings are gathered.
 template <bool NARROW>
 __device__ __forceinline__ void kz_resolve(const KzFrame &f, const KzLaneTri &L, int32_t X0, int32_t Y0,
                                            uint32_t total, uint32_t lane, uint32_t *s_color, float *s_depth,
-                                           uint32_t *s_claim, const uint32_t *s_frag, unsigned long long &nfrag,
-                                           unsigned long long &npass) {
+                                           uint32_t *s_claim, const uint32_t *s_frag, uint32_t &nfrag,
+                                           uint32_t &npass) {
     for (uint32_t c0 = 0; c0 < total; c0 += 64) {
         const uint32_t qi = c0 + lane;
         const bool active = qi < total;
@@ -1042,12 +1161,10 @@ __device__ __forceinline__ void kz_resolve(const KzFrame &f, const KzLaneTri &L,
 
         float zs[KZ_SAMPLES];
         float c01 = 0.0f, c20 = 0.0f, c12 = 0.0f;  // one sample per pixel: it is the pixel centre
-        uint32_t nf = 0;
 #pragma unroll
         for (int s = 0; s < KZ_SAMPLES; ++s) {
             zs[s] = 0.0f;
             if ((mask >> s) & 1u) {
-                ++nf;
                 float e01, e20, e12;
                 kz_edges_f(NARROW, x0, y0, d1x, d1y, d2x, d2y, S, px * 16 + kz_sample_x[s],
                            py * 16 + kz_sample_y[s], e01, e20, e12);
@@ -1061,7 +1178,7 @@ __device__ __forceinline__ void kz_resolve(const KzFrame &f, const KzLaneTri &L,
                 zs[s] = fminf(fmaxf(z, f.z_lo), f.z_hi);
             }
         }
-        nfrag += nf;
+        nfrag += (uint32_t)__popc(mask);
 
         // The samples that can still pass the depth test: those that pass
         // against the depth the tile holds now. The round's earlier
@@ -1078,6 +1195,7 @@ __device__ __forceinline__ void kz_resolve(const KzFrame &f, const KzLaneTri &L,
             maybe = m;
         }
 #endif
+        if (kz_ballot(maybe != 0) == 0) continue;  // nothing of the round is visible
 
         // varyings at the pixel centre and the fragment shader
         float col[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -1095,20 +1213,10 @@ __device__ __forceinline__ void kz_resolve(const KzFrame &f, const KzLaneTri &L,
                 float e01 = c01, e20 = c20, e12 = c12;
                 if (KZ_SAMPLES != 1)
                     kz_edges_f(NARROW, x0, y0, d1x, d1y, d2x, d2y, S, px * 16 + 8, py * 16 + 8, e01, e20, e12);
-                const float l0 = e12 * invS, l1 = e20 * invS, l2 = e01 * invS;
-                const float q = ((l0 * iw0) + (l1 * iw1)) + (l2 * iw2);
-                const float rq = 1.0f / q;
-                const float b1 = (l1 * iw1) * rq, b2 = (l2 * iw2) * rq;
-                float vary[KZ_NVA];
-#pragma unroll
-                for (int i = 0; i < KZ_NV; ++i) vary[i] = (a0[i] + b1 * da1[i]) + b2 * da2[i];
-                const float zc = fminf(fmaxf((z0 + l1 * dz1) + l2 * dz2, f.z_lo), f.z_hi);
-                const float frag_coord[4] = {(float)px + 0.5f, (float)py + 0.5f, zc, q};
                 // a discarded fragment takes no part in the depth test,
                 // depth write or blend
-                if (!kz_fragment(f, vary, frag_coord, col)) maybe = 0;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) col[c] = kz_clamp01(col[c]);
+                if (!kz_shade(f, px, py, e01, e20, e12, invS, z0, dz1, dz2, iw0, iw1, iw2, a0, da1, da2, col))
+                    maybe = 0;
             }
         }
 
@@ -1307,15 +1415,15 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
         L.cy0 = max(L.t.py0, Y0);
         L.cy1 = min(L.t.py1, Y0 + RW - 1);
         L.live = ok && L.cx0 <= L.cx1 && L.cy0 <= L.cy1;
-        L.c = kz_cov_setup(L.t);
         const int32_t cw = L.cx1 - L.cx0 + 1;
         const int32_t cand = L.live ? cw * (L.cy1 - L.cy0 + 1) : 0;
-        // a triangle with few candidate pixels here and short edges: one lane
-        // walks its candidates (the others: the whole wave, one at a time)
-        const bool small = cand <= KZ_SMALL_CAND && L.c.small;
+        // a triangle with few candidate pixels here: one lane walks its
+        // candidates (the others: the whole wave, one at a time)
+        const bool small = cand <= KZ_SMALL_CAND;
         // every triangle of the batch that can have fragments here has short
-        // edges: the resolve evaluates edges in 32 bits
-        const bool narrow = kz_ballot(L.live && !L.c.small) == 0;
+        // edges: edges are evaluated in 32 bits
+        const bool narrow = kz_ballot(L.live && !kz_small_deltas(L.t.d1x, L.t.d1y, L.t.d2x, L.t.d2y)) == 0;
+        const KzTileCov lc = kz_tile_cov(L.t, X0, Y0, narrow);
 
         // --- phase 1: covered pixels per triangle ------------------------
         // (small triangles keep their sample masks, KZ_SAMPLES bits per
@@ -1332,7 +1440,7 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
             // those steps are dropped below), shifting each pixel's sign bit
             // (set: outside) in at bit 31, so that pixel j of maxc ends at bit
             // 32 - maxc + j: two instructions a pixel, no mask switching.
-            kz_walk_init(wk, L.t, L.c, L.cx0, L.cy0, cw);
+            kz_tile_walk_init(wk, lc, L.cx0 - X0, L.cy0 - Y0, cw);
             int32_t dx = 0;
             uint32_t out = 0;
             for (int32_t j = 0; j < maxc; ++j) {
@@ -1351,7 +1459,7 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
             // sample outside) shift in at the top of a 64-bit word, so that
             // pixel j of maxc (at most 16) ends at bits 4 (16 - maxc + j) ..
             // + 3; the count is of pixels with any sample covered.
-            kz_walk_init(wk, L.t, L.c, L.cx0, L.cy0, cw);
+            kz_tile_walk_init(wk, lc, L.cx0 - X0, L.cy0 - Y0, cw);
             int32_t dx = 0;
             uint64_t out = 0;
             for (int32_t j = 0; j < maxc; ++j) {
@@ -1369,7 +1477,7 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
                 cnt = (uint32_t)__popcll(any & 0x1111111111111111ull);
             }
 #else
-            if (small) kz_walk_init(wk, L.t, L.c, L.cx0, L.cy0, cw);
+            if (small) kz_tile_walk_init(wk, lc, L.cx0 - X0, L.cy0 - Y0, cw);
             int32_t dx = 0;
             for (int32_t j = 0; j < maxc; ++j) {
                 if (small && j < cand) {
@@ -1389,22 +1497,8 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
         while (bigm) {
             const uint32_t b = (uint32_t)__builtin_ctzll(bigm);
             bigm &= bigm - 1;
-            KzTri tb;
-            tb.x0 = kz_readlane_i(L.t.x0, b);
-            tb.y0 = kz_readlane_i(L.t.y0, b);
-            tb.d1x = kz_readlane_i(L.t.d1x, b);
-            tb.d1y = kz_readlane_i(L.t.d1y, b);
-            tb.d2x = kz_readlane_i(L.t.d2x, b);
-            tb.d2y = kz_readlane_i(L.t.d2y, b);
-            tb.S = (int64_t)(((uint64_t)(uint32_t)kz_readlane_i((int32_t)(uint32_t)(uint64_t)L.t.S, b)) |
-                             ((uint64_t)(uint32_t)kz_readlane_i((int32_t)((uint64_t)L.t.S >> 32), b) << 32));
-            KzCov cb;
-            cb.flip = kz_readlane_i(L.c.flip, b);
-            cb.th01 = kz_readlane_i(L.c.th01, b);
-            cb.th12 = kz_readlane_i(L.c.th12, b);
-            cb.th20 = kz_readlane_i(L.c.th20, b);
-            cb.small = kz_readlane_i(L.c.small, b);
-            const int32_t bx0 = kz_readlane_i(L.cx0, b), by0 = kz_readlane_i(L.cy0, b);
+            const KzTileCov cb = kz_tile_cov_of(lc, b);
+            const int32_t bx0 = kz_readlane_i(L.cx0, b) - X0, by0 = kz_readlane_i(L.cy0, b) - Y0;
             const int32_t bw = kz_readlane_i(cw, b), bc = kz_readlane_i(cand, b);
             // candidate i is pixel (i % bw, i / bw) of the box; the row is
             // floor((i + 0.5) / bw) through the reciprocal: that quotient is
@@ -1417,7 +1511,7 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
                 bool cov = false;
                 if (i < bc) {
                     const int32_t dy = (int32_t)(((float)i + 0.5f) * rbw);
-                    cov = kz_cover_mask(tb, cb, bx0 + i - dy * bw, by0 + dy) != 0;
+                    cov = kz_tile_mask(cb, bx0 + i - dy * bw, by0 + dy) != 0;
                 }
                 c += (uint32_t)__popcll(kz_ballot(cov));
             }
@@ -1463,22 +1557,8 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
         while (bigm) {
             const uint32_t b = (uint32_t)__builtin_ctzll(bigm);
             bigm &= bigm - 1;
-            KzTri tb;
-            tb.x0 = kz_readlane_i(L.t.x0, b);
-            tb.y0 = kz_readlane_i(L.t.y0, b);
-            tb.d1x = kz_readlane_i(L.t.d1x, b);
-            tb.d1y = kz_readlane_i(L.t.d1y, b);
-            tb.d2x = kz_readlane_i(L.t.d2x, b);
-            tb.d2y = kz_readlane_i(L.t.d2y, b);
-            tb.S = (int64_t)(((uint64_t)(uint32_t)kz_readlane_i((int32_t)(uint32_t)(uint64_t)L.t.S, b)) |
-                             ((uint64_t)(uint32_t)kz_readlane_i((int32_t)((uint64_t)L.t.S >> 32), b) << 32));
-            KzCov cb;
-            cb.flip = kz_readlane_i(L.c.flip, b);
-            cb.th01 = kz_readlane_i(L.c.th01, b);
-            cb.th12 = kz_readlane_i(L.c.th12, b);
-            cb.th20 = kz_readlane_i(L.c.th20, b);
-            cb.small = kz_readlane_i(L.c.small, b);
-            const int32_t bx0 = kz_readlane_i(L.cx0, b), by0 = kz_readlane_i(L.cy0, b);
+            const KzTileCov cb = kz_tile_cov_of(lc, b);
+            const int32_t bx0 = kz_readlane_i(L.cx0, b) - X0, by0 = kz_readlane_i(L.cy0, b) - Y0;
             const int32_t bw = kz_readlane_i(cw, b), bc = kz_readlane_i(cand, b);
             uint32_t w = (uint32_t)kz_readlane_i((int32_t)excl, b);
             const float rbw = __builtin_amdgcn_rcpf((float)bw);  // (rows as in phase 1)
@@ -1490,10 +1570,10 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
                     const int32_t dy = (int32_t)(((float)i + 0.5f) * rbw);
                     px = bx0 + i - dy * bw;
                     py = by0 + dy;
-                    m = kz_cover_mask(tb, cb, px, py);
+                    m = kz_tile_mask(cb, px, py);
                 }
                 const uint64_t bal = kz_ballot(m != 0);
-                if (m) s_frag[w + kz_rank(bal)] = kz_pack_frag((uint32_t)((py - Y0) * KZ_TS + (px - X0)), b, m);
+                if (m) s_frag[w + kz_rank(bal)] = kz_pack_frag((uint32_t)(py * KZ_TS + px), b, m);
                 w += (uint32_t)__popcll(bal);
             }
         }
@@ -1502,10 +1582,13 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
         if (!filter) kz_ahead_indices(nx, f);
 
         // --- resolve the queue 64 fragments at a time --------------------
+        uint32_t bfrag = 0, bpass = 0;
         if (narrow)
-            kz_resolve<true>(f, L, X0, Y0, total, lane, s_color, s_depth, s_claim, s_frag, nfrag, npass);
+            kz_resolve<true>(f, L, X0, Y0, total, lane, s_color, s_depth, s_claim, s_frag, bfrag, bpass);
         else
-            kz_resolve<false>(f, L, X0, Y0, total, lane, s_color, s_depth, s_claim, s_frag, nfrag, npass);
+            kz_resolve<false>(f, L, X0, Y0, total, lane, s_color, s_depth, s_claim, s_frag, bfrag, bpass);
+        nfrag += bfrag;
+        npass += bpass;
         k = next_k;
         ks = next_ks;
         __syncthreads();
