@@ -251,14 +251,15 @@ enum {
 #define KZ_SPLIT_CHUNK 256u
 
 // Radix binning: kz_bin_count adds the (triangle, tile) pairs of each block
-// of KZ_BIN_BLOCK triangles; pairs are generated KZ_PAIR_CHUNK triangles
-// (KZ_PAIR_CHUNK / KZ_BIN_BLOCK blocks) per workgroup.
+// of KZ_BIN_BLOCK triangles; pairs are generated per chunk of
+// KZ_PAIR_CHUNK triangles (KZ_PAIR_CHUNK / KZ_BIN_BLOCK blocks).
 #define KZ_BIN_BLOCK 256u
-#define KZ_PAIR_CHUNK 4096u
+#define KZ_PAIR_CHUNK 1024u
 enum {
     KZ_BIN_PAIRS = 0,  // pairs generated and sorted this batch (<= list capacity)
     KZ_BIN_CUT = 1,    // first pair chunk whose pairs did not fit (chunks when all fit)
     KZ_BIN_OVER = 2,   // 1 when chunks were cut
+    KZ_BIN_EXTRA = 3,  // pieces of chunks' pairs after their first
     KZ_BIN_WORDS = 4
 };
 

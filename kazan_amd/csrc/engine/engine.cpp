@@ -47,7 +47,7 @@ Engine::~Engine() {
     hipFree(sort_tmp_);
     hipFree(tri_rect_);
     hipFree(tri_rec_);
-    for (uint32_t *p : {tri_draw_, block_pairs_, chunk_offsets_, bin_ctrl_, tile_flag_, pair_keys_[0], pair_keys_[1],
+    for (uint32_t *p : {tri_draw_, block_pairs_, chunk_offsets_, chunk_extra_, bin_ctrl_, tile_flag_, pair_keys_[0], pair_keys_[1],
                         pair_vals_[0], pair_vals_[1], radix_table_, radix_totals_})
         hipFree(p);
     for (uint32_t *p : {tile_level_, split_slot_, split_info_, queue_, ctrl_, split_counts_, split_offsets_,
@@ -253,6 +253,7 @@ hipError_t Engine::ensure_scratch(uint32_t tiles, uint32_t tris) {
         if (radix_) {
             KZ_TRY(regrow(block_pairs_, (t + KZ_BIN_BLOCK - 1) / KZ_BIN_BLOCK));
             KZ_TRY(regrow(chunk_offsets_, (t + KZ_PAIR_CHUNK - 1) / KZ_PAIR_CHUNK));
+            KZ_TRY(regrow(chunk_extra_, (t + KZ_PAIR_CHUNK - 1) / KZ_PAIR_CHUNK));
         }
         cap_tris_ = t;
     }
@@ -406,7 +407,7 @@ hipError_t Engine::run_batch(const Op &op, const BatchConfig &cfg) {
         // pairs in primitive order, a stable radix sort by tile whose last
         // pass writes the lists, counts and offsets
         f.block_pairs = block_pairs_;
-        KzRadixScratch rs{chunk_offsets_, bin_ctrl_, tile_flag_, {pair_keys_[0], pair_keys_[1]},
+        KzRadixScratch rs{chunk_offsets_, chunk_extra_, bin_ctrl_, tile_flag_, {pair_keys_[0], pair_keys_[1]},
                           {pair_vals_[0], pair_vals_[1]}, radix_table_, radix_totals_,
                           kz_radix_blocks(list_capacity_)};
         KZ_TRY(mark(KS_BIN_COUNT, false));

@@ -343,7 +343,7 @@ class Engine {
     // or, with KAZAN_BINNING=sort, per-tile counts, an unordered scatter and
     // a sort of every list.
     bool radix_ = true;
-    uint32_t *block_pairs_ = nullptr, *chunk_offsets_ = nullptr, *bin_ctrl_ = nullptr, *tile_flag_ = nullptr;
+    uint32_t *block_pairs_ = nullptr, *chunk_offsets_ = nullptr, *chunk_extra_ = nullptr, *bin_ctrl_ = nullptr, *tile_flag_ = nullptr;
     uint32_t *pair_keys_[2] = {nullptr, nullptr}, *pair_vals_[2] = {nullptr, nullptr};
     // (balanced form) the list entries' 4 x 4 sub-tile masks
     uint16_t *list_mask_ = nullptr;

@@ -20,6 +20,7 @@ hipError_t kz_launch_scan(hipStream_t st, uint32_t *counts, uint32_t *offsets, u
 // Radix binning, after kz_bin_count wrote f.tri_rect and f.block_pairs.
 struct KzRadixScratch {
     uint32_t *chunk_offsets;  // [ceil(tris / KZ_PAIR_CHUNK)]
+    uint32_t *chunk_extra;    // [ceil(tris / KZ_PAIR_CHUNK)]
     uint32_t *ctrl;           // KZ_BIN_WORDS
     uint32_t *tile_flag;      // [tiles], cleared with the counts before a batch
     uint32_t *keys[2], *vals[2];  // [list capacity] each

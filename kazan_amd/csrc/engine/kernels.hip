@@ -80,6 +80,20 @@ __device__ __forceinline__ uint32_t readlane(uint32_t v, uint32_t l) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
 }
 
+// Inclusive sum over the wave's lanes (all active), by DPP: within rows of
+// 16 lanes, then each row's last lane to the rows after it.
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
+#define KZ_DPP_ADD(ctrl, rows) v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xF, false)
+    KZ_DPP_ADD(0x111, 0xF);  // row_shr:1
+    KZ_DPP_ADD(0x112, 0xF);
+    KZ_DPP_ADD(0x114, 0xF);
+    KZ_DPP_ADD(0x118, 0xF);
+    KZ_DPP_ADD(0x142, 0xA);  // row_bcast:15 into rows 1 and 3
+    KZ_DPP_ADD(0x143, 0xC);  // row_bcast:31 into rows 2 and 3
+#undef KZ_DPP_ADD
+    return v;
+}
+
 __device__ __forceinline__ void unpack_box(uint64_t r, uint32_t &x0, uint32_t &y0, uint32_t &x1, uint32_t &y1) {
     x0 = (uint32_t)(r & 0xFFFF);
     y0 = (uint32_t)((r >> 16) & 0xFFFF);
@@ -580,9 +594,15 @@ __global__ __launch_bounds__(kSortThreads) void kz_sort_lists(const uint32_t *co
 // costs the same whatever the skew: a tile holding a million pairs is as
 // cheap as a million tiles holding one.
 
-constexpr uint32_t kPairThreads = 1024;
+constexpr uint32_t kPairThreads = 256;
 constexpr uint32_t kPairPer = KZ_PAIR_CHUNK / kPairThreads;  // triangles per thread
+constexpr uint32_t kPairPiece = 1024;                        // pairs one workgroup writes
+constexpr uint32_t kPairExtraGrid = 1024;                    // workgroups for the pieces after a chunk's first
+constexpr uint32_t kPairInline = 8;                          // pairs of one triangle that its own lane writes
 constexpr uint32_t kBlocksPerChunk = KZ_PAIR_CHUNK / KZ_BIN_BLOCK;
+static_assert(kBlocksPerChunk == 4, "a chunk's block counts are one 16-byte load");
+constexpr uint32_t kPairScanThreads = 1024;
+constexpr uint32_t kPairScanPer = 4;  // chunks per thread and step
 constexpr uint32_t kRadixThreads = 512;
 constexpr uint32_t kRadixWaves = kRadixThreads / 64;
 constexpr uint32_t kRadixRounds = 8;                            // pairs per lane
@@ -618,140 +638,258 @@ __device__ __forceinline__ uint32_t box_sub_mask16(uint32_t x0, uint32_t y0, uin
 // exceed `capacity`, the chunks from the first one that does not fit on are
 // cut: ctrl[KZ_BIN_CUT] is that chunk and ctrl[KZ_BIN_PAIRS] the pairs
 // before it (kz_pair_write then flags the tiles of the cut triangles).
-__global__ __launch_bounds__(kScanThreads) void kz_pair_scan(const uint32_t *block_pairs, uint32_t nblocks,
-                                                             uint32_t *chunk_offsets, uint32_t nchunks,
-                                                             uint32_t capacity, uint32_t *ctrl,
-                                                             unsigned long long *stats) {
-    __shared__ unsigned long long s_wave[kScanThreads / 64];
-    __shared__ unsigned long long s_carry, s_cut;  // s_cut: first cut chunk << 32 | its offset
+// chunk_extra[c]: the pieces of kPairPiece pairs after the first of all
+// chunks before c (ctrl[KZ_BIN_EXTRA] in all), which kz_pair_write gives to
+// workgroups of their own.
+// Bound by the latency of its loads: a step takes 4,096 chunks, each thread
+// 4 consecutive ones with all their loads in flight at once (8.4 M
+// triangles: two steps; 256 threads of one chunk each took 8 steps of 4,096
+// triangles a chunk, MEAS_PSCAN).
+__global__ __launch_bounds__(kPairScanThreads) void kz_pair_scan(const uint32_t *block_pairs, uint32_t ntris,
+                                                                 uint32_t *chunk_offsets, uint32_t *chunk_extra,
+                                                                 uint32_t nchunks, uint32_t capacity, uint32_t *ctrl,
+                                                                 unsigned long long *stats) {
+    __shared__ unsigned long long s_wave[kPairScanThreads / 64];
+    __shared__ uint32_t s_ewave[kPairScanThreads / 64];
+    __shared__ unsigned long long s_cut;  // first cut chunk << 32 | its offset
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) {
-        s_carry = 0;
-        s_cut = ~0ull;
-    }
-    __syncthreads();
-    for (uint32_t c0 = 0; c0 < nchunks; c0 += kScanThreads) {
-        const uint32_t c = c0 + tid;
-        unsigned long long v = 0;
+    const uint32_t nblocks = (ntris + KZ_BIN_BLOCK - 1) / KZ_BIN_BLOCK;
+    if (tid == 0) s_cut = ~0ull;
+    unsigned long long carry = 0;
+    uint32_t ecarry = 0;
+    for (uint32_t c0 = 0; c0 < nchunks; c0 += kPairScanThreads * kPairScanPer) {
+        const uint32_t c = c0 + tid * kPairScanPer;
+        uint32_t b[kPairScanPer][kBlocksPerChunk];
 #pragma unroll
-        for (uint32_t j = 0; j < kBlocksPerChunk; ++j) {
-            const uint32_t b = c * kBlocksPerChunk + j;
-            v += c < nchunks && b < nblocks ? block_pairs[b] : 0u;
+        for (uint32_t i = 0; i < kPairScanPer; ++i) {
+            const uint32_t first = (c + i) * kBlocksPerChunk;
+            uint4 v = make_uint4(0u, 0u, 0u, 0u);
+            if (c + i < nchunks) {
+                if (first + kBlocksPerChunk <= nblocks) {
+                    v = *(const uint4 *)(block_pairs + first);
+                } else {
+                    v.x = block_pairs[first];  // (a chunk has at least one block)
+                    v.y = first + 1 < nblocks ? block_pairs[first + 1] : 0u;
+                    v.z = first + 2 < nblocks ? block_pairs[first + 2] : 0u;
+                }
+            }
+            b[i][0] = v.x;
+            b[i][1] = v.y;
+            b[i][2] = v.z;
+            b[i][3] = v.w;
         }
-        unsigned long long x = v;
+        unsigned long long v[kPairScanPer], sum = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < kPairScanPer; ++i) {
+            v[i] = (unsigned long long)b[i][0] + b[i][1] + b[i][2] + b[i][3];
+            sum += v[i];
+        }
+        unsigned long long x = sum;
         for (uint32_t d = 1; d < 64; d <<= 1) {
             const unsigned long long o = __shfl_up(x, d, 64);
             if (lane >= d) x += o;
         }
         if (lane == 63) s_wave[wave] = x;
         __syncthreads();
-        unsigned long long wbase = 0, total = 0;
-        for (uint32_t w = 0; w < kScanThreads / 64; ++w) {
+        unsigned long long run = carry + x - sum;
+        for (uint32_t w = 0; w < kPairScanThreads / 64; ++w) {
             const unsigned long long t = s_wave[w];
-            if (w < wave) wbase += t;
-            total += t;
+            if (w < wave) run += t;
+            carry += t;
         }
-        const unsigned long long carry = s_carry;
-        if (c < nchunks) {
-            const unsigned long long excl = carry + wbase + x - v;
-            chunk_offsets[c] = (uint32_t)min(excl, (unsigned long long)capacity);
-            if (excl + v > capacity) atomicMin(&s_cut, ((unsigned long long)c << 32) | (uint32_t)min(excl, (unsigned long long)capacity));
+        // (a chunk that ends past the capacity is cut, and so are all after it)
+        uint32_t e[kPairScanPer], esum = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < kPairScanPer; ++i) {
+            e[i] = 0;
+            if (c + i < nchunks) {
+                chunk_offsets[c + i] = (uint32_t)min(run, (unsigned long long)capacity);
+                if (run + v[i] > capacity)
+                    atomicMin(&s_cut, ((unsigned long long)(c + i) << 32) |
+                                          (uint32_t)min(run, (unsigned long long)capacity));
+                else if (v[i] > 2 * min(KZ_PAIR_CHUNK, ntris - (c + i) * KZ_PAIR_CHUNK))
+                    e[i] = (uint32_t)((v[i] + kPairPiece - 1) / kPairPiece) - 1u;
+            }
+            run += v[i];
+            esum += e[i];
         }
+        const uint32_t ex = wave_incl_scan(esum);
+        if (lane == 63) s_ewave[wave] = ex;
         __syncthreads();
-        if (tid == 0) s_carry = carry + total;
-        __syncthreads();
+        uint32_t erun = ecarry + ex - esum;
+        for (uint32_t w = 0; w < kPairScanThreads / 64; ++w) {
+            const uint32_t t = s_ewave[w];
+            if (w < wave) erun += t;
+            ecarry += t;
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < kPairScanPer; ++i) {
+            if (c + i < nchunks) chunk_extra[c + i] = erun;
+            erun += e[i];
+        }
     }
+    __syncthreads();
     if (tid == 0) {
-        const unsigned long long pairs = s_carry, cut = s_cut;
+        const unsigned long long cut = s_cut;
         const bool over = cut != ~0ull;
         ctrl[KZ_BIN_CUT] = over ? (uint32_t)(cut >> 32) : nchunks;
-        ctrl[KZ_BIN_PAIRS] = over ? (uint32_t)cut : (uint32_t)pairs;
+        ctrl[KZ_BIN_PAIRS] = over ? (uint32_t)cut : (uint32_t)carry;
         ctrl[KZ_BIN_OVER] = over ? 1u : 0u;
+        ctrl[KZ_BIN_EXTRA] = ecarry;
         if (stats) {
-            atomicAdd(&stats[KZ_STAT_LIST_ENTRIES], pairs);
+            atomicAdd(&stats[KZ_STAT_LIST_ENTRIES], carry);
             if (over) atomicAdd(&stats[KZ_STAT_LIST_OVERFLOW], 1ull);
         }
     }
 }
 
-// Writes the pairs of chunk c = blockIdx.x (triangles [c * KZ_PAIR_CHUNK,
-// ...)) from its offset on: the chunk's q-th pair is the k-th tile of the
-// triangle whose prefix range holds q. A cut chunk instead flags every tile
-// its triangles' boxes touch; kz_tile_list reads a flagged tile as one for
-// the in-order scan of all pixel boxes. With key_masks (fewer than 65536
-// tiles) a key carries the pair's box_sub_mask16 in its upper 16 bits, for
-// the split of the tile's list; the sort's digits read only the tile bits.
-__global__ __launch_bounds__(kPairThreads) void kz_pair_write(const uint64_t *rect, uint32_t ntris, uint32_t sh,
-                                                              uint32_t tiles_x, const uint32_t *chunk_offsets,
-                                                              const uint32_t *ctrl, uint32_t *keys, uint32_t *vals,
-                                                              uint32_t key_masks, uint32_t *tile_flag) {
+// Where pairs go: keys carry the tile and, with masks (fewer than 65536
+// tiles), the pair's box_sub_mask16 in their upper 16 bits, for the split of
+// the tile's list; the sort's digits read only the tile bits.
+struct PairOut {
+    uint32_t *keys, *vals;
+    uint32_t sh, tiles_x, masks;
+    __device__ __forceinline__ void put(uint32_t at, uint64_t r, uint32_t tx, uint32_t ty, uint32_t g) const {
+        uint32_t x0, y0, x1, y1;
+        unpack_box(r, x0, y0, x1, y1);
+        const uint32_t tile = ty * tiles_x + tx;
+        keys[at] = masks ? tile | (box_sub_mask16(x0, y0, x1, y1, tx, ty, sh) << 16) : tile;
+        vals[at] = g;
+    }
+};
+
+// Writes the pairs of chunk c (triangles [c * KZ_PAIR_CHUNK, ...)) from its
+// offset on, in primitive order, each triangle's tiles row-major in its pixel
+// box. A cut chunk instead flags every tile its triangles' boxes touch;
+// kz_tile_list reads a flagged tile as one for the in-order scan of all
+// pixel boxes.
+// A chunk of at most two pairs a triangle (meshes of small triangles) is
+// written by its triangles' lanes, consecutive lanes to consecutive places:
+// the prefix is all it computes. A triangle of more than kPairInline tiles
+// takes its wave. The pairs of the other chunks are written kPairPiece at a
+// time, one workgroup each (the first with the chunk, the others taken in
+// turn by the workgroups past the chunks'), whose lanes find their triangle
+// by binary search over the prefix in LDS: a few hundred large triangles are
+// one chunk, and one workgroup for all its pairs was most of their binning.
+// A search for every pair of 4,096-triangle chunks took (us, before -> now):
+// 1,024 large triangles at 256^2 113 -> 7, 40,400 around a camera 51 -> 12,
+// 8.4 M of about one pixel 54 -> 32, 4.2 M in a cluster 17.5 -> 14.6, a grid
+// of 11,834 16.5 -> 6.7.
+__global__ __launch_bounds__(kPairThreads) void kz_pair_write(const uint64_t *rect, uint32_t ntris, uint32_t nchunks,
+                                                              PairOut o, const uint32_t *chunk_offsets,
+                                                              const uint32_t *chunk_extra, const uint32_t *ctrl,
+                                                              uint32_t *tile_flag) {
     __shared__ uint64_t s_rect[KZ_PAIR_CHUNK];
     __shared__ uint32_t s_pfx[KZ_PAIR_CHUNK];
-    __shared__ uint32_t s_wave[kPairThreads / 64];
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t t0 = blockIdx.x * KZ_PAIR_CHUNK;
-    if (t0 >= ntris) return;
-    const uint32_t n = min(KZ_PAIR_CHUNK, ntris - t0);
-    if (blockIdx.x >= ctrl[KZ_BIN_CUT]) {
-        for (uint32_t i = tid; i < n; i += kPairThreads) {
-            const uint64_t r = rect[t0 + i];
-            if (r == KZ_RECT_EMPTY) continue;
+    __shared__ uint32_t s_wave[kPairPer][kPairThreads / 64];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, sh = o.sh;
+    const bool first = blockIdx.x < nchunks;
+    const uint32_t nextra = first ? 0u : ctrl[KZ_BIN_EXTRA];
+    for (uint32_t e = first ? 0u : blockIdx.x - nchunks; first || e < nextra; e += gridDim.x - nchunks) {
+        uint32_t c = blockIdx.x, piece = 0;
+        if (!first) {  // extra piece e: of the last chunk whose pieces start at or before it
+            uint32_t lo = 0, hi = nchunks;
+            while (hi - lo > 1) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (chunk_extra[mid] <= e) lo = mid;
+                else hi = mid;
+            }
+            c = lo;
+            piece = e - chunk_extra[c] + 1;
+        }
+        const uint32_t t0 = c * KZ_PAIR_CHUNK, n = min(KZ_PAIR_CHUNK, ntris - t0);
+        if (c >= ctrl[KZ_BIN_CUT]) {  // (such a chunk has no extra pieces)
+            for (uint32_t i = tid; i < n; i += kPairThreads) {
+                const uint64_t r = rect[t0 + i];
+                if (r == KZ_RECT_EMPTY) continue;
+                uint32_t x0, y0, x1, y1;
+                unpack_box(r, x0, y0, x1, y1);
+                for (uint32_t ty = y0 >> sh; ty <= (y1 >> sh); ++ty)
+                    for (uint32_t tx = x0 >> sh; tx <= (x1 >> sh); ++tx) tile_flag[ty * o.tiles_x + tx] = 1u;
+            }
+            return;
+        }
+        // thread tid's j-th triangle is t0 + j * kPairThreads + tid
+        uint64_t r[kPairPer];
+        uint32_t cnt[kPairPer], pfx[kPairPer];
+#pragma unroll
+        for (uint32_t j = 0; j < kPairPer; ++j) {
+            const uint32_t i = j * kPairThreads + tid;
+            r[j] = i < n ? rect[t0 + i] : KZ_RECT_EMPTY;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kPairPer; ++j) {
+            cnt[j] = box_tiles(r[j], sh);
+            const uint32_t x = wave_incl_scan(cnt[j]);
+            pfx[j] = x - cnt[j];
+            if (lane == 63) s_wave[j][wave] = x;
+        }
+        __syncthreads();
+        uint32_t total = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kPairPer; ++j)
+#pragma unroll
+            for (uint32_t w = 0; w < kPairThreads / 64; ++w) {
+                if (w == wave) pfx[j] += total;
+                total += s_wave[j][w];
+            }
+        const uint32_t out = chunk_offsets[c];
+        if (total <= 2 * n) {  // (no extra pieces: kz_pair_scan)
+#pragma unroll
+            for (uint32_t j = 0; j < kPairPer; ++j) {
+                const uint32_t g = t0 + j * kPairThreads + tid;
+                uint32_t x0, y0, x1, y1;
+                unpack_box(r[j], x0, y0, x1, y1);
+                const uint32_t tx0 = x0 >> sh, tx1 = x1 >> sh;
+                if (cnt[j] <= kPairInline) {
+                    uint32_t tx = tx0, ty = y0 >> sh;
+                    for (uint32_t k = 0; k < cnt[j]; ++k) {
+                        o.put(out + pfx[j] + k, r[j], tx, ty, g);
+                        ty += tx == tx1 ? 1u : 0u;
+                        tx = tx == tx1 ? tx0 : tx + 1;
+                    }
+                }
+                uint64_t m = __ballot(cnt[j] > kPairInline);
+                while (m) {
+                    const uint32_t b = (uint32_t)__builtin_ctzll(m);
+                    m &= m - 1;
+                    const uint64_t rb = (uint64_t)readlane((uint32_t)r[j], b) |
+                                        ((uint64_t)readlane((uint32_t)(r[j] >> 32), b) << 32);
+                    const uint32_t cb = readlane(cnt[j], b), at = out + readlane(pfx[j], b), gb = readlane(g, b);
+                    uint32_t bx0, by0, bx1, by1;
+                    unpack_box(rb, bx0, by0, bx1, by1);
+                    const uint32_t bt = bx0 >> sh, tw = (bx1 >> sh) - bt + 1;
+                    for (uint32_t k = lane; k < cb; k += 64) {
+                        const uint32_t ky = k / tw;
+                        o.put(at + k, rb, bt + k - ky * tw, (by0 >> sh) + ky, gb);
+                    }
+                }
+            }
+            return;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kPairPer; ++j) {
+            s_rect[j * kPairThreads + tid] = r[j];
+            s_pfx[j * kPairThreads + tid] = pfx[j];
+        }
+        __syncthreads();
+        for (uint32_t q = piece * kPairPiece + tid; q < min(total, (piece + 1) * kPairPiece); q += kPairThreads) {
+            // the last triangle whose prefix is <= q (s_pfx[0] = 0 <= q)
+            uint32_t lo = 0, hi = KZ_PAIR_CHUNK;
+            while (hi - lo > 1) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (s_pfx[mid] <= q) lo = mid;
+                else hi = mid;
+            }
+            const uint32_t k = q - s_pfx[lo];
             uint32_t x0, y0, x1, y1;
-            unpack_box(r, x0, y0, x1, y1);
-            for (uint32_t ty = y0 >> sh; ty <= (y1 >> sh); ++ty)
-                for (uint32_t tx = x0 >> sh; tx <= (x1 >> sh); ++tx) tile_flag[ty * tiles_x + tx] = 1u;
+            unpack_box(s_rect[lo], x0, y0, x1, y1);
+            const uint32_t tx0 = x0 >> sh, tw = (x1 >> sh) - tx0 + 1;
+            const uint32_t ky = k / tw;
+            o.put(out + q, s_rect[lo], tx0 + k - ky * tw, (y0 >> sh) + ky, t0 + lo);
         }
-        return;
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < kPairPer; ++j) {
-        const uint32_t i = j * kPairThreads + tid;
-        s_rect[i] = i < n ? rect[t0 + i] : KZ_RECT_EMPTY;
-    }
-    __syncthreads();
-    // prefix of the pair counts, kPairPer consecutive triangles per thread
-    uint32_t cnt[kPairPer], sum = 0;
-#pragma unroll
-    for (uint32_t j = 0; j < kPairPer; ++j) {
-        cnt[j] = box_tiles(s_rect[tid * kPairPer + j], sh);
-        sum += cnt[j];
-    }
-    uint32_t x = sum;
-    for (uint32_t d = 1; d < 64; d <<= 1) {
-        const uint32_t o = __shfl_up(x, d, 64);
-        if (lane >= d) x += o;
-    }
-    if (lane == 63) s_wave[wave] = x;
-    __syncthreads();
-    uint32_t run = x - sum, total = 0;
-    for (uint32_t w = 0; w < kPairThreads / 64; ++w) {
-        const uint32_t t = s_wave[w];
-        if (w < wave) run += t;
-        total += t;
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < kPairPer; ++j) {
-        s_pfx[tid * kPairPer + j] = run;
-        run += cnt[j];
-    }
-    __syncthreads();
-    const uint32_t out = chunk_offsets[blockIdx.x];
-    for (uint32_t q = tid; q < total; q += kPairThreads) {
-        // the last triangle whose prefix is <= q (s_pfx[0] = 0 <= q)
-        uint32_t lo = 0, hi = KZ_PAIR_CHUNK;
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (s_pfx[mid] <= q) lo = mid;
-            else hi = mid;
-        }
-        const uint32_t k = q - s_pfx[lo];
-        uint32_t x0, y0, x1, y1;
-        unpack_box(s_rect[lo], x0, y0, x1, y1);
-        const uint32_t tx0 = x0 >> sh, tw = (x1 >> sh) - tx0 + 1;
-        const uint32_t ky = k / tw, kx = k - ky * tw;
-        const uint32_t tile = ((y0 >> sh) + ky) * tiles_x + tx0 + kx;
-        keys[out + q] = key_masks ? tile | (box_sub_mask16(x0, y0, x1, y1, tx0 + kx, (y0 >> sh) + ky, sh) << 16) : tile;
-        vals[out + q] = t0 + lo;
+        if (first) return;
+        __syncthreads();  // the next piece overwrites the LDS tables
     }
 }
 
@@ -2098,13 +2236,16 @@ uint32_t kz_radix_passes(uint32_t ntiles) {
 
 hipError_t kz_launch_bin_pairs(hipStream_t st, const KzFrame &f, const KzRadixScratch &s) {
     if (f.total_tris == 0) return hipSuccess;
-    const uint32_t nblocks = (f.total_tris + KZ_BIN_BLOCK - 1) / KZ_BIN_BLOCK;
     const uint32_t nchunks = (f.total_tris + KZ_PAIR_CHUNK - 1) / KZ_PAIR_CHUNK;
-    kz_pair_scan<<<1, kScanThreads, 0, st>>>(f.block_pairs, nblocks, s.chunk_offsets, nchunks, f.list_capacity,
-                                             s.ctrl, f.stats);
-    kz_pair_write<<<nchunks, kPairThreads, 0, st>>>(f.tri_rect, f.total_tris, f.tile_shift, f.tiles_x,
-                                                    s.chunk_offsets, s.ctrl, s.keys[0], s.vals[0],
-                                                    f.list_mask ? 1u : 0u, s.tile_flag);
+    kz_pair_scan<<<1, kPairScanThreads, 0, st>>>(f.block_pairs, f.total_tris, s.chunk_offsets, s.chunk_extra, nchunks,
+                                                 f.list_capacity, s.ctrl, f.stats);
+    // workgroups for the pieces after the chunks' first: no more than the
+    // largest pair count (and the list capacity) can make
+    const uint64_t most = std::min<uint64_t>((uint64_t)f.total_tris * f.tiles_x * f.tiles_y, f.list_capacity);
+    const uint32_t extra = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(most / kPairPiece, 1), kPairExtraGrid);
+    const PairOut out{s.keys[0], s.vals[0], f.tile_shift, f.tiles_x, f.list_mask ? 1u : 0u};
+    kz_pair_write<<<nchunks + extra, kPairThreads, 0, st>>>(f.tri_rect, f.total_tris, nchunks, out, s.chunk_offsets,
+                                                            s.chunk_extra, s.ctrl, s.tile_flag);
     return hipGetLastError();
 }
 
