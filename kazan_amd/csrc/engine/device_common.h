@@ -92,15 +92,26 @@ struct KzFrame {
     uint32_t *tile_offsets;  // [tiles] first entry of the tile's list (any value when empty)
     uint32_t *tile_cursor;   // [tiles] scatter cursors
     uint32_t *tile_flag;     // [tiles] nonzero: cut by the list capacity (radix binning), or null
-    const uint32_t *bin_ctrl;  // KZ_BIN_* words of radix binning (the first cut chunk), or null
+    uint32_t *bin_ctrl;      // KZ_BIN_* words of radix binning (the first cut chunk), or null
     uint32_t *tile_lists;    // [list_capacity] triangle ids, per tile, sorted
     uint32_t *sort_tmp;      // [list_capacity] merge scratch for long lists
     uint32_t list_capacity;
     uint32_t pad0;
-    uint64_t *tri_rect;      // [total_tris] packed pixel bounding box or ~0
+    uint64_t *tri_rect;      // [total_tris + clip_cap] packed pixel bounding box or ~0, then the clip pieces'
     uint32_t *tri_rec;       // [total_tris * KZ_REC_WORDS_FOR(varyings)] setup records, or null
     uint32_t *block_pairs;   // [ceil(total_tris / 256)] (triangle, tile) pairs per binning block, or null
     uint32_t *tri_draw;      // [total_tris] draw of each triangle (batches of several draws), or null
+    uint32_t *chunk_offsets;  // [ceil(total_tris / KZ_PAIR_CHUNK)] first pair of each chunk (radix binning)
+    uint32_t *chunk_extra;    // [ceil(total_tris / KZ_PAIR_CHUNK)] pieces of pairs after the chunks' first, before it
+    // Clip pieces (radix binning without setup records; else null): a
+    // triangle that needs clipping is clipped while binning, and its pieces
+    // are list entries of their own, id total_tris + piece, with their pixel
+    // boxes in tri_rect and their setup records in clip_rec.
+    uint32_t *clip_of;        // [total_tris] of a triangle with pieces (KZ_RECT_PIECES): first piece << 4 | pieces
+    uint32_t *clip_tris;      // [clip_cap] the triangles with pieces, in any order
+    uint32_t *clip_rec;       // [clip_cap * KZ_REC_WORDS_FOR(varyings)]
+    uint32_t clip_cap;
+    uint32_t pad2;
     unsigned long long *stats;  // KZ_STAT_* counters
 
     // Load-balanced mode. A work item is a square sub-tile of a screen
@@ -255,12 +266,17 @@ enum {
 // KZ_PAIR_CHUNK triangles (KZ_PAIR_CHUNK / KZ_BIN_BLOCK blocks).
 #define KZ_BIN_BLOCK 256u
 #define KZ_PAIR_CHUNK 1024u
+#define KZ_PAIR_PIECE 1024u  // pairs of a chunk that one workgroup writes
 enum {
     KZ_BIN_PAIRS = 0,  // pairs generated and sorted this batch (<= list capacity)
     KZ_BIN_CUT = 1,    // first pair chunk whose pairs did not fit (chunks when all fit)
     KZ_BIN_OVER = 2,   // 1 when chunks were cut
     KZ_BIN_EXTRA = 3,  // pieces of chunks' pairs after their first
-    KZ_BIN_WORDS = 4
+    // clip pieces reserved (past clip_cap: not kept) and triangles with
+    // pieces; zero before a batch (kz_pair_write clears them for the next)
+    KZ_BIN_PIECES = 4,
+    KZ_BIN_CLIPPED = 5,
+    KZ_BIN_WORDS = 8
 };
 
 // Statistics are accumulated in KZ_STAT_STRIPES copies (a workgroup adds to
@@ -271,6 +287,9 @@ enum {
 // Per-triangle pixel bounding box (inclusive, clipped to the scissor),
 // packed as px0 | py0 << 16 | px1 << 32 | py1 << 48; ~0 = no pixels.
 #define KZ_RECT_EMPTY (~0ULL)
+// Set in the box of a triangle that has clip pieces (the box is their
+// union): bit 15 of px0, pixel coordinates taking 14 bits.
+#define KZ_RECT_PIECES 0x8000ULL
 
 // 32-bit words of a setup record with nv varyings: 16 words of edge and
 // plane constants, 3 per varying (base, two deltas), rounded up to 16 B.
@@ -370,6 +389,20 @@ __device__ __forceinline__ uint32_t kz_f2u(float x) {
 }
 // A shader array's run-time word index, clamped into its n words.
 __device__ __forceinline__ int32_t kz_word_index(int32_t i, int32_t n) { return i < 0 ? 0 : (i >= n ? n - 1 : i); }
+
+// Inclusive sum over the wave's lanes (all active), by DPP: within rows of
+// 16 lanes, then each row's last lane to the rows after it.
+__device__ __forceinline__ uint32_t kz_wave_incl_scan(uint32_t v) {
+#define KZ_DPP_ADD(ctrl, rows) v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xF, false)
+    KZ_DPP_ADD(0x111, 0xF);  // row_shr:1
+    KZ_DPP_ADD(0x112, 0xF);
+    KZ_DPP_ADD(0x114, 0xF);
+    KZ_DPP_ADD(0x118, 0xF);
+    KZ_DPP_ADD(0x142, 0xA);  // row_bcast:15 into rows 1 and 3
+    KZ_DPP_ADD(0x143, 0xC);  // row_bcast:31 into rows 2 and 3
+#undef KZ_DPP_ADD
+    return v;
+}
 
 // Tile t's list: its offset and count. A tile flagged by a cut (binning
 // dropped the pairs of triangles past the list capacity, some of them in

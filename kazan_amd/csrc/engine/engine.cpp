@@ -25,6 +25,13 @@ hipError_t grow(T *&p, uint64_t count) {
     return hipMalloc((void **)&p, std::max<uint64_t>(count, 1) * sizeof(T));
 }
 
+// clip pieces kept per batch: their records take 64 B and 12 B per varying
+constexpr uint32_t kMaxClipPieces = 65536;
+
+// workgroups of kz_pair_scan that write the clip pieces' records (16 waves
+// each, one triangle a wave at a time)
+constexpr uint32_t kClipGrid = 64;
+
 // striped partial counters followed by their totals
 constexpr uint64_t kStatWords = (uint64_t)(KZ_STAT_STRIPES + 1) * KZ_STAT_COUNT;
 
@@ -48,7 +55,7 @@ Engine::~Engine() {
     hipFree(tri_rect_);
     hipFree(tri_rec_);
     for (uint32_t *p : {tri_draw_, block_pairs_, chunk_offsets_, chunk_extra_, bin_ctrl_, tile_flag_, pair_keys_[0], pair_keys_[1],
-                        pair_vals_[0], pair_vals_[1], radix_table_, radix_totals_})
+                        pair_vals_[0], pair_vals_[1], radix_table_, radix_totals_, clip_of_, clip_tris_, clip_rec_})
         hipFree(p);
     for (uint32_t *p : {tile_level_, split_slot_, split_info_, queue_, ctrl_, split_counts_, split_offsets_,
                         chunk_desc_, chunk_counts_, split_lists_, plan_table_, tile_acc_, tile_cycles_, tile_frags_, tri_z_})
@@ -92,6 +99,7 @@ bool Engine::init(int hip_device, std::string &err) {
     if (const char *e = std::getenv("KAZAN_SPLIT_LEVEL")) default_max_level_ = (uint32_t)std::min(std::max(std::atoi(e), 0), 2);
     if (radix_ &&
         ((e = hipMalloc((void **)&bin_ctrl_, KZ_BIN_WORDS * sizeof(uint32_t))) != hipSuccess ||
+         (e = kz_launch_fill_u32(stream_, bin_ctrl_, KZ_BIN_WORDS, 0u)) != hipSuccess ||
          (e = hipMalloc((void **)&radix_totals_, kz_radix_digits_max() * sizeof(uint32_t))) != hipSuccess)) {
         err = hipGetErrorString(e);
         return false;
@@ -248,8 +256,15 @@ hipError_t Engine::ensure_scratch(uint32_t tiles, uint32_t tris) {
     }
     if (tris > cap_tris_) {
         const uint32_t t = std::max(tris, cap_tris_ + cap_tris_ / 2);
-        KZ_TRY(regrow(tri_rect_, t));
+        // (clip pieces: as many as there are triangles in a small batch; past
+        // kMaxClipPieces the raster clips what is left tile by tile)
+        cap_clip_ = radix_ && !setup_records_ ? std::min(std::max(t, 1024u), kMaxClipPieces) : 0u;
+        KZ_TRY(regrow(tri_rect_, (uint64_t)t + cap_clip_));
         KZ_TRY(regrow(tri_draw_, t));
+        if (cap_clip_) {
+            KZ_TRY(regrow(clip_of_, t));
+            KZ_TRY(regrow(clip_tris_, cap_clip_));
+        }
         if (radix_) {
             KZ_TRY(regrow(block_pairs_, (t + KZ_BIN_BLOCK - 1) / KZ_BIN_BLOCK));
             KZ_TRY(regrow(chunk_offsets_, (t + KZ_PAIR_CHUNK - 1) / KZ_PAIR_CHUNK));
@@ -312,6 +327,12 @@ hipError_t Engine::prepare_batch(const Op &op, uint32_t shift) {
             KZ_TRY(regrow(tri_rec_, w));
             cap_rec_words_ = w;
         }
+    }
+    const uint64_t clip_words = (uint64_t)cap_clip_ * KZ_REC_WORDS_FOR(op.variants->fixed.num_varyings);
+    if (clip_words > cap_clip_words_) {
+        KZ_TRY(hipStreamSynchronize(stream_));
+        KZ_TRY(regrow(clip_rec_, clip_words));
+        cap_clip_words_ = clip_words;
     }
     if (balanced_) KZ_TRY(ensure_split_scratch(ntiles));
     if ((cost_model_d_ != nullptr && balanced_) || tile_profile_) KZ_TRY(ensure_model_scratch(ntiles, f.total_tris));
@@ -407,7 +428,13 @@ hipError_t Engine::run_batch(const Op &op, const BatchConfig &cfg) {
         // pairs in primitive order, a stable radix sort by tile whose last
         // pass writes the lists, counts and offsets
         f.block_pairs = block_pairs_;
-        KzRadixScratch rs{chunk_offsets_, chunk_extra_, bin_ctrl_, tile_flag_, {pair_keys_[0], pair_keys_[1]},
+        f.chunk_offsets = chunk_offsets_;
+        f.chunk_extra = chunk_extra_;
+        f.clip_cap = cap_clip_;
+        f.clip_of = clip_of_;
+        f.clip_tris = clip_tris_;
+        f.clip_rec = clip_rec_;
+        KzRadixScratch rs{bin_ctrl_, tile_flag_, {pair_keys_[0], pair_keys_[1]},
                           {pair_vals_[0], pair_vals_[1]}, radix_table_, radix_totals_,
                           kz_radix_blocks(list_capacity_)};
         KZ_TRY(mark(KS_BIN_COUNT, false));
@@ -415,6 +442,7 @@ hipError_t Engine::run_batch(const Op &op, const BatchConfig &cfg) {
                                      nullptr));
         KZ_TRY(mark(KS_BIN_COUNT, true));
         KZ_TRY(mark(KS_BIN_HIST, false));
+        KZ_TRY(hipModuleLaunchKernel(kern->pair_scan, 1 + kClipGrid, 1, 1, 1024, 1, 1, 0, stream_, args, nullptr));
         KZ_TRY(kz_launch_bin_pairs(stream_, f, rs));
         KZ_TRY(mark(KS_BIN_HIST, true));
         KZ_TRY(mark(KS_BIN_SCATTER, false));

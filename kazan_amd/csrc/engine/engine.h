@@ -36,6 +36,7 @@ struct FixedState {
 struct PipelineKernels {
     hipModule_t module = nullptr;
     hipFunction_t bin_count = nullptr;
+    hipFunction_t pair_scan = nullptr;          // pair offsets and the clip pieces' records
     hipFunction_t raster = nullptr;             // one workgroup per tile
     hipFunction_t raster_persistent = nullptr;  // pops the work-item queue
     uint32_t persistent_blocks = 0;             // resident workgroups that fill the device
@@ -338,6 +339,10 @@ class Engine {
     uint32_t *tile_counts_ = nullptr, *tile_offsets_ = nullptr, *tile_cursor_ = nullptr;
     uint32_t *tile_lists_ = nullptr, *sort_tmp_ = nullptr;
     uint64_t *tri_rect_ = nullptr;
+    // clip pieces (radix binning without setup records)
+    uint32_t *clip_of_ = nullptr, *clip_tris_ = nullptr, *clip_rec_ = nullptr;
+    uint32_t cap_clip_ = 0;
+    uint64_t cap_clip_words_ = 0;
     uint32_t *tri_draw_ = nullptr;  // draw of each triangle, for batches of several draws
     // Binning: radix (pairs in primitive order, stable radix sort by tile)
     // or, with KAZAN_BINNING=sort, per-tile counts, an unordered scatter and

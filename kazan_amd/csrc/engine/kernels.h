@@ -17,10 +17,9 @@ hipError_t kz_launch_fill_rect_u32(hipStream_t st, uint32_t *dst, uint32_t width
 // offsets itself).
 hipError_t kz_launch_scan(hipStream_t st, uint32_t *counts, uint32_t *offsets, uint32_t *cursor, uint32_t n,
                           uint32_t capacity, unsigned long long *stats);
-// Radix binning, after kz_bin_count wrote f.tri_rect and f.block_pairs.
+// Radix binning, after kz_bin_count and kz_pair_scan (the pipeline's) wrote
+// f.tri_rect and the pair offsets.
 struct KzRadixScratch {
-    uint32_t *chunk_offsets;  // [ceil(tris / KZ_PAIR_CHUNK)]
-    uint32_t *chunk_extra;    // [ceil(tris / KZ_PAIR_CHUNK)]
     uint32_t *ctrl;           // KZ_BIN_WORDS
     uint32_t *tile_flag;      // [tiles], cleared with the counts before a batch
     uint32_t *keys[2], *vals[2];  // [list capacity] each
@@ -32,7 +31,7 @@ uint32_t kz_radix_blocks(uint64_t capacity);
 uint32_t kz_radix_digits_max();
 // counting-sort passes for `ntiles` keys
 uint32_t kz_radix_passes(uint32_t ntiles);
-// Pair offsets per chunk and the pairs in primitive order (2 launches).
+// The pairs in primitive order (1 launch).
 hipError_t kz_launch_bin_pairs(hipStream_t st, const KzFrame &f, const KzRadixScratch &s);
 // The passes, the last into f.tile_lists with f.tile_counts (zeroed by the
 // caller); with f.tile_acc (zeroed by the caller), the pair statistics

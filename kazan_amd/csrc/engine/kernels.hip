@@ -80,22 +80,8 @@ __device__ __forceinline__ uint32_t readlane(uint32_t v, uint32_t l) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
 }
 
-// Inclusive sum over the wave's lanes (all active), by DPP: within rows of
-// 16 lanes, then each row's last lane to the rows after it.
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
-#define KZ_DPP_ADD(ctrl, rows) v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xF, false)
-    KZ_DPP_ADD(0x111, 0xF);  // row_shr:1
-    KZ_DPP_ADD(0x112, 0xF);
-    KZ_DPP_ADD(0x114, 0xF);
-    KZ_DPP_ADD(0x118, 0xF);
-    KZ_DPP_ADD(0x142, 0xA);  // row_bcast:15 into rows 1 and 3
-    KZ_DPP_ADD(0x143, 0xC);  // row_bcast:31 into rows 2 and 3
-#undef KZ_DPP_ADD
-    return v;
-}
-
 __device__ __forceinline__ void unpack_box(uint64_t r, uint32_t &x0, uint32_t &y0, uint32_t &x1, uint32_t &y1) {
-    x0 = (uint32_t)(r & 0xFFFF);
+    x0 = (uint32_t)(r & (0xFFFF & ~KZ_RECT_PIECES));
     y0 = (uint32_t)((r >> 16) & 0xFFFF);
     x1 = (uint32_t)((r >> 32) & 0xFFFF);
     y1 = (uint32_t)(r >> 48);
@@ -596,13 +582,8 @@ __global__ __launch_bounds__(kSortThreads) void kz_sort_lists(const uint32_t *co
 
 constexpr uint32_t kPairThreads = 256;
 constexpr uint32_t kPairPer = KZ_PAIR_CHUNK / kPairThreads;  // triangles per thread
-constexpr uint32_t kPairPiece = 1024;                        // pairs one workgroup writes
 constexpr uint32_t kPairExtraGrid = 1024;                    // workgroups for the pieces after a chunk's first
 constexpr uint32_t kPairInline = 8;                          // pairs of one triangle that its own lane writes
-constexpr uint32_t kBlocksPerChunk = KZ_PAIR_CHUNK / KZ_BIN_BLOCK;
-static_assert(kBlocksPerChunk == 4, "a chunk's block counts are one 16-byte load");
-constexpr uint32_t kPairScanThreads = 1024;
-constexpr uint32_t kPairScanPer = 4;  // chunks per thread and step
 constexpr uint32_t kRadixThreads = 512;
 constexpr uint32_t kRadixWaves = kRadixThreads / 64;
 constexpr uint32_t kRadixRounds = 8;                            // pairs per lane
@@ -633,122 +614,36 @@ __device__ __forceinline__ uint32_t box_sub_mask16(uint32_t x0, uint32_t y0, uin
     return m;
 }
 
-// Pair offsets of the KZ_PAIR_CHUNK-triangle chunks (one workgroup; chunk c
-// sums blocks [c * kBlocksPerChunk, ...) of kz_bin_count). When the pairs
-// exceed `capacity`, the chunks from the first one that does not fit on are
-// cut: ctrl[KZ_BIN_CUT] is that chunk and ctrl[KZ_BIN_PAIRS] the pairs
-// before it (kz_pair_write then flags the tiles of the cut triangles).
-// chunk_extra[c]: the pieces of kPairPiece pairs after the first of all
-// chunks before c (ctrl[KZ_BIN_EXTRA] in all), which kz_pair_write gives to
-// workgroups of their own.
-// Bound by the latency of its loads: a step takes 4,096 chunks, each thread
-// 4 consecutive ones with all their loads in flight at once (8.4 M
-// triangles: two steps; 256 threads of one chunk each took 8 steps of 4,096
-// triangles a chunk, MEAS_PSCAN).
-__global__ __launch_bounds__(kPairScanThreads) void kz_pair_scan(const uint32_t *block_pairs, uint32_t ntris,
-                                                                 uint32_t *chunk_offsets, uint32_t *chunk_extra,
-                                                                 uint32_t nchunks, uint32_t capacity, uint32_t *ctrl,
-                                                                 unsigned long long *stats) {
-    __shared__ unsigned long long s_wave[kPairScanThreads / 64];
-    __shared__ uint32_t s_ewave[kPairScanThreads / 64];
-    __shared__ unsigned long long s_cut;  // first cut chunk << 32 | its offset
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t nblocks = (ntris + KZ_BIN_BLOCK - 1) / KZ_BIN_BLOCK;
-    if (tid == 0) s_cut = ~0ull;
-    unsigned long long carry = 0;
-    uint32_t ecarry = 0;
-    for (uint32_t c0 = 0; c0 < nchunks; c0 += kPairScanThreads * kPairScanPer) {
-        const uint32_t c = c0 + tid * kPairScanPer;
-        uint32_t b[kPairScanPer][kBlocksPerChunk];
-#pragma unroll
-        for (uint32_t i = 0; i < kPairScanPer; ++i) {
-            const uint32_t first = (c + i) * kBlocksPerChunk;
-            uint4 v = make_uint4(0u, 0u, 0u, 0u);
-            if (c + i < nchunks) {
-                if (first + kBlocksPerChunk <= nblocks) {
-                    v = *(const uint4 *)(block_pairs + first);
-                } else {
-                    v.x = block_pairs[first];  // (a chunk has at least one block)
-                    v.y = first + 1 < nblocks ? block_pairs[first + 1] : 0u;
-                    v.z = first + 2 < nblocks ? block_pairs[first + 2] : 0u;
-                }
-            }
-            b[i][0] = v.x;
-            b[i][1] = v.y;
-            b[i][2] = v.z;
-            b[i][3] = v.w;
-        }
-        unsigned long long v[kPairScanPer], sum = 0;
-#pragma unroll
-        for (uint32_t i = 0; i < kPairScanPer; ++i) {
-            v[i] = (unsigned long long)b[i][0] + b[i][1] + b[i][2] + b[i][3];
-            sum += v[i];
-        }
-        unsigned long long x = sum;
-        for (uint32_t d = 1; d < 64; d <<= 1) {
-            const unsigned long long o = __shfl_up(x, d, 64);
-            if (lane >= d) x += o;
-        }
-        if (lane == 63) s_wave[wave] = x;
-        __syncthreads();
-        unsigned long long run = carry + x - sum;
-        for (uint32_t w = 0; w < kPairScanThreads / 64; ++w) {
-            const unsigned long long t = s_wave[w];
-            if (w < wave) run += t;
-            carry += t;
-        }
-        // (a chunk that ends past the capacity is cut, and so are all after it)
-        uint32_t e[kPairScanPer], esum = 0;
-#pragma unroll
-        for (uint32_t i = 0; i < kPairScanPer; ++i) {
-            e[i] = 0;
-            if (c + i < nchunks) {
-                chunk_offsets[c + i] = (uint32_t)min(run, (unsigned long long)capacity);
-                if (run + v[i] > capacity)
-                    atomicMin(&s_cut, ((unsigned long long)(c + i) << 32) |
-                                          (uint32_t)min(run, (unsigned long long)capacity));
-                else if (v[i] > 2 * min(KZ_PAIR_CHUNK, ntris - (c + i) * KZ_PAIR_CHUNK))
-                    e[i] = (uint32_t)((v[i] + kPairPiece - 1) / kPairPiece) - 1u;
-            }
-            run += v[i];
-            esum += e[i];
-        }
-        const uint32_t ex = wave_incl_scan(esum);
-        if (lane == 63) s_ewave[wave] = ex;
-        __syncthreads();
-        uint32_t erun = ecarry + ex - esum;
-        for (uint32_t w = 0; w < kPairScanThreads / 64; ++w) {
-            const uint32_t t = s_ewave[w];
-            if (w < wave) erun += t;
-            ecarry += t;
-        }
-#pragma unroll
-        for (uint32_t i = 0; i < kPairScanPer; ++i) {
-            if (c + i < nchunks) chunk_extra[c + i] = erun;
-            erun += e[i];
-        }
-    }
-    __syncthreads();
-    if (tid == 0) {
-        const unsigned long long cut = s_cut;
-        const bool over = cut != ~0ull;
-        ctrl[KZ_BIN_CUT] = over ? (uint32_t)(cut >> 32) : nchunks;
-        ctrl[KZ_BIN_PAIRS] = over ? (uint32_t)cut : (uint32_t)carry;
-        ctrl[KZ_BIN_OVER] = over ? 1u : 0u;
-        ctrl[KZ_BIN_EXTRA] = ecarry;
-        if (stats) {
-            atomicAdd(&stats[KZ_STAT_LIST_ENTRIES], carry);
-            if (over) atomicAdd(&stats[KZ_STAT_LIST_OVERFLOW], 1ull);
-        }
-    }
-}
-
 // Where pairs go: keys carry the tile and, with masks (fewer than 65536
 // tiles), the pair's box_sub_mask16 in their upper 16 bits, for the split of
 // the tile's list; the sort's digits read only the tile bits.
 struct PairOut {
     uint32_t *keys, *vals;
     uint32_t sh, tiles_x, masks;
+    const uint64_t *rect;
+    const uint32_t *clip_of;
+    uint32_t ntris;
+    // pairs of triangle g, whose box is r: its box's tiles, or its pieces'
+    __device__ __forceinline__ uint32_t count(uint64_t r, uint32_t g) const {
+        if (r == KZ_RECT_EMPTY || !(r & KZ_RECT_PIECES)) return box_tiles(r, sh);
+        const uint32_t c = clip_of[g], base = ntris + (c >> 4);
+        uint32_t n = 0;
+        for (uint32_t i = 0; i < (c & 15u); ++i) n += box_tiles(rect[base + i], sh);
+        return n;
+    }
+    // of triangle g (box r), the list entry that its k-th pair belongs to
+    // (itself or a piece); r becomes that entry's box, k the pair's place in it
+    __device__ __forceinline__ uint32_t entry(uint64_t &r, uint32_t &k, uint32_t g) const {
+        if (!(r & KZ_RECT_PIECES)) return g;
+        const uint32_t c = clip_of[g], base = ntris + (c >> 4);
+        for (uint32_t i = 0; i < (c & 15u); ++i) {
+            r = rect[base + i];
+            const uint32_t t = box_tiles(r, sh);
+            if (k < t) return base + i;
+            k -= t;
+        }
+        return g;  // (k is below the triangle's count: not reached)
+    }
     __device__ __forceinline__ void put(uint32_t at, uint64_t r, uint32_t tx, uint32_t ty, uint32_t g) const {
         uint32_t x0, y0, x1, y1;
         unpack_box(r, x0, y0, x1, y1);
@@ -766,7 +661,7 @@ struct PairOut {
 // A chunk of at most two pairs a triangle (meshes of small triangles) is
 // written by its triangles' lanes, consecutive lanes to consecutive places:
 // the prefix is all it computes. A triangle of more than kPairInline tiles
-// takes its wave. The pairs of the other chunks are written kPairPiece at a
+// takes its wave. The pairs of the other chunks are written KZ_PAIR_PIECE at a
 // time, one workgroup each (the first with the chunk, the others taken in
 // turn by the workgroups past the chunks'), whose lanes find their triangle
 // by binary search over the prefix in LDS: a few hundred large triangles are
@@ -777,13 +672,14 @@ struct PairOut {
 // of 11,834 16.5 -> 6.7.
 __global__ __launch_bounds__(kPairThreads) void kz_pair_write(const uint64_t *rect, uint32_t ntris, uint32_t nchunks,
                                                               PairOut o, const uint32_t *chunk_offsets,
-                                                              const uint32_t *chunk_extra, const uint32_t *ctrl,
+                                                              const uint32_t *chunk_extra, uint32_t *ctrl,
                                                               uint32_t *tile_flag) {
     __shared__ uint64_t s_rect[KZ_PAIR_CHUNK];
     __shared__ uint32_t s_pfx[KZ_PAIR_CHUNK];
     __shared__ uint32_t s_wave[kPairPer][kPairThreads / 64];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, sh = o.sh;
     const bool first = blockIdx.x < nchunks;
+    if (blockIdx.x == 0 && tid < 2) ctrl[tid ? KZ_BIN_CLIPPED : KZ_BIN_PIECES] = 0;  // for the next batch
     const uint32_t nextra = first ? 0u : ctrl[KZ_BIN_EXTRA];
     for (uint32_t e = first ? 0u : blockIdx.x - nchunks; first || e < nextra; e += gridDim.x - nchunks) {
         uint32_t c = blockIdx.x, piece = 0;
@@ -819,8 +715,8 @@ __global__ __launch_bounds__(kPairThreads) void kz_pair_write(const uint64_t *re
         }
 #pragma unroll
         for (uint32_t j = 0; j < kPairPer; ++j) {
-            cnt[j] = box_tiles(r[j], sh);
-            const uint32_t x = wave_incl_scan(cnt[j]);
+            cnt[j] = o.count(r[j], t0 + j * kPairThreads + tid);
+            const uint32_t x = kz_wave_incl_scan(cnt[j]);
             pfx[j] = x - cnt[j];
             if (lane == 63) s_wave[j][wave] = x;
         }
@@ -841,7 +737,8 @@ __global__ __launch_bounds__(kPairThreads) void kz_pair_write(const uint64_t *re
                 uint32_t x0, y0, x1, y1;
                 unpack_box(r[j], x0, y0, x1, y1);
                 const uint32_t tx0 = x0 >> sh, tx1 = x1 >> sh;
-                if (cnt[j] <= kPairInline) {
+                const bool pieces = cnt[j] != 0 && (r[j] & KZ_RECT_PIECES);
+                if (cnt[j] <= kPairInline && !pieces) {
                     uint32_t tx = tx0, ty = y0 >> sh;
                     for (uint32_t k = 0; k < cnt[j]; ++k) {
                         o.put(out + pfx[j] + k, r[j], tx, ty, g);
@@ -849,19 +746,20 @@ __global__ __launch_bounds__(kPairThreads) void kz_pair_write(const uint64_t *re
                         tx = tx == tx1 ? tx0 : tx + 1;
                     }
                 }
-                uint64_t m = __ballot(cnt[j] > kPairInline);
+                uint64_t m = __ballot(cnt[j] > kPairInline || pieces);
                 while (m) {
                     const uint32_t b = (uint32_t)__builtin_ctzll(m);
                     m &= m - 1;
                     const uint64_t rb = (uint64_t)readlane((uint32_t)r[j], b) |
                                         ((uint64_t)readlane((uint32_t)(r[j] >> 32), b) << 32);
                     const uint32_t cb = readlane(cnt[j], b), at = out + readlane(pfx[j], b), gb = readlane(g, b);
-                    uint32_t bx0, by0, bx1, by1;
-                    unpack_box(rb, bx0, by0, bx1, by1);
-                    const uint32_t bt = bx0 >> sh, tw = (bx1 >> sh) - bt + 1;
-                    for (uint32_t k = lane; k < cb; k += 64) {
-                        const uint32_t ky = k / tw;
-                        o.put(at + k, rb, bt + k - ky * tw, (by0 >> sh) + ky, gb);
+                    for (uint32_t q = lane; q < cb; q += 64) {
+                        uint64_t re = rb;
+                        uint32_t k = q, bx0, by0, bx1, by1;
+                        const uint32_t id = o.entry(re, k, gb);
+                        unpack_box(re, bx0, by0, bx1, by1);
+                        const uint32_t bt = bx0 >> sh, tw = (bx1 >> sh) - bt + 1, ky = k / tw;
+                        o.put(at + q, re, bt + k - ky * tw, (by0 >> sh) + ky, id);
                     }
                 }
             }
@@ -873,7 +771,7 @@ __global__ __launch_bounds__(kPairThreads) void kz_pair_write(const uint64_t *re
             s_pfx[j * kPairThreads + tid] = pfx[j];
         }
         __syncthreads();
-        for (uint32_t q = piece * kPairPiece + tid; q < min(total, (piece + 1) * kPairPiece); q += kPairThreads) {
+        for (uint32_t q = piece * KZ_PAIR_PIECE + tid; q < min(total, (piece + 1) * KZ_PAIR_PIECE); q += kPairThreads) {
             // the last triangle whose prefix is <= q (s_pfx[0] = 0 <= q)
             uint32_t lo = 0, hi = KZ_PAIR_CHUNK;
             while (hi - lo > 1) {
@@ -881,12 +779,12 @@ __global__ __launch_bounds__(kPairThreads) void kz_pair_write(const uint64_t *re
                 if (s_pfx[mid] <= q) lo = mid;
                 else hi = mid;
             }
-            const uint32_t k = q - s_pfx[lo];
-            uint32_t x0, y0, x1, y1;
-            unpack_box(s_rect[lo], x0, y0, x1, y1);
-            const uint32_t tx0 = x0 >> sh, tw = (x1 >> sh) - tx0 + 1;
-            const uint32_t ky = k / tw;
-            o.put(out + q, s_rect[lo], tx0 + k - ky * tw, (y0 >> sh) + ky, t0 + lo);
+            uint64_t re = s_rect[lo];
+            uint32_t k = q - s_pfx[lo], x0, y0, x1, y1;
+            const uint32_t id = o.entry(re, k, t0 + lo);
+            unpack_box(re, x0, y0, x1, y1);
+            const uint32_t tx0 = x0 >> sh, tw = (x1 >> sh) - tx0 + 1, ky = k / tw;
+            o.put(out + q, re, tx0 + k - ky * tw, (y0 >> sh) + ky, id);
         }
         if (first) return;
         __syncthreads();  // the next piece overwrites the LDS tables
@@ -997,7 +895,7 @@ struct RadixAcc {
     const uint64_t *rect;
     const uint32_t *tri_z;
     uint32_t *acc;  // KZ_ACC words per tile, or null
-    uint32_t sh, tiles_x;
+    uint32_t sh, tiles_x, ntris;
 };
 
 // One stable counting-sort pass by the digit (key >> shift) & (2^bits - 1)
@@ -1127,7 +1025,8 @@ __global__ __launch_bounds__(kRadixThreads) void kz_radix_scatter(const uint32_t
             // six counters of at most 64 per wave, 10 bits each
             lo = bin < 3 ? 1u << (10 * bin) : 0u;
             hi = (bin >= 3 ? 1u << (10 * (bin - 3)) : 0u) + (shared << 20);
-            const uint32_t z = acc.tri_z[v];
+            // (a clip piece: depth range [0, 1], its planes are not kept)
+            const uint32_t z = v < acc.ntris ? acc.tri_z[v] : 0xFFFF0000u;
             zinv = 65535u - (z & 0xFFFFu);
             zmax = z >> 16;
         }
@@ -2237,15 +2136,14 @@ uint32_t kz_radix_passes(uint32_t ntiles) {
 hipError_t kz_launch_bin_pairs(hipStream_t st, const KzFrame &f, const KzRadixScratch &s) {
     if (f.total_tris == 0) return hipSuccess;
     const uint32_t nchunks = (f.total_tris + KZ_PAIR_CHUNK - 1) / KZ_PAIR_CHUNK;
-    kz_pair_scan<<<1, kPairScanThreads, 0, st>>>(f.block_pairs, f.total_tris, s.chunk_offsets, s.chunk_extra, nchunks,
-                                                 f.list_capacity, s.ctrl, f.stats);
     // workgroups for the pieces after the chunks' first: no more than the
     // largest pair count (and the list capacity) can make
     const uint64_t most = std::min<uint64_t>((uint64_t)f.total_tris * f.tiles_x * f.tiles_y, f.list_capacity);
-    const uint32_t extra = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(most / kPairPiece, 1), kPairExtraGrid);
-    const PairOut out{s.keys[0], s.vals[0], f.tile_shift, f.tiles_x, f.list_mask ? 1u : 0u};
-    kz_pair_write<<<nchunks + extra, kPairThreads, 0, st>>>(f.tri_rect, f.total_tris, nchunks, out, s.chunk_offsets,
-                                                            s.chunk_extra, s.ctrl, s.tile_flag);
+    const uint32_t extra = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(most / KZ_PAIR_PIECE, 1), kPairExtraGrid);
+    const PairOut out{s.keys[0],  s.vals[0], f.tile_shift, f.tiles_x, f.list_mask ? 1u : 0u,
+                      f.tri_rect, f.clip_of, f.total_tris};
+    kz_pair_write<<<nchunks + extra, kPairThreads, 0, st>>>(f.tri_rect, f.total_tris, nchunks, out, f.chunk_offsets,
+                                                            f.chunk_extra, s.ctrl, s.tile_flag);
     return hipGetLastError();
 }
 
@@ -2255,7 +2153,7 @@ hipError_t kz_launch_bin_radix(hipStream_t st, const KzFrame &f, const KzRadixSc
     while (bits < 32 && (1ull << bits) < ntiles) ++bits;
     const uint32_t passes = kz_radix_passes(ntiles);
     const uint32_t d = (bits + passes - 1) / passes;
-    RadixAcc acc{f.tri_rect, f.tri_z, f.tile_acc, f.tile_shift, f.tiles_x};
+    RadixAcc acc{f.tri_rect, f.tri_z, f.tile_acc, f.tile_shift, f.tiles_x, f.total_tris};
     for (uint32_t p = 0; p < passes; ++p) {
         const uint32_t in = p & 1u, out = in ^ 1u;
         const uint32_t shift = p * d, pb = std::min(d, bits - shift);
@@ -2267,7 +2165,7 @@ hipError_t kz_launch_bin_radix(hipStream_t st, const KzFrame &f, const KzRadixSc
             last ? f.tile_lists : nullptr, last ? (uint16_t *)f.list_mask : nullptr, last ? f.tile_counts : nullptr,
             last ? f.tile_offsets : nullptr, s.ctrl,
             s.table, s.tstride, s.totals,
-            shift, pb, last ? acc : RadixAcc{nullptr, nullptr, nullptr, 0, 0});
+            shift, pb, last ? acc : RadixAcc{nullptr, nullptr, nullptr, 0, 0, 0});
     }
     return hipGetLastError();
 }

@@ -83,20 +83,16 @@ __device__ __forceinline__ float kz_readlane_f(float v, uint32_t lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
-__device__ __forceinline__ uint32_t kz_wave_incl_scan(uint32_t v, uint32_t lane) {
-    for (uint32_t d = 1; d < 64; d <<= 1) {
-        uint32_t o = (uint32_t)kz_bperm_i((int32_t)v, lane >= d ? lane - d : lane);
-        if (lane >= d) v += o;
-    }
-    return v;
-}
-
 __device__ __forceinline__ int32_t kz_wave_max(int32_t v, uint32_t lane) {
     for (uint32_t d = 32; d > 0; d >>= 1) {
         int32_t o = kz_bperm_i(v, lane ^ d);
         v = v > o ? v : o;
     }
     return v;
+}
+
+__device__ __forceinline__ uint32_t kz_wave_sum(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)kz_wave_incl_scan(v), 63);
 }
 
 __device__ __forceinline__ unsigned long long kz_wave_sum_u64(unsigned long long v, uint32_t lane) {
@@ -583,8 +579,8 @@ __device__ __forceinline__ unsigned long long *kz_stats_stripe(const KzFrame &f)
 // list entry instead of index -> vertex -> setup again.
 #define KZ_REC_WORDS KZ_REC_WORDS_FOR(KZ_NV)
 
-__device__ __forceinline__ void kz_store_rec(const KzFrame &f, uint32_t g, const KzTri &t,
-                                             const float vary[3][KZ_NVA]) {
+__device__ __forceinline__ void kz_store_rec(uint32_t *recs, uint32_t rec, const KzTri &t, const float a0[KZ_NVA],
+                                             const float da1[KZ_NVA], const float da2[KZ_NVA]) {
     uint32_t w[KZ_REC_WORDS];
     w[0] = (uint32_t)t.x0;
     w[1] = (uint32_t)t.y0;
@@ -604,13 +600,13 @@ __device__ __forceinline__ void kz_store_rec(const KzFrame &f, uint32_t g, const
     w[15] = 0u;
 #pragma unroll
     for (int i = 0; i < KZ_NV; ++i) {
-        w[16 + 3 * i] = __float_as_uint(vary[0][i]);
-        w[17 + 3 * i] = __float_as_uint(vary[1][i] - vary[0][i]);
-        w[18 + 3 * i] = __float_as_uint(vary[2][i] - vary[0][i]);
+        w[16 + 3 * i] = __float_as_uint(a0[i]);
+        w[17 + 3 * i] = __float_as_uint(da1[i]);
+        w[18 + 3 * i] = __float_as_uint(da2[i]);
     }
 #pragma unroll
     for (int i = 16 + 3 * KZ_NV; i < KZ_REC_WORDS; ++i) w[i] = 0u;
-    uint4 *dst = (uint4 *)(f.tri_rec + (size_t)g * KZ_REC_WORDS);
+    uint4 *dst = (uint4 *)(recs + (size_t)rec * KZ_REC_WORDS);
 #pragma unroll
     for (int q = 0; q < KZ_REC_WORDS / 4; ++q) dst[q] = make_uint4(w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]);
 }
@@ -649,12 +645,13 @@ __device__ __forceinline__ void kz_load_clip_rec(const KzFrame &f, uint32_t g, f
     }
 }
 
-// The record of triangle g and its pixel box: the values kz_setup and the
-// varying differences gave when the record was written. Returns whether the
-// triangle needs clipping (its other values are then meaningless).
-__device__ __forceinline__ bool kz_load_rec(const KzFrame &f, uint32_t g, KzTri &t, float *a0, float *da1,
-                                            float *da2) {
-    const uint4 *src = (const uint4 *)(f.tri_rec + (size_t)g * KZ_REC_WORDS);
+// The record of triangle g (the rec-th of recs) and its pixel box: the values
+// kz_setup and the varying differences gave when the record was written.
+// Returns whether the triangle needs clipping (its other values are then
+// meaningless).
+__device__ __forceinline__ bool kz_load_rec(const KzFrame &f, const uint32_t *recs, uint32_t rec, uint32_t g,
+                                            KzTri &t, float *a0, float *da1, float *da2) {
+    const uint4 *src = (const uint4 *)(recs + (size_t)rec * KZ_REC_WORDS);
     uint32_t w[KZ_REC_WORDS];
 #pragma unroll
     for (int q = 0; q < KZ_REC_WORDS / 4; ++q) {
@@ -748,7 +745,15 @@ extern "C" __global__ __launch_bounds__(KZ_BIN_BLOCK) void kz_bin_count(KzFrame 
             if (t.px0 <= t.px1 && t.py0 <= t.py1) {
                 rect = (uint64_t)(uint32_t)t.px0 | ((uint64_t)(uint32_t)t.py0 << 16) |
                        ((uint64_t)(uint32_t)t.px1 << 32) | ((uint64_t)(uint32_t)t.py1 << 48);
-                if (KZ_SETUP_RECORDS && f.tri_rec) kz_store_rec(f, g, t, vary);
+                if (KZ_SETUP_RECORDS && f.tri_rec) {
+                    float da1[KZ_NVA], da2[KZ_NVA];
+#pragma unroll
+                    for (int i = 0; i < KZ_NV; ++i) {
+                        da1[i] = vary[1][i] - vary[0][i];
+                        da2[i] = vary[2][i] - vary[0][i];
+                    }
+                    kz_store_rec(f.tri_rec, g, t, vary[0], da1, da2);
+                }
             }
             if (f.tri_z) {  // cost-model feature: the triangle's depth range
                 const float z1 = t.z0 + t.dz1, z2 = t.z0 + t.dz2;
@@ -759,8 +764,11 @@ extern "C" __global__ __launch_bounds__(KZ_BIN_BLOCK) void kz_bin_count(KzFrame 
         }
     }
     // Triangles that need clipping: the whole wave clips each in turn (lane
-    // j sets up piece j); the triangle is binned by the union of its
-    // pieces' pixel boxes, and counts as set up when one of them is.
+    // j sets up piece j), and the triangle counts as set up when one of its
+    // pieces is. Its pieces with a pixel box become list entries of their
+    // own (kz_pair_scan writes their records); without room for them the
+    // triangle is binned by the union of their boxes and the raster clips it
+    // again in every tile.
     uint64_t cm = kz_ballot(st == 2);
     while (cm) {
         const uint32_t b = (uint32_t)__builtin_ctzll(cm);
@@ -777,6 +785,31 @@ extern "C" __global__ __launch_bounds__(KZ_BIN_BLOCK) void kz_bin_count(KzFrame 
         const int32_t bx1 = kz_wave_max(boxed ? pt.px1 : none, lane);
         const int32_t by1 = kz_wave_max(boxed ? pt.py1 : none, lane);
         const bool any = kz_ballot(piece) != 0;
+        const uint64_t mb = kz_ballot(boxed);
+        const uint32_t npc = (uint32_t)__popcll(mb);
+        bool kept = false;
+        if (f.clip_cap && npc) {
+            uint32_t base = 0;
+            if (lane == b) base = atomicAdd(&f.bin_ctrl[KZ_BIN_PIECES], npc);
+            base = (uint32_t)kz_readlane_i((int32_t)base, b);
+            kept = base < f.clip_cap && npc <= f.clip_cap - base;
+            if (kept) {
+                uint32_t tiles = 0;
+                if (boxed) {
+                    f.tri_rect[f.total_tris + base + kz_rank(mb)] =
+                        (uint64_t)(uint32_t)pt.px0 | ((uint64_t)(uint32_t)pt.py0 << 16) |
+                        ((uint64_t)(uint32_t)pt.px1 << 32) | ((uint64_t)(uint32_t)pt.py1 << 48);
+                    tiles = (uint32_t)(((pt.px1 >> KZ_TILE_SHIFT) - (pt.px0 >> KZ_TILE_SHIFT) + 1) *
+                                       ((pt.py1 >> KZ_TILE_SHIFT) - (pt.py0 >> KZ_TILE_SHIFT) + 1));
+                }
+                tiles = kz_wave_sum(tiles);
+                if (lane == b) {
+                    f.clip_of[g] = base << 4 | npc;
+                    f.clip_tris[atomicAdd(&f.bin_ctrl[KZ_BIN_CLIPPED], 1u)] = g;
+                    n_pairs = tiles;
+                }
+            }
+        }
         if (lane == b) {
             n_clip = 1;
             n_setup = any ? 1 : 0;
@@ -786,7 +819,7 @@ extern "C" __global__ __launch_bounds__(KZ_BIN_BLOCK) void kz_bin_count(KzFrame 
                 t.px1 = bx1;
                 t.py1 = by1;
                 rect = (uint64_t)(uint32_t)bx0 | ((uint64_t)(uint32_t)by0 << 16) | ((uint64_t)(uint32_t)bx1 << 32) |
-                       ((uint64_t)(uint32_t)by1 << 48);
+                       ((uint64_t)(uint32_t)by1 << 48) | (kept ? KZ_RECT_PIECES : 0ull);
             }
         }
     }
@@ -796,8 +829,8 @@ extern "C" __global__ __launch_bounds__(KZ_BIN_BLOCK) void kz_bin_count(KzFrame 
             if (f.tri_z) f.tri_z[g] = 0xFFFF0000u;  // depth range [0, 1]: the pieces are not kept
         }
         f.tri_rect[g] = rect;
-        // (triangle, tile) pairs: the tiles of the pixel box
-        if (rect != KZ_RECT_EMPTY)
+        // (triangle, tile) pairs: the tiles of the pixel box (or of the pieces')
+        if (rect != KZ_RECT_EMPTY && !(rect & KZ_RECT_PIECES))
             n_pairs = (uint32_t)(((t.px1 >> KZ_TILE_SHIFT) - (t.px0 >> KZ_TILE_SHIFT) + 1) *
                                  ((t.py1 >> KZ_TILE_SHIFT) - (t.py0 >> KZ_TILE_SHIFT) + 1));
     }
@@ -1073,7 +1106,7 @@ struct KzLaneTri {
 // Does pixel box r overlap the square [X0, X0 + RW) x [Y0, Y0 + RW)?
 __device__ __forceinline__ bool kz_box_overlaps(uint64_t r, int32_t X0, int32_t Y0, int32_t RW) {
     if (r == KZ_RECT_EMPTY) return false;
-    const int32_t x0 = (int32_t)(r & 0xFFFF), y0 = (int32_t)((r >> 16) & 0xFFFF);
+    const int32_t x0 = (int32_t)(r & (0xFFFF & ~KZ_RECT_PIECES)), y0 = (int32_t)((r >> 16) & 0xFFFF);
     const int32_t x1 = (int32_t)((r >> 32) & 0xFFFF), y1 = (int32_t)(r >> 48);
     return x1 >= X0 && x0 < X0 + RW && y1 >= Y0 && y0 < Y0 + RW;
 }
@@ -1104,7 +1137,7 @@ __device__ __forceinline__ void kz_ahead_ids(KzAhead &a, const uint32_t *ids, ui
 __device__ __forceinline__ void kz_ahead_indices(KzAhead &a, const KzFrame &f) {
     a.draw = 0;
     a.idx[0] = a.idx[1] = a.idx[2] = 0;
-    if (!a.valid || (KZ_SETUP_RECORDS && f.tri_rec)) return;
+    if (!a.valid || (KZ_SETUP_RECORDS && f.tri_rec) || a.g >= f.total_tris) return;  // (a clip piece has a record)
     a.draw = kz_draw_of(f, a.g);
     kz_triangle_indices(f, a.g, a.draw, a.idx);
 }
@@ -1288,6 +1321,147 @@ __device__ __forceinline__ KzClipBatch kz_clip_batch(const KzFrame &f, uint32_t 
     return o;
 }
 
+// ---------------------------------------------------------------------------
+// binning, pass 2: pair offsets and the clip pieces' records (one launch)
+
+#define KZ_PAIR_SCAN_THREADS 1024
+#define KZ_PAIR_SCAN_PER 4  // chunks per thread and step
+#define KZ_CHUNK_BLOCKS (KZ_PAIR_CHUNK / KZ_BIN_BLOCK)
+static_assert(KZ_CHUNK_BLOCKS == 4, "a chunk's block counts are one 16-byte load");
+
+__device__ __forceinline__ unsigned long long kz_min64(unsigned long long a, unsigned long long b) {
+    return a < b ? a : b;
+}
+
+// The setup records of the clip pieces kz_bin_count reserved, one wave per
+// triangle (lane j: its piece j), by the raster's own clip and setup, so that
+// a tile's raster loads a piece as one lane of an ordinary batch. Clipped in
+// every tile instead, each such triangle was a batch of its own there and
+// ended the batch before it: a frame of 40,400 triangles around a camera, 400
+// of them large and most of those clipped, 1127 us -> 645.
+__device__ __forceinline__ void kz_clip_records(const KzFrame &f, uint32_t first, uint32_t step) {
+    const uint32_t lane = kz_lane(), n = f.clip_cap ? f.bin_ctrl[KZ_BIN_CLIPPED] : 0u;
+    for (uint32_t i = first; i < n; i += step) {
+        const uint32_t g = f.clip_tris[i];
+        const KzClipBatch cb = kz_clip_batch(f, g, 0, lane);
+        // (the pieces with a pixel box, as kz_bin_count numbered them)
+        const bool boxed = cb.ok && cb.t.px0 <= cb.t.px1 && cb.t.py0 <= cb.t.py1;
+        const uint32_t at = (f.clip_of[g] >> 4) + kz_rank(kz_ballot(boxed));
+        if (boxed) kz_store_rec(f.clip_rec, at, cb.t, cb.a0, cb.da1, cb.da2);
+    }
+}
+
+// Pair offsets of the KZ_PAIR_CHUNK-triangle chunks (workgroup 0; chunk c sums
+// its 4 blocks of kz_bin_count). When the pairs
+// exceed `capacity`, the chunks from the first one that does not fit on are
+// cut: ctrl[KZ_BIN_CUT] is that chunk and ctrl[KZ_BIN_PAIRS] the pairs
+// before it (kz_pair_write then flags the tiles of the cut triangles).
+// chunk_extra[c]: the pieces of KZ_PAIR_PIECE pairs after the first of all
+// chunks before c (ctrl[KZ_BIN_EXTRA] in all), which kz_pair_write gives to
+// workgroups of their own.
+// Bound by the latency of its loads: a step takes 4,096 chunks, each thread
+// 4 consecutive ones with all their loads in flight at once (8.4 M
+// triangles: two steps; 256 threads of one chunk each took 8 steps of 4,096
+// triangles a chunk, MEAS_PSCAN).
+extern "C" __global__ __launch_bounds__(KZ_PAIR_SCAN_THREADS) void kz_pair_scan(KzFrame f) {
+    if (blockIdx.x > 0) {
+        kz_clip_records(f, (blockIdx.x - 1) * (KZ_PAIR_SCAN_THREADS / 64) + (threadIdx.x >> 6),
+                        (gridDim.x - 1) * (KZ_PAIR_SCAN_THREADS / 64));
+        return;
+    }
+    const uint32_t nblocks = (f.total_tris + KZ_BIN_BLOCK - 1) / KZ_BIN_BLOCK;
+    const uint32_t nchunks = (f.total_tris + KZ_PAIR_CHUNK - 1) / KZ_PAIR_CHUNK, capacity = f.list_capacity;
+    __shared__ unsigned long long s_wave[KZ_PAIR_SCAN_THREADS / 64];
+    __shared__ uint32_t s_ewave[KZ_PAIR_SCAN_THREADS / 64];
+    __shared__ unsigned long long s_cut;  // first cut chunk << 32 | its offset
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid == 0) s_cut = ~0ull;
+    unsigned long long carry = 0;
+    uint32_t ecarry = 0;
+    for (uint32_t c0 = 0; c0 < nchunks; c0 += KZ_PAIR_SCAN_THREADS * KZ_PAIR_SCAN_PER) {
+        const uint32_t c = c0 + tid * KZ_PAIR_SCAN_PER;
+        uint32_t b[KZ_PAIR_SCAN_PER][KZ_CHUNK_BLOCKS];
+#pragma unroll
+        for (uint32_t i = 0; i < KZ_PAIR_SCAN_PER; ++i) {
+            const uint32_t first = (c + i) * KZ_CHUNK_BLOCKS;
+            uint4 v = make_uint4(0u, 0u, 0u, 0u);
+            if (c + i < nchunks) {
+                if (first + KZ_CHUNK_BLOCKS <= nblocks) {
+                    v = *(const uint4 *)(f.block_pairs + first);
+                } else {
+                    v.x = f.block_pairs[first];  // (a chunk has at least one block)
+                    v.y = first + 1 < nblocks ? f.block_pairs[first + 1] : 0u;
+                    v.z = first + 2 < nblocks ? f.block_pairs[first + 2] : 0u;
+                }
+            }
+            b[i][0] = v.x;
+            b[i][1] = v.y;
+            b[i][2] = v.z;
+            b[i][3] = v.w;
+        }
+        unsigned long long v[KZ_PAIR_SCAN_PER], sum = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < KZ_PAIR_SCAN_PER; ++i) {
+            v[i] = (unsigned long long)b[i][0] + b[i][1] + b[i][2] + b[i][3];
+            sum += v[i];
+        }
+        unsigned long long x = sum;
+        for (uint32_t d = 1; d < 64; d <<= 1) {
+            const unsigned long long o = __shfl_up(x, d, 64);
+            if (lane >= d) x += o;
+        }
+        if (lane == 63) s_wave[wave] = x;
+        __syncthreads();
+        unsigned long long run = carry + x - sum;
+        for (uint32_t w = 0; w < KZ_PAIR_SCAN_THREADS / 64; ++w) {
+            const unsigned long long t = s_wave[w];
+            if (w < wave) run += t;
+            carry += t;
+        }
+        // (a chunk that ends past the capacity is cut, and so are all after it)
+        uint32_t e[KZ_PAIR_SCAN_PER], esum = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < KZ_PAIR_SCAN_PER; ++i) {
+            e[i] = 0;
+            if (c + i < nchunks) {
+                f.chunk_offsets[c + i] = (uint32_t)kz_min64(run, (unsigned long long)capacity);
+                if (run + v[i] > capacity)
+                    atomicMin(&s_cut, ((unsigned long long)(c + i) << 32) |
+                                          (uint32_t)kz_min64(run, (unsigned long long)capacity));
+                else if (v[i] > 2 * min(KZ_PAIR_CHUNK, f.total_tris - (c + i) * KZ_PAIR_CHUNK))
+                    e[i] = (uint32_t)((v[i] + KZ_PAIR_PIECE - 1) / KZ_PAIR_PIECE) - 1u;
+            }
+            run += v[i];
+            esum += e[i];
+        }
+        const uint32_t ex = kz_wave_incl_scan(esum);
+        if (lane == 63) s_ewave[wave] = ex;
+        __syncthreads();
+        uint32_t erun = ecarry + ex - esum;
+        for (uint32_t w = 0; w < KZ_PAIR_SCAN_THREADS / 64; ++w) {
+            const uint32_t t = s_ewave[w];
+            if (w < wave) erun += t;
+            ecarry += t;
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < KZ_PAIR_SCAN_PER; ++i) {
+            if (c + i < nchunks) f.chunk_extra[c + i] = erun;
+            erun += e[i];
+        }
+    }
+    __syncthreads();
+    if (tid == 0) {
+        const unsigned long long cut = s_cut;
+        const bool over = cut != ~0ull;
+        f.bin_ctrl[KZ_BIN_CUT] = over ? (uint32_t)(cut >> 32) : nchunks;
+        f.bin_ctrl[KZ_BIN_PAIRS] = over ? (uint32_t)cut : (uint32_t)carry;
+        f.bin_ctrl[KZ_BIN_OVER] = over ? 1u : 0u;
+        f.bin_ctrl[KZ_BIN_EXTRA] = ecarry;
+        atomicAdd(&f.stats[KZ_STAT_LIST_ENTRIES], carry);
+        if (over) atomicAdd(&f.stats[KZ_STAT_LIST_OVERFLOW], 1ull);
+    }
+}
+
 // Rasterises n triangles into the square of side 1 << RS at (X0, Y0) (a
 // whole tile, or a sub-tile of the balanced mode), in primitive order. The
 // triangles are ids[0, n) (ids = null: triangles 0 .. n-1); with `filter`,
@@ -1339,7 +1513,7 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
                 k += 64;
                 continue;
             }
-            if (valid && !(KZ_SETUP_RECORDS && f.tri_rec)) {
+            if (valid && !(KZ_SETUP_RECORDS && f.tri_rec) && g < f.total_tris) {
                 draw = kz_draw_of(f, g);
                 kz_triangle_indices(f, g, draw, idx);
             }
@@ -1372,7 +1546,7 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
             L.t.px1 = L.t.py1 = -1;
 #pragma unroll
             for (int i = 0; i < KZ_NVA; ++i) L.a0[i] = L.da1[i] = L.da2[i] = 0.0f;
-            if (valid) clip = kz_load_rec(f, g, L.t, L.a0, L.da1, L.da2);
+            if (valid) clip = kz_load_rec(f, f.tri_rec, g, g, L.t, L.a0, L.da1, L.da2);
             ok = valid && !clip;
         } else {
             kz_fetch_vertices(f, draw, idx, p, vary);
@@ -1387,8 +1561,18 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
                 L.da1[i] = i < KZ_NV ? vary[1][i] - vary[0][i] : 0.0f;
                 L.da2[i] = i < KZ_NV ? vary[2][i] - vary[0][i] : 0.0f;
             }
+            // clip pieces: their records (their lanes ran the above on vertex
+            // indices 0, as lanes without a triangle do)
+            const bool piece = valid && g >= f.total_tris;
+            if (kz_ballot(piece)) {
+                if (piece) {
+                    kz_load_rec(f, f.clip_rec, g - f.total_tris, g, L.t, L.a0, L.da1, L.da2);
+                    ok = true;
+                    clip = false;
+                }
+            }
         }
-        // A triangle that needs clipping is drawn as its own batch of
+        // A triangle that needs clipping (and has no pieces) is drawn as its own batch of
         // pieces (lane j: piece ks + j), in its place: a batch whose first
         // triangle needs it draws that triangle's pieces (out of line), any
         // other batch ends before its first such triangle.
@@ -1519,7 +1703,7 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
         }
 
         // --- batch cut: keep the longest lane prefix whose fragments fit ---
-        const uint32_t incl = kz_wave_incl_scan(cnt, lane);
+        const uint32_t incl = kz_wave_incl_scan(cnt);
         // (a batch that is not a clip batch also ends before its first
         // triangle that needs clipping)
         const uint32_t take = min((uint32_t)__popcll(kz_ballot(incl <= KZ_FRAG_CAP)), clip_batch ? 64u : first_clip);
