@@ -83,25 +83,29 @@ __device__ __forceinline__ float kz_readlane_f(float v, uint32_t lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
-__device__ __forceinline__ int32_t kz_wave_max(int32_t v, uint32_t lane) {
-    for (uint32_t d = 32; d > 0; d >>= 1) {
-        int32_t o = kz_bperm_i(v, lane ^ d);
-        v = v > o ? v : o;
-    }
-    return v;
+// The wave's largest v, by DPP as kz_wave_incl_scan (all lanes active).
+__device__ __forceinline__ int32_t kz_wave_max(int32_t v) {
+#define KZ_DPP_MAX(ctrl, rows) v = max(v, __builtin_amdgcn_update_dpp(v, v, ctrl, rows, 0xF, false))
+    KZ_DPP_MAX(0x111, 0xF);
+    KZ_DPP_MAX(0x112, 0xF);
+    KZ_DPP_MAX(0x114, 0xF);
+    KZ_DPP_MAX(0x118, 0xF);
+    KZ_DPP_MAX(0x142, 0xA);
+    KZ_DPP_MAX(0x143, 0xC);
+#undef KZ_DPP_MAX
+    return __builtin_amdgcn_readlane(v, 63);
 }
 
 __device__ __forceinline__ uint32_t kz_wave_sum(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_readlane((int)kz_wave_incl_scan(v), 63);
 }
 
-__device__ __forceinline__ unsigned long long kz_wave_sum_u64(unsigned long long v, uint32_t lane) {
-    for (uint32_t d = 32; d > 0; d >>= 1) {
-        uint32_t lo = (uint32_t)kz_bperm_i((int32_t)(uint32_t)v, lane ^ d);
-        uint32_t hi = (uint32_t)kz_bperm_i((int32_t)(uint32_t)(v >> 32), lane ^ d);
-        v += ((unsigned long long)hi << 32) | lo;
-    }
-    return v;
+// samples set in the wave's masks (wave-uniform)
+__device__ __forceinline__ uint32_t kz_wave_samples(uint32_t mask) {
+    uint32_t n = 0;
+#pragma unroll
+    for (int s = 0; s < KZ_SAMPLES; ++s) n += (uint32_t)__popcll(kz_ballot((mask >> s) & 1u));
+    return n;
 }
 
 // ---------------------------------------------------------------------------
@@ -400,11 +404,14 @@ __device__ __forceinline__ void kz_edges_f(bool narrow, int32_t x0, int32_t y0, 
         f12 = (float)((int32_t)S - a - b);
         return;
     }
-    int64_t e01, e20, e12;
-    kz_edges(x0, y0, d1x, d1y, d2x, d2y, S, sx, sy, e01, e20, e12);
-    f01 = (float)e01;
-    f20 = (float)e20;
-    f12 = (float)e12;
+    // The values are below 2^38, so f64 arithmetic is exact and its
+    // conversion rounds as the int64 one does; it takes about 20
+    // instructions where 64-bit integer products and conversions took 70.
+    const double rx = (double)(sx - x0), ry = (double)(sy - y0);
+    const double a = (double)d1x * ry - (double)d1y * rx, b = (double)d2y * rx - (double)d2x * ry;
+    f01 = (float)a;
+    f20 = (float)b;
+    f12 = (float)((double)S - a - b);
 }
 
 __device__ __forceinline__ bool kz_inside(int64_t e01, int64_t e20, int64_t e12, int32_t flip, int32_t th01,
@@ -780,10 +787,10 @@ extern "C" __global__ __launch_bounds__(KZ_BIN_BLOCK) void kz_bin_count(KzFrame 
         const bool piece = (int)lane + 2 < np && kz_setup_rt(f, q, pt, true) == 1;
         const bool boxed = piece && pt.px0 <= pt.px1 && pt.py0 <= pt.py1;
         const int32_t none = -0x40000000;  // below any pixel coordinate (an empty box when no piece has one)
-        const int32_t bx0 = -kz_wave_max(boxed ? -pt.px0 : none, lane);
-        const int32_t by0 = -kz_wave_max(boxed ? -pt.py0 : none, lane);
-        const int32_t bx1 = kz_wave_max(boxed ? pt.px1 : none, lane);
-        const int32_t by1 = kz_wave_max(boxed ? pt.py1 : none, lane);
+        const int32_t bx0 = -kz_wave_max(boxed ? -pt.px0 : none);
+        const int32_t by0 = -kz_wave_max(boxed ? -pt.py0 : none);
+        const int32_t bx1 = kz_wave_max(boxed ? pt.px1 : none);
+        const int32_t by1 = kz_wave_max(boxed ? pt.py1 : none);
         const bool any = kz_ballot(piece) != 0;
         const uint64_t mb = kz_ballot(boxed);
         const uint32_t npc = (uint32_t)__popcll(mb);
@@ -1174,8 +1181,8 @@ __device__ __forceinline__ bool kz_shade(const KzFrame &f, int32_t px, int32_t p
 template <bool NARROW>
 __device__ __forceinline__ void kz_resolve(const KzFrame &f, const KzLaneTri &L, int32_t X0, int32_t Y0,
                                            uint32_t total, uint32_t lane, uint32_t *s_color, float *s_depth,
-                                           uint32_t *s_claim, const uint32_t *s_frag, uint32_t &nfrag,
-                                           uint32_t &npass) {
+                                           uint32_t *s_claim, const uint32_t *s_frag,
+                                           unsigned long long &nfrag, unsigned long long &npass) {
     for (uint32_t c0 = 0; c0 < total; c0 += 64) {
         const uint32_t qi = c0 + lane;
         const bool active = qi < total;
@@ -1211,7 +1218,7 @@ __device__ __forceinline__ void kz_resolve(const KzFrame &f, const KzLaneTri &L,
                 zs[s] = fminf(fmaxf(z, f.z_lo), f.z_hi);
             }
         }
-        nfrag += (uint32_t)__popc(mask);
+        nfrag += KZ_SAMPLES == 1 ? min(total - c0, 64u) : kz_wave_samples(mask);
 
         // The samples that can still pass the depth test: those that pass
         // against the depth the tile holds now. The round's earlier
@@ -1280,7 +1287,100 @@ __device__ __forceinline__ void kz_resolve(const KzFrame &f, const KzLaneTri &L,
             }
             __syncthreads();
         }
-        npass += (uint32_t)__popc(pass);
+        npass += kz_wave_samples(pass);
+    }
+}
+
+// Draws the triangles of the lanes m, in lane order, without the fragment
+// queue: 64 candidate pixels at a time, their coverage, depth test, shading
+// and blend at once. A triangle's pixels are all different, so there is
+// nothing to order within it, and its constants are wave-uniform: no queue
+// entry, no second coverage pass, no gathers and no claims per fragment. It
+// leaves lanes idle where a candidate is not covered, so it is for batches
+// of larger triangles (the rule is in kz_raster_rect): raster of 1,024 large
+// triangles at 256^2 128 us -> 69; a frame of 40,400 triangles around a
+// camera 645 -> 267.
+__device__ __forceinline__ void kz_direct(const KzFrame &f, const KzLaneTri &L, const KzTileCov &lc, bool narrow,
+                                          int32_t X0, int32_t Y0, uint64_t m, uint32_t lane, uint32_t *s_color,
+                                          float *s_depth, unsigned long long &nfrag,
+                                          unsigned long long &npass) {
+    while (m) {
+        const uint32_t b = (uint32_t)__builtin_ctzll(m);
+        m &= m - 1;
+        const KzTileCov cb = kz_tile_cov_of(lc, b);
+        const int32_t bx0 = kz_readlane_i(L.cx0, b) - X0, by0 = kz_readlane_i(L.cy0, b) - Y0;
+        const int32_t bw = kz_readlane_i(L.cx1, b) - X0 - bx0 + 1;
+        const int32_t bc = bw * (kz_readlane_i(L.cy1, b) - Y0 - by0 + 1);
+        // (candidate i's row as in phase 1 of kz_raster_rect)
+        const float rbw = __builtin_amdgcn_rcpf((float)bw);
+        for (int32_t i0 = 0; i0 < bc; i0 += 64) {
+            const int32_t i = i0 + (int32_t)lane;
+            const int32_t dy = (int32_t)(((float)i + 0.5f) * rbw);
+            const int32_t lx = bx0 + i - dy * bw, ly = by0 + dy;
+            const uint32_t mask = i < bc ? kz_tile_mask(cb, lx, ly) : 0u;
+            if (kz_ballot(mask != 0) == 0) continue;
+            nfrag += kz_wave_samples(mask);
+            const uint32_t pix = mask ? (uint32_t)(ly * KZ_TS + lx) : 0u;
+            const int32_t px = X0 + lx, py = Y0 + ly;
+            const int32_t x0 = kz_readlane_i(L.t.x0, b), y0 = kz_readlane_i(L.t.y0, b);
+            const int32_t d1x = kz_readlane_i(L.t.d1x, b), d1y = kz_readlane_i(L.t.d1y, b);
+            const int32_t d2x = kz_readlane_i(L.t.d2x, b), d2y = kz_readlane_i(L.t.d2y, b);
+            const int32_t s_lo = kz_readlane_i((int32_t)(uint32_t)(uint64_t)L.t.S, b);
+            const int32_t s_hi = kz_readlane_i((int32_t)((uint64_t)L.t.S >> 32), b);
+            const int64_t S = (int64_t)(((uint64_t)(uint32_t)s_lo) | ((uint64_t)(uint32_t)s_hi << 32));
+            const float invS = kz_readlane_f(L.t.invS, b);
+            const float z0 = kz_readlane_f(L.t.z0, b), dz1 = kz_readlane_f(L.t.dz1, b), dz2 = kz_readlane_f(L.t.dz2, b);
+            float zs[KZ_SAMPLES], c01 = 0.0f, c20 = 0.0f, c12 = 0.0f;
+            uint32_t maybe = 0;
+#pragma unroll
+            for (int s = 0; s < KZ_SAMPLES; ++s) {
+                float e01, e20, e12;
+                kz_edges_f(narrow, x0, y0, d1x, d1y, d2x, d2y, S, px * 16 + kz_sample_x[s], py * 16 + kz_sample_y[s],
+                           e01, e20, e12);
+                if (KZ_SAMPLES == 1) {
+                    c01 = e01;
+                    c20 = e20;
+                    c12 = e12;
+                }
+                const float l1 = e20 * invS, l2 = e01 * invS;
+                zs[s] = fminf(fmaxf((z0 + l1 * dz1) + l2 * dz2, f.z_lo), f.z_hi);
+                bool ok = (mask >> s) & 1u;
+#if KZ_DEPTH_TEST
+                ok = ok && kz_depth_cmp(zs[s], s_depth[pix * KZ_SAMPLES + s]);
+#endif
+                maybe |= ok ? 1u << s : 0u;
+            }
+            if (kz_ballot(maybe != 0) == 0) continue;
+            float a0[KZ_NVA], da1[KZ_NVA], da2[KZ_NVA];
+#pragma unroll
+            for (int v = 0; v < KZ_NV; ++v) {
+                a0[v] = kz_readlane_f(L.a0[v], b);
+                da1[v] = kz_readlane_f(L.da1[v], b);
+                da2[v] = kz_readlane_f(L.da2[v], b);
+            }
+            const float iw0 = kz_readlane_f(L.t.iw0, b), iw1 = kz_readlane_f(L.t.iw1, b),
+                        iw2 = kz_readlane_f(L.t.iw2, b);
+            uint32_t pass = 0;
+            if (maybe) {
+                float col[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                float e01 = c01, e20 = c20, e12 = c12;
+                if (KZ_SAMPLES != 1)
+                    kz_edges_f(narrow, x0, y0, d1x, d1y, d2x, d2y, S, px * 16 + 8, py * 16 + 8, e01, e20, e12);
+                if (kz_shade(f, px, py, e01, e20, e12, invS, z0, dz1, dz2, iw0, iw1, iw2, a0, da1, da2, col)) {
+#pragma unroll
+                    for (int s = 0; s < KZ_SAMPLES; ++s) {
+                        if (!((maybe >> s) & 1u)) continue;
+#if KZ_DEPTH_TEST && KZ_DEPTH_WRITE
+                        s_depth[pix * KZ_SAMPLES + s] = zs[s];
+#endif
+                        s_color[pix * KZ_SAMPLES + s] = kz_rop(s_color[pix * KZ_SAMPLES + s], col);
+                    }
+                    pass = maybe;
+                }
+            }
+            npass += kz_wave_samples(pass);
+        }
+        __syncthreads();  // the next triangle reads what this one wrote
     }
 }
 
@@ -1496,7 +1596,7 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
     }
     __syncthreads();
 
-    unsigned long long nfrag = 0, npass = 0;
+    unsigned long long nfrag = 0, npass = 0;  // (wave-uniform)
     // a scan of the triangles (filter without ids) starts at the first cut
     // chunk's first triangle: the ones before it were in the tile's list
     uint32_t k = filter && !ids && f.bin_ctrl ? min(f.bin_ctrl[KZ_BIN_CUT] * KZ_PAIR_CHUNK, n) : 0u;
@@ -1608,6 +1708,45 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
         // edges: edges are evaluated in 32 bits
         const bool narrow = kz_ballot(L.live && !kz_small_deltas(L.t.d1x, L.t.d1y, L.t.d2x, L.t.d2y)) == 0;
         const KzTileCov lc = kz_tile_cov(L.t, X0, Y0, narrow);
+        // A larger triangle whose box meets the square need not: none of its
+        // candidates is covered when one of its edges has them all outside
+        // (the largest edge value is at a corner of their samples' box).
+        uint64_t livem = kz_ballot(L.live), bigm = kz_ballot(L.live && !small);
+        if (bigm) {
+            const int32_t lo = KZ_SAMPLES == 4 ? 2 : 8, hi = KZ_SAMPLES == 4 ? 14 : 8;
+            const int32_t dx0 = (L.cx0 - X0) * 16 + lo, dx1 = (L.cx1 - X0) * 16 + hi;
+            const int32_t dy0 = (L.cy0 - Y0) * 16 + lo, dy1 = (L.cy1 - Y0) * 16 + hi;
+            bool out = false;
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                out |= __mul24(lc.a[e], lc.a[e] > 0 ? dx1 : dx0) + __mul24(lc.b[e], lc.b[e] > 0 ? dy1 : dy0) < lc.k[e];
+            const uint64_t outm = kz_ballot(out && !small);
+            bigm &= ~outm;
+            livem &= ~outm;
+        }
+        // A batch of mostly larger triangles is drawn triangle by triangle
+        // where the lanes that leaves idle cost little: the triangles fill
+        // the square (their boxes cover half of it and more), or most
+        // fragments fail the depth test (three in four so far) and end there.
+        // A textured grid of 10 px triangles, all of them visible and half
+        // of their candidates covered, stays with the queue: 29 us, against 41.
+        bool direct = bigm != 0 && 2 * __popcll(bigm) >= __popcll(livem);
+        if (direct)
+            direct = 2u * kz_wave_sum((bigm >> lane) & 1ull ? (uint32_t)cand : 0u) >=
+                         (uint32_t)__popcll(bigm) * (uint32_t)(RW * RW) ||
+                     4u * npass < nfrag;
+        if (direct) {
+            if (clip_batch) {
+                ks = ks + 64 < npieces ? ks + 64 : 0u;
+                k = ks ? k : k + 1;
+            } else {
+                k += first_clip;
+            }
+            if (!filter && nx.k != k) kz_ahead_ids(nx, ids, k, n, lane);
+            if (!filter) kz_ahead_indices(nx, f);
+            kz_direct(f, L, lc, narrow, X0, Y0, livem, lane, s_color, s_depth, nfrag, npass);
+            continue;
+        }
 
         // --- phase 1: covered pixels per triangle ------------------------
         // (small triangles keep their sample masks, KZ_SAMPLES bits per
@@ -1616,7 +1755,7 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
         KzCandMask cmask = 0;
         {
             // (the wave's longest walk, a scalar loop bound)
-            const int32_t maxc = __builtin_amdgcn_readfirstlane(kz_wave_max(small ? cand : 0, lane));
+            const int32_t maxc = kz_wave_max(small ? cand : 0);
             KzWalk wk;
 #if KZ_SAMPLES == 1
             // Every lane steps maxc times (a lane that walks nothing, or
@@ -1677,10 +1816,8 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
             }
 #endif
         }
-        uint64_t bigm = kz_ballot(L.live && !small);
-        while (bigm) {
-            const uint32_t b = (uint32_t)__builtin_ctzll(bigm);
-            bigm &= bigm - 1;
+        for (uint64_t m = bigm; m; m &= m - 1) {
+            const uint32_t b = (uint32_t)__builtin_ctzll(m);
             const KzTileCov cb = kz_tile_cov_of(lc, b);
             const int32_t bx0 = kz_readlane_i(L.cx0, b) - X0, by0 = kz_readlane_i(L.cy0, b) - Y0;
             const int32_t bw = kz_readlane_i(cw, b), bc = kz_readlane_i(cand, b);
@@ -1737,7 +1874,7 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
                 s_frag[w++] = kz_pack_frag((uint32_t)((cy - Y0) * KZ_TS + (cx - X0)), lane, m);
             }
         }
-        bigm = kz_ballot(taken && L.live && !small);
+        bigm &= kz_ballot(taken);
         while (bigm) {
             const uint32_t b = (uint32_t)__builtin_ctzll(bigm);
             bigm &= bigm - 1;
@@ -1766,13 +1903,10 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
         if (!filter) kz_ahead_indices(nx, f);
 
         // --- resolve the queue 64 fragments at a time --------------------
-        uint32_t bfrag = 0, bpass = 0;
         if (narrow)
-            kz_resolve<true>(f, L, X0, Y0, total, lane, s_color, s_depth, s_claim, s_frag, bfrag, bpass);
+            kz_resolve<true>(f, L, X0, Y0, total, lane, s_color, s_depth, s_claim, s_frag, nfrag, npass);
         else
-            kz_resolve<false>(f, L, X0, Y0, total, lane, s_color, s_depth, s_claim, s_frag, bfrag, bpass);
-        nfrag += bfrag;
-        npass += bpass;
+            kz_resolve<false>(f, L, X0, Y0, total, lane, s_color, s_depth, s_claim, s_frag, nfrag, npass);
         k = next_k;
         ks = next_ks;
         __syncthreads();
@@ -1790,8 +1924,6 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
             }
         }
     }
-    nfrag = kz_wave_sum_u64(nfrag, lane);
-    npass = kz_wave_sum_u64(npass, lane);
     if (lane == 0) {
         unsigned long long *st = kz_stats_stripe(f);
         atomicAdd(&st[KZ_STAT_FRAGMENTS], nfrag);
