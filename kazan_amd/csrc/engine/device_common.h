@@ -111,7 +111,19 @@ struct KzFrame {
     uint32_t *clip_tris;      // [clip_cap] the triangles with pieces, in any order
     uint32_t *clip_rec;       // [clip_cap * KZ_REC_WORDS_FOR(varyings)]
     uint32_t clip_cap;
-    uint32_t pad2;
+    // Gather binning (batches of few triangles; else gather_seg is null):
+    // squares of 2^super_shift tiles a side and segments of KZ_GATHER_SEG
+    // triangles. The pair gather_seg[2 * (square * gather_segs + segment)] is
+    // the first place and the number of the segment's triangles that meet the
+    // square, in gather_list[square * gather_cap + ...] (their tiles in the
+    // square, KZ_GATHER_TILES, and the triangle, bit 31 for one with clip
+    // pieces); (KZ_GATHER_ALL, the segment's triangles) where they did not fit.
+    uint32_t super_shift;
+    uint32_t supers_x, supers_y;
+    uint32_t gather_segs, gather_cap;
+    uint32_t *gather_seg;
+    uint32_t *gather_list;    // (2 words each)
+    uint32_t *super_state;    // [squares * KZ_SUPER_WORDS], zeroed by kz_bin_count
     unsigned long long *stats;  // KZ_STAT_* counters
 
     // Load-balanced mode. A work item is a square sub-tile of a screen
@@ -266,6 +278,23 @@ enum {
 // KZ_PAIR_CHUNK triangles (KZ_PAIR_CHUNK / KZ_BIN_BLOCK blocks).
 #define KZ_BIN_BLOCK 256u
 #define KZ_PAIR_CHUNK 1024u
+// gather binning: triangles per segment, the most segments of a batch, log2
+// of a square's side in pixels
+#define KZ_GATHER_SEG 2048u
+#define KZ_GATHER_SEGS 64u  // (a lane each)
+#define KZ_SUPER_PX_SHIFT 7u
+#define KZ_GATHER_ALL 0xFFFFFFFFu
+#define KZ_GATHER_PIECES 0x80000000u  // in an entry's triangle: it has clip pieces
+// A box's tiles within a square of at most 16 x 16: bit c for column c, bit
+// 16 + r for row r; it meets tile (c, r) when it has both bits.
+#define KZ_GATHER_TILES(c0, c1, r0, r1) \
+    (((2u << (c1)) - (1u << (c0))) | (((2u << (r1)) - (1u << (r0))) << 16))
+enum {
+    KZ_SUPER_PAIRS = 0,   // (triangle, tile) pairs of the square
+    KZ_SUPER_COARSE = 1,  // its coarse entries reserved
+    KZ_SUPER_TAKEN = 2,   // list entries its tiles have reserved
+    KZ_SUPER_WORDS = 4
+};
 #define KZ_PAIR_PIECE 1024u  // pairs of a chunk that one workgroup writes
 enum {
     KZ_BIN_PAIRS = 0,  // pairs generated and sorted this batch (<= list capacity)

@@ -28,6 +28,13 @@ hipError_t grow(T *&p, uint64_t count) {
 // clip pieces kept per batch: their records take 64 B and 12 B per varying
 constexpr uint32_t kMaxClipPieces = 65536;
 
+// gather binning: the most triangles and squares of a batch
+constexpr uint32_t kGatherTris = 65536, kGatherSquares = 1024;
+static_assert(kGatherTris <= KZ_GATHER_SEG * KZ_GATHER_SEGS, "segments of a batch");
+
+// tiles whose state one thread of kz_bin_count clears, at least
+constexpr uint32_t kInitTiles = 4;
+
 // workgroups of kz_pair_scan that write the clip pieces' records (16 waves
 // each, one triangle a wave at a time)
 constexpr uint32_t kClipGrid = 64;
@@ -54,8 +61,9 @@ Engine::~Engine() {
     hipFree(sort_tmp_);
     hipFree(tri_rect_);
     hipFree(tri_rec_);
-    for (uint32_t *p : {tri_draw_, block_pairs_, chunk_offsets_, chunk_extra_, bin_ctrl_, tile_flag_, pair_keys_[0], pair_keys_[1],
-                        pair_vals_[0], pair_vals_[1], radix_table_, radix_totals_, clip_of_, clip_tris_, clip_rec_})
+    for (uint32_t *p : {tri_draw_, block_pairs_, chunk_offsets_, chunk_extra_, bin_ctrl_, tile_flag_, pair_keys_[0],
+                        pair_keys_[1], pair_vals_[0], pair_vals_[1], radix_table_, radix_totals_, clip_of_, clip_tris_,
+                        clip_rec_, gather_seg_, gather_list_, super_state_})
         hipFree(p);
     for (uint32_t *p : {tile_level_, split_slot_, split_info_, queue_, ctrl_, split_counts_, split_offsets_,
                         chunk_desc_, chunk_counts_, split_lists_, plan_table_, tile_acc_, tile_cycles_, tile_frags_, tri_z_})
@@ -91,7 +99,10 @@ bool Engine::init(int hip_device, std::string &err) {
     if (const char *e = std::getenv("KAZAN_AUTOTUNE")) autotune_ = std::strcmp(e, "0") != 0;
     if (const char *e = std::getenv("KAZAN_GRAPHS")) graphs_ = std::strcmp(e, "0") != 0;
     if (const char *e = std::getenv("KAZAN_SETUP_RECORDS")) setup_records_ = std::strcmp(e, "0") != 0;
-    if (const char *e = std::getenv("KAZAN_BINNING")) radix_ = std::strcmp(e, "sort") != 0;
+    if (const char *e = std::getenv("KAZAN_BINNING")) {
+        radix_ = std::strcmp(e, "sort") != 0;
+        gather_ = radix_ && std::strcmp(e, "radix") != 0;
+    }
     if (const char *e = std::getenv("KAZAN_GRID_DIVISOR")) {
         const int d = std::atoi(e);
         default_grid_div_ = d == 2 || d == 4 ? (uint32_t)d : 1u;
@@ -280,6 +291,49 @@ hipError_t Engine::ensure_scratch(uint32_t tiles, uint32_t tris) {
     return hipSuccess;
 }
 
+namespace {
+// The squares of gather binning over a w x h framebuffer
+uint32_t squares(uint32_t px) { return (px + (1u << KZ_SUPER_PX_SHIFT) - 1) >> KZ_SUPER_PX_SHIFT; }
+
+// entries of one square's coarse list: 32 per triangle over all squares (a
+// square that needs more tests its segments' triangles one by one)
+uint32_t gather_square_cap(uint32_t tris, uint32_t supers) {
+    return (uint32_t)std::min<uint64_t>(tris, std::max<uint64_t>(4096, 32ull * tris / supers));
+}
+}  // namespace
+
+// Gather binning is for batches whose squares' triangle lists are short: the
+// tiles of a square all read its list, so the work grows with the square of
+// the triangles' density, where radix binning's grows with the pairs. At
+// 65,536 triangles and 720p its two launches took 37 us against the radix
+// chain's 45 (a cluster), 34 against 46 (64 meshes) and 25 against 52 (a
+// grid); at 131,072 in 64 meshes, most of them in a few squares, 150 against
+// 62. (squares: their totals are summed by every workgroup.)
+bool Engine::use_gather(const KzFrame &f) const {
+    return gather_ && f.total_tris <= kGatherTris && (uint64_t)squares(f.width) * squares(f.height) <= kGatherSquares;
+}
+
+hipError_t Engine::ensure_gather(const KzFrame &f) {
+    const uint32_t supers = squares(f.width) * squares(f.height);
+    const uint32_t segs = supers * ((f.total_tris + KZ_GATHER_SEG - 1) / KZ_GATHER_SEG);
+    const uint64_t entries = (uint64_t)supers * gather_square_cap(f.total_tris, supers);
+    if (supers <= cap_supers_ && segs <= cap_gather_segs_ && entries <= cap_gather_) return hipSuccess;
+    KZ_TRY(hipStreamSynchronize(stream_));
+    if (supers > cap_supers_) {
+        KZ_TRY(regrow(super_state_, (uint64_t)supers * KZ_SUPER_WORDS));
+        cap_supers_ = supers;
+    }
+    if (segs > cap_gather_segs_) {
+        KZ_TRY(regrow(gather_seg_, 2ull * segs));
+        cap_gather_segs_ = segs;
+    }
+    if (entries > cap_gather_) {
+        KZ_TRY(regrow(gather_list_, 2 * entries));
+        cap_gather_ = entries;
+    }
+    return hipSuccess;
+}
+
 hipError_t Engine::alloc_lists(uint64_t capacity) {
     list_capacity_ = 0;
     KZ_TRY(regrow(tile_lists_, capacity));
@@ -328,6 +382,7 @@ hipError_t Engine::prepare_batch(const Op &op, uint32_t shift) {
             cap_rec_words_ = w;
         }
     }
+    if (use_gather(f)) KZ_TRY(ensure_gather(f));
     const uint64_t clip_words = (uint64_t)cap_clip_ * KZ_REC_WORDS_FOR(op.variants->fixed.num_varyings);
     if (clip_words > cap_clip_words_) {
         KZ_TRY(hipStreamSynchronize(stream_));
@@ -415,16 +470,40 @@ hipError_t Engine::run_batch(const Op &op, const BatchConfig &cfg) {
         }
     }
     void *args[] = {&f};
-    const uint32_t tri_blocks = (f.total_tris + 255) / 256;
+    // a thread per triangle, and enough of them to clear the tiles' state
+    const uint32_t tri_blocks = std::max((f.total_tris + 255) / 256,
+                                         std::min((ntiles + 256 * kInitTiles - 1) / (256 * kInitTiles), 4096u));
     uint32_t launches = 0;
 
     // binning: pixel boxes, then the per-tile lists in primitive order
-    KZ_TRY(mark(KS_CLEAR_COUNTS, false));
-    KZ_TRY(kz_launch_fill_tiles(stream_, tile_counts_, tile_offsets_, radix_ ? tile_flag_ : nullptr, ntiles));
-    if (acc) KZ_TRY(kz_launch_fill_u32(stream_, tile_acc_, (uint64_t)KZ_ACC * ntiles, 0u));
-    KZ_TRY(mark(KS_CLEAR_COUNTS, true));
-    launches += acc ? 2 : 1;
-    if (radix_) {
+    if (use_gather(f)) {
+        const uint32_t supers_x = squares(f.width), supers_y = squares(f.height);
+        f.super_shift = KZ_SUPER_PX_SHIFT - shift;
+        f.supers_x = supers_x;
+        f.supers_y = supers_y;
+        f.gather_segs = (f.total_tris + KZ_GATHER_SEG - 1) / KZ_GATHER_SEG;
+        f.gather_cap = gather_square_cap(f.total_tris, supers_x * supers_y);
+        f.gather_seg = gather_seg_;
+        f.gather_list = gather_list_;
+        f.super_state = super_state_;
+        f.tile_flag = nullptr;  // (no cut: a list that does not fit is a scan)
+        f.clip_cap = cap_clip_;
+        f.clip_of = clip_of_;
+        f.clip_tris = clip_tris_;
+        f.clip_rec = clip_rec_;
+        KZ_TRY(mark(KS_BIN_COUNT, false));
+        KZ_TRY(hipModuleLaunchKernel(kern->bin_count, tri_blocks, 1, 1, KZ_BIN_BLOCK, 1, 1, 0, stream_, args,
+                                     nullptr));
+        KZ_TRY(mark(KS_BIN_COUNT, true));
+        KZ_TRY(mark(KS_BIN_HIST, false));
+        KZ_TRY(hipModuleLaunchKernel(kern->gather_coarse, supers_x * supers_y * f.gather_segs + kClipGrid, 1, 1, 256, 1,
+                                     1, 0, stream_, args, nullptr));
+        KZ_TRY(mark(KS_BIN_HIST, true));
+        KZ_TRY(mark(KS_BIN_SCATTER, false));
+        KZ_TRY(kz_launch_gather_lists(stream_, f));
+        KZ_TRY(mark(KS_BIN_SCATTER, true));
+        launches += 3;
+    } else if (radix_) {
         // pairs in primitive order, a stable radix sort by tile whose last
         // pass writes the lists, counts and offsets
         f.block_pairs = block_pairs_;

@@ -37,6 +37,7 @@ struct PipelineKernels {
     hipModule_t module = nullptr;
     hipFunction_t bin_count = nullptr;
     hipFunction_t pair_scan = nullptr;          // pair offsets and the clip pieces' records
+    hipFunction_t gather_coarse = nullptr;      // gather binning: each square's triangles, and the records
     hipFunction_t raster = nullptr;             // one workgroup per tile
     hipFunction_t raster_persistent = nullptr;  // pops the work-item queue
     uint32_t persistent_blocks = 0;             // resident workgroups that fill the device
@@ -344,10 +345,16 @@ class Engine {
     uint32_t cap_clip_ = 0;
     uint64_t cap_clip_words_ = 0;
     uint32_t *tri_draw_ = nullptr;  // draw of each triangle, for batches of several draws
-    // Binning: radix (pairs in primitive order, stable radix sort by tile)
-    // or, with KAZAN_BINNING=sort, per-tile counts, an unordered scatter and
-    // a sort of every list.
-    bool radix_ = true;
+    // Binning: for batches of few triangles every tile gathers its list; else
+    // radix (pairs in primitive order, stable radix sort by tile). With
+    // KAZAN_BINNING=radix always radix, with =sort per-tile counts, an
+    // unordered scatter and a sort of every list.
+    bool radix_ = true, gather_ = true;
+    bool use_gather(const KzFrame &f) const;
+    hipError_t ensure_gather(const KzFrame &f);
+    uint32_t *gather_seg_ = nullptr, *gather_list_ = nullptr, *super_state_ = nullptr;
+    uint64_t cap_gather_ = 0;
+    uint32_t cap_gather_segs_ = 0, cap_supers_ = 0;
     uint32_t *block_pairs_ = nullptr, *chunk_offsets_ = nullptr, *chunk_extra_ = nullptr, *bin_ctrl_ = nullptr, *tile_flag_ = nullptr;
     uint32_t *pair_keys_[2] = {nullptr, nullptr}, *pair_vals_[2] = {nullptr, nullptr};
     // (balanced form) the list entries' 4 x 4 sub-tile masks

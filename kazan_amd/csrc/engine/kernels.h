@@ -6,9 +6,6 @@
 #include "device_common.h"
 
 hipError_t kz_launch_fill_u32(hipStream_t st, uint32_t *dst, uint64_t n, uint32_t value);
-// Per-tile list state before a batch's binning: counts 0, offsets all ones,
-// cut flags 0 (flags may be null).
-hipError_t kz_launch_fill_tiles(hipStream_t st, uint32_t *counts, uint32_t *offsets, uint32_t *flags, uint32_t n);
 hipError_t kz_launch_fill_rect_u32(hipStream_t st, uint32_t *dst, uint32_t width, int32_t x0, int32_t y0, uint32_t w,
                                    uint32_t h, uint32_t spp, uint32_t value);
 // Exclusive scan of counts[0, n) into offsets and cursor (or null); with
@@ -33,6 +30,9 @@ uint32_t kz_radix_digits_max();
 uint32_t kz_radix_passes(uint32_t ntiles);
 // The pairs in primitive order (1 launch).
 hipError_t kz_launch_bin_pairs(hipStream_t st, const KzFrame &f, const KzRadixScratch &s);
+// Gather binning, after the pipeline's kz_bin_count and kz_gather_coarse:
+// every tile's list, count and offset (and f.tile_acc's statistics).
+hipError_t kz_launch_gather_lists(hipStream_t st, const KzFrame &f);
 // The passes, the last into f.tile_lists with f.tile_counts (zeroed by the
 // caller); with f.tile_acc (zeroed by the caller), the pair statistics
 // (3 launches per pass).

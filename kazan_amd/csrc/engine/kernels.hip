@@ -165,16 +165,6 @@ __global__ __launch_bounds__(kScanThreads) void kz_scan(uint32_t *counts, uint32
     }
 }
 
-// A batch's per-tile list state before binning: counts 0, offsets all ones
-// (lowered by radix binning's last pass), cut flags 0 (flags may be null).
-__global__ void kz_fill_tiles(uint32_t *counts, uint32_t *offsets, uint32_t *flags, uint32_t n) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        counts[i] = 0u;
-        offsets[i] = 0xFFFFFFFFu;
-        if (flags) flags[i] = 0u;
-    }
-}
-
 // --- binning -----------------------------------------------------------
 
 // LDS open-addressing tables of 1 << LOG slots: keys[] (kNone = free) and
@@ -1050,6 +1040,322 @@ __global__ __launch_bounds__(kRadixThreads) void kz_radix_scatter(const uint32_t
             if (h[5]) atomicAdd(&c[KZ_ACC_SHARED], h[5]);
             atomicMax(&c[KZ_ACC_ZMIN], zinv);
             atomicMax(&c[KZ_ACC_ZMAX], zmax);
+        }
+    }
+}
+
+// --- gather binning -------------------------------------------------------
+//
+// For batches of few triangles, where the radix chain's launches (8 to 11,
+// about 4.5 us each in a replayed graph however small) are most of the frame:
+// every tile gathers its own list. kz_gather_coarse (the pipeline's) lists the
+// triangles of each 128 px square; here one wave per tile tests its square's
+// triangles in primitive order, keeps those that meet the tile and writes
+// them to the square's range of the list storage.
+
+constexpr uint32_t kGatherWaves = 8;  // tiles of a square per workgroup
+constexpr uint32_t kGatherThreads = kGatherWaves * 64;
+constexpr uint32_t kGatherPer = 8;    // candidates a thread fetches at a time
+constexpr uint32_t kGatherChunk = kGatherThreads * kGatherPer;
+static_assert(kGatherPer * kGatherWaves == 64, "a chunk's counts are one wave's scan");
+constexpr uint32_t kGatherHeld = kGatherChunk + 2048;  // candidates in LDS
+
+struct GatherAcc {
+    uint32_t area, hist[5], shared, zinv, zmax;
+};
+
+// The pair statistics of one list entry (box r) of tile (tx, ty).
+__device__ __forceinline__ void gather_stat(GatherAcc &a, uint64_t r, uint32_t z, uint32_t tx, uint32_t ty,
+                                            uint32_t sh) {
+    uint32_t x0, y0, x1, y1;
+    unpack_box(r, x0, y0, x1, y1);
+    const uint32_t X0 = tx << sh, Y0 = ty << sh, X1 = X0 + (1u << sh) - 1, Y1 = Y0 + (1u << sh) - 1;
+    const uint32_t area = (min(x1, X1) - max(x0, X0) + 1) * (min(y1, Y1) - max(y0, Y0) + 1);
+    a.area += area;
+    a.hist[0] += area <= 2 ? 1u : 0u;
+    a.hist[1] += area > 2 && area <= 8 ? 1u : 0u;
+    a.hist[2] += area > 8 && area <= 32 ? 1u : 0u;
+    a.hist[3] += area > 32 && area <= 128 ? 1u : 0u;
+    a.hist[4] += area > 128 ? 1u : 0u;
+    a.shared += box_tiles(r, sh) > 1 ? 1u : 0u;
+    a.zinv = max(a.zinv, 65535u - (z & 0xFFFFu));
+    a.zmax = max(a.zmax, z >> 16);
+}
+
+__device__ __forceinline__ bool box_in_tile(uint64_t r, uint32_t tx, uint32_t ty, uint32_t sh) {
+    uint32_t x0, y0, x1, y1;
+    unpack_box(r, x0, y0, x1, y1);
+    return r != KZ_RECT_EMPTY && (x0 >> sh) <= tx && (x1 >> sh) >= tx && (y0 >> sh) <= ty && (y1 >> sh) >= ty;
+}
+
+struct GatherLds {
+    uint32_t pfx[KZ_GATHER_SEGS + 1], at[KZ_GATHER_SEGS];
+    uint32_t cnt[2][64];  // of a chunk's kGatherPer rounds, wave by wave
+    uint32_t tiles[kGatherHeld], tri[kGatherHeld];
+};
+
+// A workgroup's tiles: a square, and in it a block of columns and rows
+struct GatherBlock {
+    uint32_t sq, sx, sy, ex, ey;  // the square's first and last tile
+    uint32_t cols, rows;          // the block's bits of KZ_GATHER_TILES
+};
+
+// Appends to the `have` candidates in LDS those of the square's candidates
+// [q0, q0 + kGatherChunk) that meet the block, in order; returns how many
+// there are now. The whole workgroup calls it, `par` alternating.
+__device__ __forceinline__ uint32_t gather_append(const KzFrame &f, GatherLds &l, const GatherBlock &k, uint32_t q0,
+                                                  uint32_t have, uint32_t par) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, sh = f.tile_shift;
+    const uint32_t total = l.pfx[KZ_GATHER_SEGS], start = l.pfx[lane];
+    uint2 v[kGatherPer];
+    uint64_t m[kGatherPer];
+#pragma unroll
+    for (uint32_t j = 0; j < kGatherPer; ++j) {
+        const uint32_t q = q0 + j * kGatherThreads + tid;
+        v[j] = make_uint2(0u, 0u);  // (no tile)
+        if (q - lane >= total) continue;  // (the whole wave)
+        // the last segment that starts at or before q: at or after the last
+        // that starts at or before the wave's first candidate
+        uint32_t lo = (uint32_t)__popcll(__ballot(start <= q - lane)) - 1u;
+        if (q >= total) continue;
+        while (l.pfx[lo + 1] <= q) ++lo;
+        const uint32_t i = q - l.pfx[lo];
+        if (l.at[lo] != KZ_GATHER_ALL) {
+            v[j] = ((const uint2 *)f.gather_list)[(size_t)k.sq * f.gather_cap + l.at[lo] + i];
+            continue;
+        }
+        const uint32_t g = lo * KZ_GATHER_SEG + i;
+        const uint64_t r = f.tri_rect[g];
+        uint32_t x0, y0, x1, y1;
+        unpack_box(r, x0, y0, x1, y1);
+        x0 >>= sh, y0 >>= sh, x1 >>= sh, y1 >>= sh;
+        if (r != KZ_RECT_EMPTY && x0 <= k.ex && x1 >= k.sx && y0 <= k.ey && y1 >= k.sy)
+            v[j] = make_uint2(KZ_GATHER_TILES(max(x0, k.sx) - k.sx, min(x1, k.ex) - k.sx, max(y0, k.sy) - k.sy,
+                                              min(y1, k.ey) - k.sy),
+                              r & KZ_RECT_PIECES ? g | KZ_GATHER_PIECES : g);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kGatherPer; ++j) {
+        m[j] = __ballot((v[j].x & k.cols) && (v[j].x & k.rows));
+        if (lane == 0) l.cnt[par][j * kGatherWaves + wave] = (uint32_t)__popcll(m[j]);
+    }
+    __syncthreads();
+    const uint32_t c = l.cnt[par][lane], x = kz_wave_incl_scan(c);
+#pragma unroll
+    for (uint32_t j = 0; j < kGatherPer; ++j) {
+        const uint32_t at = have + readlane(x - c, j * kGatherWaves + wave) + rank_in(m[j]);
+        if ((m[j] >> lane) & 1ull) {
+            l.tiles[at] = v[j].x;
+            l.tri[at] = v[j].y;
+        }
+    }
+    return have + readlane(x, 63);
+}
+
+// List entry e (box r, depth range z) of tile (tx, ty): its place `at` in the list storage
+// (if it is stored), sub-tile mask and statistics.
+__device__ __forceinline__ void gather_put(const KzFrame &f, uint32_t at, uint32_t e, uint64_t r, uint32_t z,
+                                           uint32_t tx, uint32_t ty, bool store, GatherAcc &acc) {
+    if (store) {
+        f.tile_lists[at] = e;
+        if (f.list_mask) {
+            uint32_t x0, y0, x1, y1;
+            unpack_box(r, x0, y0, x1, y1);
+            ((uint16_t *)f.list_mask)[at] = (uint16_t)box_sub_mask16(x0, y0, x1, y1, tx, ty, f.tile_shift);
+        }
+    }
+    if (f.tile_acc) gather_stat(acc, r, z, tx, ty, f.tile_shift);
+}
+
+// A wave's entries among the `have` candidates in LDS, for its tile (`want`:
+// the tile's bits): counted, or (PUT) put from place `at` on. Returns at plus
+// their number. 256 candidates a step, so that the boxes their masks and
+// statistics need are fetched together.
+template <bool PUT>
+__device__ __forceinline__ uint32_t gather_tile(const KzFrame &f, const GatherLds &l, uint32_t have, uint32_t tx,
+                                                uint32_t ty, uint32_t want, uint32_t at, bool store, GatherAcc &acc) {
+    const uint32_t lane = threadIdx.x & 63, sh = f.tile_shift;
+    const bool boxes = f.list_mask || f.tile_acc;
+    for (uint32_t i0 = 0; i0 < have; i0 += 256) {
+        bool hit[4];
+        uint64_t m[4];
+        uint32_t any = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t i = i0 + j * 64 + lane;
+            hit[j] = i < have && (l.tiles[i] & want) == want;
+            m[j] = __ballot(hit[j]);
+            any |= m[j] ? 1u : 0u;
+        }
+        if (!any) continue;
+        uint32_t g[4], pos[4], z[4];
+        uint64_t r[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            g[j] = hit[j] ? l.tri[i0 + j * 64 + lane] : 0u;
+            const bool pieces = hit[j] && (g[j] & KZ_GATHER_PIECES);
+            pos[j] = at + rank_in(m[j]);
+            if (__ballot(pieces)) {  // as many entries as pieces that meet the tile
+                uint32_t c = hit[j] ? 1u : 0u, of = 0, base = 0;
+                if (pieces) {
+                    of = f.clip_of[g[j] & ~KZ_GATHER_PIECES];
+                    base = f.total_tris + (of >> 4);
+                    c = 0;
+                    for (uint32_t p = 0; p < (of & 15u); ++p) c += box_in_tile(f.tri_rect[base + p], tx, ty, sh) ? 1u : 0u;
+                }
+                const uint32_t x = kz_wave_incl_scan(c);
+                pos[j] = at + x - c;
+                at += readlane(x, 63);
+                if (PUT && pieces) {  // (depth range [0, 1]: a piece's planes are not kept)
+                    for (uint32_t p = 0, q = pos[j]; p < (of & 15u); ++p) {
+                        const uint64_t rp = f.tri_rect[base + p];
+                        if (box_in_tile(rp, tx, ty, sh)) gather_put(f, q++, base + p, rp, 0xFFFF0000u, tx, ty, store, acc);
+                    }
+                    hit[j] = false;
+                }
+            } else {
+                at += (uint32_t)__popcll(m[j]);
+            }
+        }
+        if (!PUT) continue;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            r[j] = boxes && hit[j] ? f.tri_rect[g[j]] : 0ull;
+            z[j] = f.tile_acc && hit[j] ? f.tri_z[g[j]] : 0u;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j)
+            if (hit[j]) gather_put(f, pos[j], g[j], r[j], z[j], tx, ty, store, acc);
+    }
+    return at;
+}
+
+// The square's candidates through LDS, kGatherHeld at a time, each wave
+// counting or putting its tile's entries from `at` on; returns at plus their
+// number. have: the candidates LDS holds at the end; one: all of them were
+// held at once (a second walk then needs no fetch).
+template <bool PUT>
+__device__ __forceinline__ uint32_t gather_walk(const KzFrame &f, GatherLds &l, const GatherBlock &k, uint32_t tx,
+                                                uint32_t ty, uint32_t want, uint32_t at, bool store, uint32_t &have,
+                                                bool &one, GatherAcc &acc) {
+    const uint32_t total = l.pfx[KZ_GATHER_SEGS];
+    uint32_t q = 0, par = 0;
+    if (PUT && one) return want ? gather_tile<PUT>(f, l, have, tx, ty, want, at, store, acc) : at;
+    do {
+        __syncthreads();  // the candidates before are done with
+        have = 0;
+        one = q == 0;
+        for (; q < total && have + kGatherChunk <= kGatherHeld; q += kGatherChunk, par ^= 1u)
+            have = gather_append(f, l, k, q, have, par);
+        one = one && q >= total;
+        __syncthreads();
+        if (want) at = gather_tile<PUT>(f, l, have, tx, ty, want, at, store, acc);
+    } while (q < total);
+    return at;
+}
+
+// Bound by the latency of a few dependent steps (segment table, candidates,
+// the square's counter, boxes), which workgroups of many squares overlap.
+// A workgroup has 8 tiles of a square (4 x 2 where there are as many), one a
+// wave: its candidates are first cut to those that meet its block, by all
+// waves together, and each wave then tests its tile against these, two
+// instructions and an LDS read per 64. 40,400 triangles around a camera at
+// 1279x719 take 19 us (one workgroup per tile testing pixel boxes: 48), a
+// grid of 11,834 at 1023x575 11 us (19).
+// The squares' ranges of the list storage follow from their pair totals; a
+// tile takes its place in its square's range with one atomic (one counter for
+// all tiles would take every workgroup's). A list past the storage's end is
+// left out and its tile drawn by a scan of every triangle, as with sort
+// binning.
+__global__ __launch_bounds__(kGatherThreads) void kz_gather_lists(KzFrame f, uint32_t groups) {
+    __shared__ GatherLds l;
+    __shared__ unsigned long long s_before[kGatherWaves], s_all[kGatherWaves];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // the block: gw columns and gh rows of the square's side (a power of two)
+    const uint32_t side = 1u << f.super_shift, gw = min(4u, side), gh = min(kGatherWaves / gw, side);
+    const uint32_t sq = blockIdx.x / groups, grp = blockIdx.x % groups;
+    const uint32_t c0 = (grp % (side / gw)) * gw, r0 = (grp / (side / gw)) * gh;
+    const uint32_t col = c0 + wave % gw, row = r0 + wave / gw;
+    GatherBlock k;
+    k.sq = sq;
+    k.sx = (sq % f.supers_x) << f.super_shift;
+    k.sy = (sq / f.supers_x) << f.super_shift;
+    k.ex = min(k.sx + side, f.tiles_x) - 1;
+    k.ey = min(k.sy + side, f.tiles_y) - 1;
+    k.cols = ((1u << gw) - 1u) << c0;
+    k.rows = (((1u << gh) - 1u) << r0) << 16;
+    const uint32_t tx = k.sx + col, ty = k.sy + row;
+    const bool tile = wave < gw * gh && tx <= k.ex && ty <= k.ey;
+    // pairs of the squares before this one and of all, in halves whose sums
+    // over 1,024 squares fit 32 bits
+    uint32_t half[4] = {0u, 0u, 0u, 0u};
+    for (uint32_t i = tid; i < f.supers_x * f.supers_y; i += kGatherThreads) {
+        const uint32_t p = f.super_state[i * KZ_SUPER_WORDS + KZ_SUPER_PAIRS];
+        half[0] += i < sq ? p & 0xFFFFu : 0u;
+        half[1] += i < sq ? p >> 16 : 0u;
+        half[2] += p & 0xFFFFu;
+        half[3] += p >> 16;
+    }
+    if (wave == 0) {
+        uint2 s = make_uint2(0u, 0u);
+        if (lane < f.gather_segs) s = ((const uint2 *)f.gather_seg)[sq * f.gather_segs + lane];
+        const uint32_t x = kz_wave_incl_scan(s.y);
+        l.pfx[lane] = x - s.y;
+        l.at[lane] = s.x;
+        if (lane == 63) l.pfx[KZ_GATHER_SEGS] = x;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) half[i] = readlane(kz_wave_incl_scan(half[i]), 63);
+    if (lane == 0) {
+        s_before[wave] = half[0] + ((unsigned long long)half[1] << 16);
+        s_all[wave] = half[2] + ((unsigned long long)half[3] << 16);
+    }
+    __syncthreads();
+    unsigned long long before = 0, all = 0;
+    for (uint32_t w = 0; w < kGatherWaves; ++w) {
+        before += s_before[w];
+        all += s_all[w];
+    }
+    const unsigned long long cap = f.list_capacity;
+    if (blockIdx.x == 0 && tid == 0) {
+        f.bin_ctrl[KZ_BIN_PAIRS] = (uint32_t)min(all, 0xFFFFFFFFull);
+        f.bin_ctrl[KZ_BIN_CUT] = 0;  // a scan of the triangles starts at the first
+        f.bin_ctrl[KZ_BIN_OVER] = all > cap ? 1u : 0u;
+        f.bin_ctrl[KZ_BIN_PIECES] = 0;  // for the next batch
+        f.bin_ctrl[KZ_BIN_CLIPPED] = 0;
+        atomicAdd(&f.stats[KZ_STAT_LIST_ENTRIES], all);
+        if (all > cap) atomicAdd(&f.stats[KZ_STAT_LIST_OVERFLOW], 1ull);
+    }
+    GatherAcc acc = {};
+    const uint32_t want = tile ? (1u << col) | (0x10000u << row) : 0u;
+    uint32_t have = 0;
+    bool one = false;
+    const uint32_t n = gather_walk<false>(f, l, k, tx, ty, want, 0u, false, have, one, acc);
+    const uint32_t t = ty * f.tiles_x + tx;
+    uint32_t taken = 0;
+    if (lane == 0 && n) taken = atomicAdd(&f.super_state[sq * KZ_SUPER_WORDS + KZ_SUPER_TAKEN], n);
+    before += readlane(taken, 0);
+    const bool fits = before + n <= cap;
+    const uint32_t off = (uint32_t)(fits ? before : cap);
+    if (tile && lane == 0) {
+        f.tile_counts[t] = n;
+        f.tile_offsets[t] = n ? off : 0u;
+    }
+    gather_walk<true>(f, l, k, tx, ty, want, off, fits, have, one, acc);
+    if (tile && f.tile_acc) {
+        uint32_t *a = f.tile_acc + (size_t)t * KZ_ACC;
+        const uint32_t sums[7] = {acc.area, acc.hist[0], acc.hist[1], acc.hist[2], acc.hist[3], acc.hist[4], acc.shared};
+        const int at[7] = {KZ_ACC_AREA,     KZ_ACC_HIST,     KZ_ACC_HIST + 1, KZ_ACC_HIST + 2,
+                           KZ_ACC_HIST + 3, KZ_ACC_HIST + 4, KZ_ACC_SHARED};
+#pragma unroll
+        for (int i = 0; i < 7; ++i) {
+            const uint32_t v = readlane(kz_wave_incl_scan(sums[i]), 63);
+            if (lane == 0) a[at[i]] = v;
+        }
+        const uint32_t zi = wave_max_u32(acc.zinv), zm = wave_max_u32(acc.zmax);
+        if (lane == 0) {
+            a[KZ_ACC_ZMIN] = zi;
+            a[KZ_ACC_ZMAX] = zm;
         }
     }
 }
@@ -2101,12 +2407,6 @@ hipError_t kz_launch_fill_u32(hipStream_t st, uint32_t *dst, uint64_t n, uint32_
     return hipGetLastError();
 }
 
-hipError_t kz_launch_fill_tiles(hipStream_t st, uint32_t *counts, uint32_t *offsets, uint32_t *flags, uint32_t n) {
-    if (n == 0) return hipSuccess;
-    kz_fill_tiles<<<grid_for(n, 256), 256, 0, st>>>(counts, offsets, flags, n);
-    return hipGetLastError();
-}
-
 hipError_t kz_launch_fill_rect_u32(hipStream_t st, uint32_t *dst, uint32_t width, int32_t x0, int32_t y0, uint32_t w,
                                    uint32_t h, uint32_t spp, uint32_t value) {
     const uint64_t n = (uint64_t)w * h * spp;
@@ -2144,6 +2444,14 @@ hipError_t kz_launch_bin_pairs(hipStream_t st, const KzFrame &f, const KzRadixSc
                       f.tri_rect, f.clip_of, f.total_tris};
     kz_pair_write<<<nchunks + extra, kPairThreads, 0, st>>>(f.tri_rect, f.total_tris, nchunks, out, f.chunk_offsets,
                                                             f.chunk_extra, s.ctrl, s.tile_flag);
+    return hipGetLastError();
+}
+
+hipError_t kz_launch_gather_lists(hipStream_t st, const KzFrame &f) {
+    // (the blocks of a square, as the kernel cuts it)
+    const uint32_t side = 1u << f.super_shift, gw = std::min(4u, side), gh = std::min(kGatherWaves / gw, side);
+    const uint32_t groups = (side / gw) * (side / gh);
+    kz_gather_lists<<<f.supers_x * f.supers_y * groups, kGatherThreads, 0, st>>>(f, groups);
     return hipGetLastError();
 }
 

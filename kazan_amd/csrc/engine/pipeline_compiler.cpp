@@ -346,6 +346,7 @@ bool load_pipeline_kernels(const std::vector<char> &code, PipelineKernels &out, 
     }
     if ((e = hipModuleGetFunction(&out.bin_count, out.module, "kz_bin_count")) != hipSuccess ||
         (e = hipModuleGetFunction(&out.pair_scan, out.module, "kz_pair_scan")) != hipSuccess ||
+        (e = hipModuleGetFunction(&out.gather_coarse, out.module, "kz_gather_coarse")) != hipSuccess ||
         (e = hipModuleGetFunction(&out.raster, out.module, "kz_raster")) != hipSuccess ||
         (e = hipModuleGetFunction(&out.raster_persistent, out.module, "kz_raster_persistent")) != hipSuccess) {
         err = std::string("hipModuleGetFunction: ") + hipGetErrorString(e);

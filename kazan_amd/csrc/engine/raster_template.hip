@@ -699,6 +699,22 @@ __device__ __forceinline__ bool kz_load_rec(const KzFrame &f, const uint32_t *re
 extern "C" __global__ __launch_bounds__(KZ_BIN_BLOCK) void kz_bin_count(KzFrame f) {
     const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t lane = kz_lane();
+    // the state that later passes add to (a launch of its own for it took
+    // 4 us of a frame)
+    {
+        const uint32_t n = gridDim.x * blockDim.x, ntiles = f.tiles_x * f.tiles_y;
+        if (f.gather_seg) {
+            for (uint32_t i = g; i < f.supers_x * f.supers_y * KZ_SUPER_WORDS; i += n) f.super_state[i] = 0;
+        } else {
+            for (uint32_t i = g; i < ntiles; i += n) {
+                f.tile_counts[i] = 0;
+                f.tile_offsets[i] = ~0u;
+                if (f.tile_flag) f.tile_flag[i] = 0;
+            }
+            if (f.tile_acc)
+                for (uint32_t i = g; i < ntiles * KZ_ACC; i += n) f.tile_acc[i] = 0;
+        }
+    }
     uint32_t n_setup = 0, n_clip = 0, n_pairs = 0;
     float p[3][4], vary[3][KZ_NVA];
     KzTri t;
@@ -848,7 +864,7 @@ extern "C" __global__ __launch_bounds__(KZ_BIN_BLOCK) void kz_bin_count(KzFrame 
         if (ms) atomicAdd(&sts[KZ_STAT_TRIANGLES_SETUP], (unsigned long long)__popcll(ms));
         if (mc) atomicAdd(&sts[KZ_STAT_TRIANGLES_CLIPPED], (unsigned long long)__popcll(mc));
     }
-    if (f.block_pairs) {  // the block's pair total, for the pair offsets of radix binning
+    if (f.block_pairs && blockIdx.x * KZ_BIN_BLOCK < f.total_tris) {  // the block's pair total, for the pair offsets of radix binning
         __shared__ uint32_t s_pairs[KZ_BIN_BLOCK / 64];
         for (uint32_t d = 32; d > 0; d >>= 1) n_pairs += (uint32_t)__shfl_xor((int)n_pairs, (int)d, 64);
         if (lane == 0) s_pairs[threadIdx.x >> 6] = n_pairs;
@@ -1460,9 +1476,9 @@ __device__ __forceinline__ void kz_clip_records(const KzFrame &f, uint32_t first
 // chunks before c (ctrl[KZ_BIN_EXTRA] in all), which kz_pair_write gives to
 // workgroups of their own.
 // Bound by the latency of its loads: a step takes 4,096 chunks, each thread
-// 4 consecutive ones with all their loads in flight at once (8.4 M
-// triangles: two steps; 256 threads of one chunk each took 8 steps of 4,096
-// triangles a chunk, MEAS_PSCAN).
+// 4 consecutive ones with all their loads in flight at once (8.4 M triangles
+// are two steps and 10.1 us, where 256 threads of one chunk of 4,096 triangles
+// each took 22.4).
 extern "C" __global__ __launch_bounds__(KZ_PAIR_SCAN_THREADS) void kz_pair_scan(KzFrame f) {
     if (blockIdx.x > 0) {
         kz_clip_records(f, (blockIdx.x - 1) * (KZ_PAIR_SCAN_THREADS / 64) + (threadIdx.x >> 6),
@@ -1560,6 +1576,93 @@ extern "C" __global__ __launch_bounds__(KZ_PAIR_SCAN_THREADS) void kz_pair_scan(
         atomicAdd(&f.stats[KZ_STAT_LIST_ENTRIES], carry);
         if (over) atomicAdd(&f.stats[KZ_STAT_LIST_OVERFLOW], 1ull);
     }
+}
+
+// Gather binning, pass 2 (with the clip pieces' records): the triangles of
+// segment `seg` whose boxes meet square `sq`, in primitive order, and the
+// square's (triangle, tile) pairs. kz_gather_lists then tests each tile
+// against its square's triangles only.
+#define KZ_GATHER_THREADS 256
+#define KZ_GATHER_PER (KZ_GATHER_SEG / KZ_GATHER_THREADS)
+
+__device__ __forceinline__ uint32_t kz_tiles_in(uint64_t r, uint32_t tx0, uint32_t ty0, uint32_t tx1, uint32_t ty1) {
+    const uint32_t x0 = (uint32_t)(r & (0xFFFF & ~KZ_RECT_PIECES)) >> KZ_TILE_SHIFT,
+                   y0 = (uint32_t)((r >> 16) & 0xFFFF) >> KZ_TILE_SHIFT;
+    const uint32_t x1 = (uint32_t)((r >> 32) & 0xFFFF) >> KZ_TILE_SHIFT, y1 = (uint32_t)(r >> 48) >> KZ_TILE_SHIFT;
+    if (r == KZ_RECT_EMPTY || x1 < tx0 || x0 > tx1 || y1 < ty0 || y0 > ty1) return 0;
+    return (min(x1, tx1) - max(x0, tx0) + 1) * (min(y1, ty1) - max(y0, ty0) + 1);
+}
+
+extern "C" __global__ __launch_bounds__(KZ_GATHER_THREADS) void kz_gather_coarse(KzFrame f) {
+    __shared__ uint32_t s_cnt[KZ_GATHER_PER][KZ_GATHER_THREADS / 64], s_pairs[KZ_GATHER_THREADS / 64];
+    __shared__ uint32_t s_at;
+    const uint32_t tid = threadIdx.x, lane = kz_lane(), wave = tid >> 6;
+    const uint32_t work = f.supers_x * f.supers_y * f.gather_segs;
+    if (blockIdx.x >= work) {
+        kz_clip_records(f, (blockIdx.x - work) * (KZ_GATHER_THREADS / 64) + wave,
+                        (gridDim.x - work) * (KZ_GATHER_THREADS / 64));
+        return;
+    }
+    const uint32_t sq = blockIdx.x / f.gather_segs, seg = blockIdx.x % f.gather_segs;
+    const uint32_t tx0 = (sq % f.supers_x) << f.super_shift, ty0 = (sq / f.supers_x) << f.super_shift;
+    const uint32_t tx1 = min(tx0 + (1u << f.super_shift), f.tiles_x) - 1;
+    const uint32_t ty1 = min(ty0 + (1u << f.super_shift), f.tiles_y) - 1;
+    const uint32_t g0 = seg * KZ_GATHER_SEG, n = min(KZ_GATHER_SEG, f.total_tris - g0);
+    uint64_t r[KZ_GATHER_PER], m[KZ_GATHER_PER];
+#pragma unroll
+    for (int j = 0; j < (int)KZ_GATHER_PER; ++j) {
+        const uint32_t i = j * KZ_GATHER_THREADS + tid;
+        r[j] = i < n ? f.tri_rect[g0 + i] : KZ_RECT_EMPTY;
+    }
+    uint32_t pairs = 0;
+#pragma unroll
+    for (int j = 0; j < (int)KZ_GATHER_PER; ++j) {
+        uint32_t c = kz_tiles_in(r[j], tx0, ty0, tx1, ty1);
+        m[j] = kz_ballot(c != 0);
+        if (c && (r[j] & KZ_RECT_PIECES)) {
+            const uint32_t of = f.clip_of[g0 + j * KZ_GATHER_THREADS + tid], base = f.total_tris + (of >> 4);
+            c = 0;
+            for (uint32_t i = 0; i < (of & 15u); ++i) c += kz_tiles_in(f.tri_rect[base + i], tx0, ty0, tx1, ty1);
+        }
+        pairs += c;
+        if (lane == 0) s_cnt[j][wave] = (uint32_t)__popcll(m[j]);
+    }
+    pairs = kz_wave_sum(pairs);
+    if (lane == 0) s_pairs[wave] = pairs;
+    __syncthreads();
+    uint32_t total = 0, at[KZ_GATHER_PER];
+#pragma unroll
+    for (int j = 0; j < (int)KZ_GATHER_PER; ++j)
+#pragma unroll
+        for (uint32_t w = 0; w < KZ_GATHER_THREADS / 64; ++w) {
+            if (w == wave) at[j] = total;
+            total += s_cnt[j][w];
+        }
+    if (tid == 0) {
+        uint32_t *st = f.super_state + sq * KZ_SUPER_WORDS;
+        const uint32_t all = s_pairs[0] + s_pairs[1] + s_pairs[2] + s_pairs[3];
+        if (all) atomicAdd(&st[KZ_SUPER_PAIRS], all);
+        const uint32_t base = total ? atomicAdd(&st[KZ_SUPER_COARSE], total) : 0u;
+        const bool fits = base <= f.gather_cap && total <= f.gather_cap - base;
+        ((uint2 *)f.gather_seg)[blockIdx.x] = make_uint2(fits ? base : KZ_GATHER_ALL, fits ? total : n);
+        s_at = fits ? base : KZ_GATHER_ALL;
+    }
+    __syncthreads();
+    if (s_at == KZ_GATHER_ALL) return;
+    uint2 *list = (uint2 *)f.gather_list + (size_t)sq * f.gather_cap + s_at;
+#pragma unroll
+    for (int j = 0; j < (int)KZ_GATHER_PER; ++j)
+        if ((m[j] >> lane) & 1ull) {
+            const uint32_t x0 = (uint32_t)(r[j] & (0xFFFF & ~KZ_RECT_PIECES)) >> KZ_TILE_SHIFT,
+                           y0 = (uint32_t)((r[j] >> 16) & 0xFFFF) >> KZ_TILE_SHIFT;
+            const uint32_t x1 = (uint32_t)((r[j] >> 32) & 0xFFFF) >> KZ_TILE_SHIFT,
+                           y1 = (uint32_t)(r[j] >> 48) >> KZ_TILE_SHIFT;
+            const uint32_t g = g0 + j * KZ_GATHER_THREADS + tid;
+            list[at[j] + kz_rank(m[j])] =
+                make_uint2(KZ_GATHER_TILES(max(x0, tx0) - tx0, min(x1, tx1) - tx0, max(y0, ty0) - ty0,
+                                           min(y1, ty1) - ty0),
+                           r[j] & KZ_RECT_PIECES ? g | KZ_GATHER_PIECES : g);
+        }
 }
 
 // Rasterises n triangles into the square of side 1 << RS at (X0, Y0) (a
