@@ -678,10 +678,16 @@ int final_choice(const BatchTuning &t) {
 // splits smaller tiles on a larger grid may pay); then the three fastest
 // twice more each. The finalist with the lowest median of its three runs
 // is kept.
-hipError_t Engine::pick_config(Op &op, BatchConfig &cfg, bool &timed) {
+hipError_t Engine::pick_config(Op &op, BatchConfig &cfg, bool &timed, bool tune) {
     cfg = default_config(op);
     timed = false;
     if (!autotune()) return hipSuccess;
+    if (!tune) {
+        // (without the model: its statistics and predictions cost more than
+        // its plan saves unless a trial has shown otherwise)
+        cfg.model = false;
+        return hipSuccess;
+    }
     const bool model = cost_model_d_ != nullptr;
     if (!op.tuning) {
         op.tuning = std::make_shared<BatchTuning>();
@@ -776,8 +782,11 @@ hipError_t Engine::execute(std::vector<Op> &ops, GraphCache *cache) {
             if (autotune() && !(op.tuning && op.tuning->done)) graphable = false;
         }
     if (!graphable || !draws || (cache->eager_runs == 0 && !cache->exec)) {
+        // a command buffer recorded for every frame would run its first trial
+        // in all of them, and never learn from it
+        const bool tune = !cache || !cache->recorded_per_frame || cache->eager_runs > 0;
         if (cache) ++cache->eager_runs;
-        return execute_eager(ops);
+        return execute_eager(ops, tune);
     }
     // every allocation before the capture
     for (Op &op : ops)
@@ -822,12 +831,12 @@ hipError_t Engine::execute(std::vector<Op> &ops, GraphCache *cache) {
     return hipSuccess;
 }
 
-hipError_t Engine::execute_eager(std::vector<Op> &ops) {
+hipError_t Engine::execute_eager(std::vector<Op> &ops, bool tune) {
     for (Op &op : ops)
         if (op.kind == Op::Batch) {
             BatchConfig cfg;
             bool timed;
-            KZ_TRY(pick_config(op, cfg, timed));
+            KZ_TRY(pick_config(op, cfg, timed, tune));
             if (timed) {
                 // a trial times the batch, not the loading of a tile size's
                 // kernels or the growth of its scratch (host work and syncs)
@@ -890,6 +899,7 @@ hipError_t Engine::launch_ops_one(const Op &op) {
 }
 
 hipError_t Engine::end_submit(hipEvent_t fence_event) {
+    ++submissions_;
     KZ_TRY(hipEventRecord(ev_end_, stream_));
     if (fence_event) KZ_TRY(hipEventRecord(fence_event, stream_));
     return hipSuccess;

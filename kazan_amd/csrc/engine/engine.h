@@ -220,6 +220,9 @@ struct GraphCache {
     uint64_t generation = 0;
     uint32_t batches = 0, launches = 0;
     uint32_t eager_runs = 0;  // a command buffer is captured from its second submission on
+    // the command buffer was recorded anew after a single submission: its
+    // first submission takes the untuned configuration
+    bool recorded_per_frame = false;
 };
 
 class Engine {
@@ -236,6 +239,7 @@ class Engine {
     hipError_t begin_submit();
     hipError_t execute(std::vector<Op> &ops, GraphCache *cache = nullptr);
     hipError_t end_submit(hipEvent_t fence_event);
+    uint64_t submissions() const { return submissions_; }
     uint32_t graph_launches() const { return graph_launches_; }
     uint32_t graph_captures() const { return graph_captures_; }
     // the configuration the most recently finished tuning chose (shift 0 =
@@ -289,11 +293,11 @@ class Engine {
     hipError_t ensure_scratch(uint32_t tiles, uint32_t tris);
     // the configuration a batch runs with this submission (tuning trial or
     // the tuned choice), and its scratch allocated for it
-    hipError_t pick_config(Op &op, BatchConfig &cfg, bool &timed);
+    hipError_t pick_config(Op &op, BatchConfig &cfg, bool &timed, bool tune = true);
     BatchConfig default_config(const Op &op) const;
     hipError_t prepare_batch(const Op &op, uint32_t shift);
     hipError_t run_batch(const Op &op, const BatchConfig &cfg);
-    hipError_t execute_eager(std::vector<Op> &ops);
+    hipError_t execute_eager(std::vector<Op> &ops, bool tune = true);
     hipError_t launch_ops(std::vector<Op> &ops);  // tuned configurations, no tuning events
     hipError_t launch_ops_one(const Op &op);      // a non-batch op
     hipError_t mark(int slot, bool end);
@@ -308,6 +312,7 @@ class Engine {
     // (KAZAN_GRID_DIVISOR, KAZAN_SPLIT_LEVEL)
     uint32_t default_grid_div_ = 1, default_max_level_ = 2;
     uint64_t generation_ = 1;  // bumped whenever captured graphs go stale
+    uint64_t submissions_ = 0;
     uint32_t graph_launches_ = 0, graph_captures_ = 0;
     BatchConfig last_tuned_{0, 0, false, false, 0, 0};
     uint64_t list_limit_ = 0;

@@ -1027,25 +1027,64 @@ VKAPI_ATTR VkResult VKAPI_CALL vkCreateCommandPool(VkDevice, const VkCommandPool
 }
 
 static void reset_cb(CommandBuffer *cb) {
-    if (!cb->device_allocs.empty() || cb->graph.exec) {
+    if (cb->submissions) {  // (a graph or draw records that kernels may be reading)
         set_device(cb->device);
-        hipStreamSynchronize(cb->device->engine->stream());
-        for (void *p : cb->device_allocs) hipFree(p);
+        hipEventSynchronize(cb->done);
+        // recorded anew after one submission: likely again
+        cb->graph.recorded_per_frame = cb->submissions == 1;
     }
     cb->graph.reset();
     cb->graph.eager_runs = 0;
-    cb->device_allocs.clear();
+    cb->records_used = 0;
+    cb->records_pending = false;
+    cb->submissions = 0;
     cb->ops.clear();
     cb->st = RecordState();
     cb->recording = false;
+}
+
+static void destroy_cb(CommandBuffer *cb) {
+    reset_cb(cb);
+    if (cb->done || !cb->records.empty()) set_device(cb->device);
+    for (DrawRecords &r : cb->records) {
+        hipFree(r.dev);
+        hipHostFree(r.host);
+    }
+    if (cb->done) hipEventDestroy(cb->done);
+    delete cb;
+}
+
+// The next draw records of cb's recording, at least `bytes` long.
+static DrawRecords *next_records(CommandBuffer *cb, size_t bytes) {
+    if (cb->records_used == cb->records.size()) cb->records.emplace_back();
+    DrawRecords &r = cb->records[cb->records_used];
+    if (r.cap < bytes) {  // (not in use: the recording before has finished)
+        hipFree(r.dev);
+        hipHostFree(r.host);
+        r = DrawRecords();
+        const size_t cap = bytes + bytes / 2;
+        if (hipMalloc((void **)&r.dev, cap) != hipSuccess) return nullptr;
+        if (hipHostMalloc((void **)&r.host, cap, hipHostMallocDefault) != hipSuccess) {
+            hipFree(r.dev);
+            r = DrawRecords();
+            return nullptr;
+        }
+        r.cap = cap;
+    }
+    if (!cb->done && hipEventCreateWithFlags(&cb->done, hipEventDisableTiming) != hipSuccess) {
+        cb->done = nullptr;
+        return nullptr;
+    }
+    r.bytes = bytes;
+    ++cb->records_used;
+    return &r;
 }
 
 VKAPI_ATTR void VKAPI_CALL vkDestroyCommandPool(VkDevice, VkCommandPool pool, const VkAllocationCallbacks *) {
     CommandPool *p = from<CommandPool>(pool);
     if (!p) return;
     for (CommandBuffer *cb : p->buffers) {
-        reset_cb(cb);
-        delete cb;
+        destroy_cb(cb);
     }
     delete p;
 }
@@ -1076,9 +1115,8 @@ VKAPI_ATTR void VKAPI_CALL vkFreeCommandBuffers(VkDevice, VkCommandPool pool, ui
     for (uint32_t i = 0; i < n; ++i) {
         CommandBuffer *cb = from<CommandBuffer>(pCbs[i]);
         if (!cb) continue;
-        reset_cb(cb);
         p->buffers.erase(std::remove(p->buffers.begin(), p->buffers.end(), cb), p->buffers.end());
-        delete cb;
+        destroy_cb(cb);
     }
 }
 
@@ -1093,7 +1131,8 @@ VKAPI_ATTR VkResult VKAPI_CALL vkEndCommandBuffer(VkCommandBuffer commandBuffer)
     CommandBuffer *cb = from<CommandBuffer>(commandBuffer);
     if (!cb->recording) return VK_ERROR_INITIALIZATION_FAILED;
     set_device(cb->device);
-    // upload each batch's draw records once; every submission reuses them
+    // each batch's draw records, copied to the device by the recording's first
+    // submission; every submission reuses them
     for (Op &op : cb->ops) {
         if (op.kind != Op::Batch || op.draws.empty()) continue;
         // the records, then their first triangles as a dense array, then
@@ -1101,9 +1140,10 @@ VKAPI_ATTR VkResult VKAPI_CALL vkEndCommandBuffer(VkCommandBuffer commandBuffer)
         // block (and the last draw), which narrows the device's search
         const size_t n = op.draws.size(), rec_bytes = n * sizeof(KzDraw);
         const size_t nblk = ((size_t)op.frame.total_tris + KZ_BIN_BLOCK - 1) / KZ_BIN_BLOCK + 1;
-        std::vector<char> host(rec_bytes + (n + nblk) * sizeof(uint32_t));
-        std::memcpy(host.data(), op.draws.data(), rec_bytes);
-        uint32_t *begin = (uint32_t *)(host.data() + rec_bytes);
+        DrawRecords *r = next_records(cb, rec_bytes + (n + nblk) * sizeof(uint32_t));
+        if (!r) return VK_ERROR_OUT_OF_DEVICE_MEMORY;
+        std::memcpy(r->host, op.draws.data(), rec_bytes);
+        uint32_t *begin = (uint32_t *)(r->host + rec_bytes);
         for (size_t i = 0; i < n; ++i) begin[i] = op.draws[i].tri_begin;
         uint32_t *block_draw = begin + n;
         for (size_t b = 0, d = 0; b < nblk; ++b) {
@@ -1111,12 +1151,9 @@ VKAPI_ATTR VkResult VKAPI_CALL vkEndCommandBuffer(VkCommandBuffer commandBuffer)
             while (d + 1 < n && op.draws[d + 1].tri_begin <= g) ++d;
             block_draw[b] = (uint32_t)d;
         }
-        void *p = nullptr;
-        if (hipMalloc(&p, host.size()) != hipSuccess) return VK_ERROR_OUT_OF_DEVICE_MEMORY;
-        cb->device_allocs.push_back(p);
-        if (hipMemcpy(p, host.data(), host.size(), hipMemcpyHostToDevice) != hipSuccess) return VK_ERROR_DEVICE_LOST;
-        op.d_draws = (KzDraw *)p;
-        op.d_draw_begin = (uint32_t *)((char *)p + rec_bytes);
+        cb->records_pending = true;
+        op.d_draws = (KzDraw *)r->dev;
+        op.d_draw_begin = (uint32_t *)(r->dev + rec_bytes);
         op.d_block_draw = op.d_draw_begin + n;
         op.frame.ndraws = (uint32_t)n;
     }
@@ -1598,9 +1635,16 @@ VKAPI_ATTR VkResult VKAPI_CALL vkWaitForFences(VkDevice device, uint32_t n, cons
         // finite timeout: poll
         std::this_thread::sleep_for(std::chrono::microseconds(20));
     }
-    // the statistics fold waits for the whole queue: only when that costs
-    // nothing more than the wait itself
-    if (waitAll || hipStreamQuery(d->engine->stream()) == hipSuccess) d->engine->collect_stats();
+    // The statistics fold waits for the whole queue: only when that costs
+    // nothing more than the wait itself, or (list capacities grow from the
+    // counters it reads) after a number of waits with later frames in flight.
+    uint64_t last = 0;
+    for (uint32_t i = 0; i < n && waitAll; ++i) last = std::max(last, from<Fence>(fences[i])->submission);
+    if (last == d->engine->submissions() || hipStreamQuery(d->engine->stream()) == hipSuccess ||
+        (waitAll && ++d->waits_behind >= 16)) {
+        d->waits_behind = 0;
+        d->engine->collect_stats();
+    }
     return VK_SUCCESS;
 }
 
@@ -1623,7 +1667,18 @@ VKAPI_ATTR VkResult VKAPI_CALL vkQueueSubmit(VkQueue queue, uint32_t submitCount
     for (uint32_t s = 0; s < submitCount; ++s)
         for (uint32_t i = 0; i < submits[s].commandBufferCount; ++i) {
             CommandBuffer *cb = from<CommandBuffer>(submits[s].pCommandBuffers[i]);
-            hipError_t e = eng.execute(cb->ops, &cb->graph);
+            hipError_t e = hipSuccess;
+            for (size_t k = 0; k < cb->records_used && cb->records_pending && e == hipSuccess; ++k)
+                e = hipMemcpyAsync(cb->records[k].dev, cb->records[k].host, cb->records[k].bytes,
+                                   hipMemcpyHostToDevice, eng.stream());
+            if (e == hipSuccess) {
+                cb->records_pending = false;
+                e = eng.execute(cb->ops, &cb->graph);
+            }
+            if (cb->done) {
+                hipEventRecord(cb->done, eng.stream());
+                ++cb->submissions;
+            }
             if (e != hipSuccess) {
                 std::fprintf(stderr, "kazan: vkQueueSubmit: %s\n", hipGetErrorString(e));
                 return VK_ERROR_DEVICE_LOST;
@@ -1634,6 +1689,7 @@ VKAPI_ATTR VkResult VKAPI_CALL vkQueueSubmit(VkQueue queue, uint32_t submitCount
     if (f) {
         f->submitted = true;
         f->signaled = false;
+        f->submission = eng.submissions();
     }
     return VK_SUCCESS;
 }

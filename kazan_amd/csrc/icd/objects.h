@@ -50,6 +50,7 @@ struct Device : Dispatchable {
     PhysicalDevice *physical = nullptr;
     std::unique_ptr<Queue> queue;
     std::unique_ptr<Engine> engine;
+    uint32_t waits_behind = 0;  // fence waits since the statistics were read, frames after them in flight
 };
 
 struct DeviceMemory {
@@ -199,11 +200,23 @@ struct RecordState {
     bool batch_open = false;  // the last op is a batch that may take more draws
 };
 
+// A batch's draw records: in pinned memory as recorded, and on the device,
+// where the first submission after the recording copies them.
+struct DrawRecords {
+    char *host = nullptr, *dev = nullptr;
+    size_t cap = 0, bytes = 0;
+};
+
 struct CommandBuffer : Dispatchable {
     Device *device = nullptr;
     CommandPool *pool = nullptr;
     std::vector<Op> ops;
-    std::vector<void *> device_allocs;
+    // kept over recordings, the first `records_used` in use by this one
+    std::vector<DrawRecords> records;
+    size_t records_used = 0;
+    bool records_pending = false;  // recorded, not copied to the device yet
+    hipEvent_t done = nullptr;     // after this recording's last submission
+    uint32_t submissions = 0;      // of this recording
     GraphCache graph;  // the ops as a hipGraph, once captured
     RecordState st;
     bool recording = false;
@@ -213,6 +226,7 @@ struct Fence {
     hipEvent_t event = nullptr;
     bool submitted = false;
     bool signaled = false;
+    uint64_t submission = 0;  // the engine's count at its submission
     Device *device = nullptr;
 };
 
