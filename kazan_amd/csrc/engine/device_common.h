@@ -57,6 +57,8 @@ struct KzComputeFrame {
     uint32_t ssbo_bytes[KZ_MAX_SSBOS];  // the bound range of each storage buffer (OpArrayLength)
     uint32_t push[KZ_PUSH_WORDS];
     uint32_t base[3];
+    uint32_t per_block;  // workgroups (along x) of a block of the launch
+    uint32_t groups[3];  // dispatched
     uint32_t pad;
 };
 

@@ -1237,6 +1237,18 @@ static void record_dispatch(CommandBuffer *cb, uint32_t bx, uint32_t by, uint32_
     op.groups[2] = z;
     for (int k = 0; k < 3; ++k) op.block[k] = p->local_size[k];
     KzComputeFrame &f = op.cframe;
+    f.groups[0] = x;
+    f.groups[1] = y;
+    f.groups[2] = z;
+    f.per_block = 1;
+    if (p->cs_per_block > 1) {  // its kernel takes linear blocks
+        // several workgroups a block, unless the last block of a row would
+        // leave more than a fifth of the row's threads without one
+        f.per_block = x >= 4 * p->cs_per_block ? p->cs_per_block : 1u;
+        op.block[0] *= op.block[1] * op.block[2] * f.per_block;
+        op.block[1] = op.block[2] = 1;
+        op.groups[0] = (x + f.per_block - 1) / f.per_block;
+    }
     f.base[0] = bx;
     f.base[1] = by;
     f.base[2] = bz;

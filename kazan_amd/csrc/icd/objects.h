@@ -146,6 +146,7 @@ struct Pipeline {
     hipModule_t cs_module = nullptr;
     hipFunction_t cs_kernel = nullptr;
     uint32_t local_size[3] = {1, 1, 1};
+    uint32_t cs_per_block = 1;  // workgroups along x that a block may take
     std::map<std::pair<uint32_t, uint32_t>, uint32_t> ssbo_slot;
     ~Pipeline() {
         if (cs_module) hipModuleUnload(cs_module);

@@ -233,7 +233,7 @@ bool create_compute_pipeline(Device *dev, const VkComputePipelineCreateInfo *ci,
     cg.ubo_slot = p->ubo_slot;
     cg.ssbo_slot = p->ssbo_slot;
     std::string source;
-    if (!generate_compute_source(cmod, cg, source, err)) return false;
+    if (!generate_compute_source(cmod, cg, source, p->cs_per_block, err)) return false;
     std::vector<char> code;
     std::string log;
     if (!compile_compute_code(source, (ci->flags & 0x1u) == 0, code, log, nullptr)) {

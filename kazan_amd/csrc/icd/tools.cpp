@@ -157,7 +157,8 @@ extern "C" int kazan_compile_compute_spirv(const uint32_t *words, size_t nwords,
     for (size_t i = 0; i < ssbos.size() && i < KZ_MAX_SSBOS; ++i) cg.ssbo_slot[ssbos[i]] = (uint32_t)i;
     for (size_t i = 0; i < ubos.size() && i < KZ_MAX_UBOS; ++i) cg.ubo_slot[ubos[i]] = (uint32_t)i;
     std::string source;
-    if (!kz::generate_compute_source(m, cg, source, err)) return put(err, out, cap, out_len, -1);
+    uint32_t per_block = 1;
+    if (!kz::generate_compute_source(m, cg, source, per_block, err)) return put(err, out, cap, out_len, -1);
     if (what == 0) return put(source, out, cap, out_len, 0);
     if (what == 1) return put(kz::compute_full_source(source), out, cap, out_len, 0);
     std::vector<char> code;

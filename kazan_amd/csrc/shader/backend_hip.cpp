@@ -765,8 +765,13 @@ bool generate_pipeline_source(const PipelineCodegenInput &in, PipelineCodegenOut
     return true;
 }
 
+namespace {
+// threads of a block that takes several workgroups
+constexpr uint64_t kComputeBlock = 256;
+}  // namespace
+
 bool generate_compute_source(const ir::Module &cs, const PipelineCodegenInput &in, std::string &out,
-                             std::string &err) {
+                             uint32_t &per_block, std::string &err) {
     const uint32_t lx = cs.local_size[0], ly = cs.local_size[1], lz = cs.local_size[2];
     const uint64_t n = (uint64_t)lx * ly * lz;
     if (cs.stage != ir::Stage::Compute || n == 0 || n > 1024) {
@@ -783,18 +788,32 @@ bool generate_compute_source(const ir::Module &cs, const PipelineCodegenInput &i
     g.is_cs = true;
     if (!g.generate("kz_cs_main")) return false;
     os << g.os.str();
-    // the kernel: one workgroup per dispatched group, one thread per invocation
-    os << "extern \"C\" __global__ __launch_bounds__(" << n << ") void kz_compute(KzComputeFrame f) {\n";
+    // The kernel: one thread per invocation. Without workgroup memory and
+    // barriers a block takes up to `per_block` consecutive workgroups along x
+    // (f.per_block of them; the last block may have fewer): a dispatch of
+    // one-wave workgroups is bound by starting its blocks, 16.8 M saxpy
+    // elements in workgroups of 64 took 62 us, in blocks of four of them 45.
+    const bool alone = !cs.workgroup_variables.empty() || g.os.str().find("__syncthreads") != std::string::npos;
+    per_block = alone ? 1u : (uint32_t)std::max<uint64_t>(1, kComputeBlock / n);
+    os << "extern \"C\" __global__ __launch_bounds__(" << n * per_block << ") void kz_compute(KzComputeFrame f) {\n";
     os << "    const uint32_t L[3] = {" << lx << "u, " << ly << "u, " << lz << "u};\n";
-    os << "    const uint32_t lid[3] = {threadIdx.x, threadIdx.y, threadIdx.z};\n";
-    os << "    const uint32_t wid[3] = {blockIdx.x + f.base[0], blockIdx.y + f.base[1], blockIdx.z + f.base[2]};\n";
+    if (per_block > 1) {
+        os << "    const uint32_t li = threadIdx.x % " << n << "u;\n";
+        os << "    const uint32_t gx = blockIdx.x * f.per_block + threadIdx.x / " << n << "u;\n";
+        os << "    if (gx >= f.groups[0]) return;\n";
+        os << "    const uint32_t lid[3] = {li % L[0], li / L[0] % L[1], li / (L[0] * L[1])};\n";
+    } else {
+        os << "    const uint32_t gx = blockIdx.x;\n";
+        os << "    const uint32_t lid[3] = {threadIdx.x, threadIdx.y, threadIdx.z};\n";
+    }
+    os << "    const uint32_t wid[3] = {gx + f.base[0], blockIdx.y + f.base[1], blockIdx.z + f.base[2]};\n";
     os << "    uint32_t kz_ids[13];\n";
     os << "    for (int k = 0; k < 3; ++k) {\n";
     os << "        kz_ids[k] = wid[k] * L[k] + lid[k];\n";
     os << "        kz_ids[3 + k] = lid[k];\n";
     os << "        kz_ids[6 + k] = wid[k];\n";
     os << "    }\n";
-    os << "    kz_ids[9] = gridDim.x; kz_ids[10] = gridDim.y; kz_ids[11] = gridDim.z;\n";
+    os << "    kz_ids[9] = f.groups[0]; kz_ids[10] = f.groups[1]; kz_ids[11] = f.groups[2];\n";
     os << "    kz_ids[12] = lid[0] + L[0] * (lid[1] + L[1] * lid[2]);\n";
     os << "    float kz_in[4] = {}, kz_out[4] = {};\n";
     os << "    kz_cs_main(f, kz_ids, kz_in, kz_out);\n";

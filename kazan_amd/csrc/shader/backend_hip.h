@@ -55,7 +55,9 @@ bool generate_pipeline_source(const PipelineCodegenInput &in, PipelineCodegenOut
 // its workgroup memory, and the kernel kz_compute(KzComputeFrame) that runs
 // one workgroup per dispatched group (the module's local size as its block).
 // Uses in.ubo_slot and in.ssbo_slot for the descriptor bindings.
+// per_block: the workgroups along x that a block of the launch may take.
 bool generate_compute_source(const ir::Module &cs, const PipelineCodegenInput &in, std::string &out,
+                             uint32_t &per_block,
                              std::string &err);
 
 }  // namespace kz
