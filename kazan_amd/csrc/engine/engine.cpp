@@ -63,7 +63,7 @@ Engine::~Engine() {
     hipFree(tri_rec_);
     for (uint32_t *p : {tri_draw_, block_pairs_, chunk_offsets_, chunk_extra_, bin_ctrl_, tile_flag_, pair_keys_[0],
                         pair_keys_[1], pair_vals_[0], pair_vals_[1], radix_table_, radix_totals_, clip_of_, clip_tris_,
-                        clip_rec_, gather_seg_, gather_list_, super_state_})
+                        clip_rec_, gather_seg_, gather_list_, super_state_, zero_word_})
         hipFree(p);
     for (uint32_t *p : {tile_level_, split_slot_, split_info_, queue_, ctrl_, split_counts_, split_offsets_,
                         chunk_desc_, chunk_counts_, split_lists_, plan_table_, tile_acc_, tile_cycles_, tile_frags_, tri_z_})
@@ -112,6 +112,11 @@ bool Engine::init(int hip_device, std::string &err) {
         ((e = hipMalloc((void **)&bin_ctrl_, KZ_BIN_WORDS * sizeof(uint32_t))) != hipSuccess ||
          (e = kz_launch_fill_u32(stream_, bin_ctrl_, KZ_BIN_WORDS, 0u)) != hipSuccess ||
          (e = hipMalloc((void **)&radix_totals_, kz_radix_digits_max() * sizeof(uint32_t))) != hipSuccess)) {
+        err = hipGetErrorString(e);
+        return false;
+    }
+    if ((e = hipMalloc((void **)&zero_word_, sizeof(uint32_t))) != hipSuccess ||
+        (e = kz_launch_fill_u32(stream_, zero_word_, 1, 0u)) != hipSuccess) {
         err = hipGetErrorString(e);
         return false;
     }
@@ -607,6 +612,7 @@ hipError_t Engine::mark(int slot, bool end) {
 }
 
 BatchTuning::~BatchTuning() {
+    if (trial) hipGraphExecDestroy(trial);
     for (hipEvent_t e : ev)
         if (e) hipEventDestroy(e);
 }
@@ -667,17 +673,17 @@ int final_choice(const BatchTuning &t) {
 
 // Candidates, one HIP-event-timed trial per submission: every tile size
 // whose kernels fit (full grid, the plan with the cost model when there is
-// one); at the fastest size, a half and a quarter grid; at the fastest of
-// those, the plan without the model and the plain raster (one workgroup per
-// tile, no plan); at the fastest planned one, splits of at most 4 sub-tiles
-// and none (many small triangles are set up once per sub-tile they touch);
-// with a cost model, the model's plan with its fragment weight times 4 and
-// 16 (a pipeline whose fragments cost more than the training pipelines');
+// one); at the fastest size, a half grid and the plain raster (one workgroup
+// per tile, no plan); at the fastest of those, the plan without the model and
+// the plain raster of the next smaller tiles (the plain raster's neighbours
+// when it is the fastest); at the fastest planned one, splits of at most 4
+// sub-tiles and none (many small triangles are set up once per sub-tile they
+// touch); with a cost model, the model's plan with its fragment weight times 4
+// and 16 (a pipeline whose fragments cost more than the training pipelines');
 // at the fastest planned one, every other pair of tile size and grid size
-// (both were chosen with the deepest splits and the model; with fewer
-// splits smaller tiles on a larger grid may pay); then the three fastest
-// twice more each. The finalist with the lowest median of its three runs
-// is kept.
+// (both were chosen with the deepest splits and the model; with fewer splits
+// smaller tiles on a larger grid may pay); then the three fastest twice more
+// each. The finalist with the lowest median of its three runs is kept.
 hipError_t Engine::pick_config(Op &op, BatchConfig &cfg, bool &timed, bool tune) {
     cfg = default_config(op);
     timed = false;
@@ -717,10 +723,14 @@ hipError_t Engine::pick_config(Op &op, BatchConfig &cfg, bool &timed, bool tune)
             const BatchConfig b = t.cand[best];
             if (t.phase == 0) {
                 t.cand.push_back({b.shift, 2u, b.model, true, 2u, 1u});
-                t.cand.push_back({b.shift, 4u, b.model, true, 2u, 1u});
-            } else if (t.phase == 1) {
-                if (b.model) t.cand.push_back({b.shift, b.grid_div, false, true, 2u, 1u});
                 t.cand.push_back({b.shift, 1u, false, false, 2u, 1u});
+            } else if (t.phase == 1) {
+                // the plain raster has only its tiles to fill the chip with:
+                // smaller ones often suit it better than the plan's best
+                const uint32_t s = b.shift > kMinTileShift ? b.shift - 1 : b.shift + 1;
+                if (b.persistent && b.model) t.cand.push_back({b.shift, b.grid_div, false, true, 2u, 1u});
+                if (!b.persistent) t.cand.push_back({s > b.shift ? s + 1 : b.shift + 1, 1u, false, false, 2u, 1u});
+                t.cand.push_back({s, 1u, false, false, 2u, 1u});
             } else if (t.phase == 2) {
                 if (b.persistent) {
                     t.cand.push_back({b.shift, b.grid_div, b.model, true, 1u, 1u});
@@ -764,6 +774,8 @@ hipError_t Engine::pick_config(Op &op, BatchConfig &cfg, bool &timed, bool tune)
     }
     const int best = final_choice(t);
     t.done = true;
+    if (t.trial) hipGraphExecDestroy(t.trial);
+    t.trial = nullptr;
     if (best >= 0) t.choice = t.cand[best];
     else t.choice = default_config(op);
     cfg = t.choice;
@@ -831,6 +843,52 @@ hipError_t Engine::execute(std::vector<Op> &ops, GraphCache *cache) {
     return hipSuccess;
 }
 
+// A first launch of the one-workgroup-per-tile raster, on one tile without
+// triangles: the planned rasters of a tile size have theirs behind them in
+// the trials before, it would have its only one timed.
+hipError_t Engine::warm_raster(const PipelineKernels *kern) {
+    KzFrame f{};
+    f.tiles_x = f.tiles_y = 1;
+    f.tile_counts = f.tile_offsets = zero_word_;
+    f.list_capacity = 1;
+    void *args[] = {&f};
+    return hipModuleLaunchKernel(kern->raster, 1, 1, 1, 64, 1, 1, 0, stream_, args, nullptr);
+}
+
+// The batch as a timed trial, as a graph of its own where the choice will run
+// in one: a kernel of a replayed graph takes at least 4.5 us, launched by
+// itself half of that, so that trials of single launches favour plans of ten
+// small kernels. The device waits first until the host has queued the rest.
+// (With the plain raster tried at smaller tiles too, 131,072 Phong triangles
+// at 720p and four samples 167 us a frame -> 130.)
+hipError_t Engine::run_trial(const Op &op, const BatchConfig &cfg) {
+    BatchTuning &t = *op.tuning;
+    if (t.trial) hipGraphExecDestroy(t.trial);  // (the trial before has ended: its events were read)
+    t.trial = nullptr;
+    if (graphs_ && !kernel_timing_) {
+        const uint32_t b0 = pending_batches_, l0 = pending_launches_;
+        const uint64_t gen = generation_;
+        hipGraph_t graph = nullptr;
+        KZ_TRY(hipStreamBeginCapture(stream_, hipStreamCaptureModeRelaxed));
+        const hipError_t e = run_batch(op, cfg);
+        const hipError_t e2 = hipStreamEndCapture(stream_, &graph);
+        const bool ok = e == hipSuccess && e2 == hipSuccess && gen == generation_ &&
+                        hipGraphInstantiate(&t.trial, graph, nullptr, nullptr, 0) == hipSuccess &&
+                        hipGraphUpload(t.trial, stream_) == hipSuccess;
+        if (graph) hipGraphDestroy(graph);
+        if (!ok) {
+            t.trial = nullptr;
+            pending_batches_ = b0;
+            pending_launches_ = l0;
+            if (e != hipSuccess) return e;
+        }
+    }
+    KZ_TRY(kz_launch_wait(stream_));
+    KZ_TRY(hipEventRecord(t.ev[0], stream_));
+    KZ_TRY(t.trial ? hipGraphLaunch(t.trial, stream_) : run_batch(op, cfg));
+    return hipEventRecord(t.ev[1], stream_);
+}
+
 hipError_t Engine::execute_eager(std::vector<Op> &ops, bool tune) {
     for (Op &op : ops)
         if (op.kind == Op::Batch) {
@@ -840,11 +898,14 @@ hipError_t Engine::execute_eager(std::vector<Op> &ops, bool tune) {
             if (timed) {
                 // a trial times the batch, not the loading of a tile size's
                 // kernels or the growth of its scratch (host work and syncs)
-                if (op.variants->get(cfg.shift)) KZ_TRY(prepare_batch(op, cfg.shift));
-                KZ_TRY(hipEventRecord(op.tuning->ev[0], stream_));
+                if (const PipelineKernels *kern = op.variants->get(cfg.shift)) {
+                    KZ_TRY(prepare_batch(op, cfg.shift));
+                    if (!cfg.persistent) KZ_TRY(warm_raster(kern));
+                }
+                KZ_TRY(run_trial(op, cfg));
+            } else {
+                KZ_TRY(run_batch(op, cfg));
             }
-            KZ_TRY(run_batch(op, cfg));
-            if (timed) KZ_TRY(hipEventRecord(op.tuning->ev[1], stream_));
         } else {
             KZ_TRY(launch_ops_one(op));
         }

@@ -151,6 +151,7 @@ struct BatchTuning {
     uint32_t next = 0;               // next candidate to try
     int pending = -1;                // candidate whose events are in flight
     hipEvent_t ev[2] = {nullptr, nullptr};
+    hipGraphExec_t trial = nullptr;  // the last trial's graph
     BatchConfig choice;              // once done
 };
 
@@ -298,6 +299,9 @@ class Engine {
     hipError_t prepare_batch(const Op &op, uint32_t shift);
     hipError_t run_batch(const Op &op, const BatchConfig &cfg);
     hipError_t execute_eager(std::vector<Op> &ops, bool tune = true);
+    hipError_t warm_raster(const PipelineKernels *kern);
+    hipError_t run_trial(const Op &op, const BatchConfig &cfg);
+    uint32_t *zero_word_ = nullptr;
     hipError_t launch_ops(std::vector<Op> &ops);  // tuned configurations, no tuning events
     hipError_t launch_ops_one(const Op &op);      // a non-batch op
     hipError_t mark(int slot, bool end);

@@ -140,6 +140,11 @@ __global__ void kz_fill_u32(uint32_t *dst, uint64_t n, uint32_t value) {
 }
 
 // Fills a rectangle of a W-wide attachment with `spp` 32-bit values per pixel.
+// (a sleep of 127 is 8,128 cycles, about 3.4 us)
+__global__ void kz_wait() {
+    for (int i = 0; i < 30; ++i) __builtin_amdgcn_s_sleep(127);
+}
+
 __global__ void kz_fill_rect_u32(uint32_t *dst, uint32_t width, int32_t x0, int32_t y0, uint32_t w, uint32_t h,
                                  uint32_t spp, uint32_t value) {
     const uint64_t n = (uint64_t)w * h * spp;
@@ -2404,6 +2409,11 @@ uint32_t bin_chunk(uint32_t ntris) {
 hipError_t kz_launch_fill_u32(hipStream_t st, uint32_t *dst, uint64_t n, uint32_t value) {
     if (n == 0) return hipSuccess;
     kz_fill_u32<<<grid_for(n, 256), 256, 0, st>>>(dst, n, value);
+    return hipGetLastError();
+}
+
+hipError_t kz_launch_wait(hipStream_t st) {
+    kz_wait<<<1, 64, 0, st>>>();
     return hipGetLastError();
 }
 
