@@ -787,26 +787,44 @@ __global__ __launch_bounds__(kPairThreads) void kz_pair_write(const uint64_t *re
 }
 
 // The lanes of `valid` whose digit (of `bits` bits) equals this lane's.
-__device__ __forceinline__ uint64_t digit_match(uint32_t d, uint32_t bits, uint64_t valid) {
-    uint64_t m = valid;
-    for (uint32_t i = 0; i < bits; ++i) {
-        const bool bit = (d >> i) & 1u;
-        const uint64_t b = __ballot(bit);
-        m &= bit ? b : ~b;
+// In 32-bit halves: a bit is one compare and, for each half, one three-input
+// operation (64-bit selects between the ballot and its complement are twice
+// that).
+template <uint32_t BITS>
+__device__ __forceinline__ uint64_t digit_match(uint32_t d, uint64_t valid) {
+    uint32_t lo = (uint32_t)valid, hi = (uint32_t)(valid >> 32);
+#pragma unroll
+    for (uint32_t i = 0; i < BITS; ++i) {
+        const uint32_t t = (uint32_t)((int32_t)(d << (31 - i)) >> 31);  // bit i in every bit
+        const uint64_t b = __ballot(t != 0);
+        lo &= ~((uint32_t)b ^ t);
+        hi &= ~((uint32_t)(b >> 32) ^ t);
     }
-    return m;
+    return lo | ((uint64_t)hi << 32);
+}
+
+// Block b of n (on XCD b % 8) to a contiguous range of blocks per XCD, a
+// bijection of [0, n): neighbouring blocks write neighbouring words of the
+// digit table and neighbouring runs of a digit's range, a few words each, and
+// only within one XCD's L2 do these become whole lines.
+__device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t n) {
+    const uint32_t xcd = b & 7u, k = b >> 3, q = n >> 3, r = n & 7u;
+    return xcd * q + min(xcd, r) + k;
 }
 
 // Histogram of the digit (key >> shift) & (2^bits - 1) per block of
-// kRadixBlock pairs: table[digit * tstride + block]. A wave counts one
-// digit group per ballot match, so a skewed digit costs no LDS contention.
+// kRadixBlock pairs: table[digit * tstride + block]. One LDS add per pair:
+// 64 pairs of one digit (a skewed frame) are 64 adds to one word, still less
+// than finding that out by ballots did. With neighbouring blocks on one XCD,
+// 10 M pairs by 9 and 8 bits take 39 us (both passes), 52 before.
 __global__ __launch_bounds__(kRadixThreads) void kz_radix_hist(const uint32_t *keys, const uint32_t *ctrl,
                                                                uint32_t shift, uint32_t bits, uint32_t *table,
                                                                uint32_t tstride) {
     __shared__ uint32_t s_cnt[kRadixMaxDigits];
     const uint32_t npairs = ctrl[KZ_BIN_PAIRS];
-    const uint32_t b0 = blockIdx.x * kRadixBlock;
-    if (b0 >= npairs) return;
+    const uint32_t nb = (npairs + kRadixBlock - 1) / kRadixBlock;
+    if (blockIdx.x >= nb) return;
+    const uint32_t blk = xcd_remap(blockIdx.x, nb), b0 = blk * kRadixBlock;
     const uint32_t nd = 1u << bits, tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
     for (uint32_t i = tid; i < nd; i += kRadixThreads) s_cnt[i] = 0;
     __syncthreads();
@@ -818,13 +836,10 @@ __global__ __launch_bounds__(kRadixThreads) void kz_radix_hist(const uint32_t *k
         dg[r] = i < npairs ? (keys[i] >> shift) & (nd - 1) : kNone;
     }
 #pragma unroll
-    for (uint32_t r = 0; r < kRadixRounds; ++r) {
-        const bool ok = dg[r] != kNone;
-        const uint64_t m = digit_match(dg[r], bits, __ballot(ok));
-        if (ok && rank_in(m) == 0) atomicAdd(&s_cnt[dg[r]], (uint32_t)__popcll(m));
-    }
+    for (uint32_t r = 0; r < kRadixRounds; ++r)
+        if (dg[r] != kNone) atomicAdd(&s_cnt[dg[r]], 1u);
     __syncthreads();
-    for (uint32_t i = tid; i < nd; i += kRadixThreads) table[(size_t)i * tstride + blockIdx.x] = s_cnt[i];
+    for (uint32_t i = tid; i < nd; i += kRadixThreads) table[(size_t)i * tstride + blk] = s_cnt[i];
 }
 
 // Exclusive scan of each digit's row over the blocks in use (one workgroup
@@ -843,14 +858,7 @@ __global__ __launch_bounds__(kScanThreads) void kz_radix_scan(uint32_t *table, u
 __device__ void radix_scan2(uint32_t *a, uint32_t *b, uint32_t n, uint32_t *s_wa, uint32_t *s_wb) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t va = tid < n ? a[tid] : 0u, vb = tid < n ? b[tid] : 0u;
-    uint32_t xa = va, xb = vb;
-    for (uint32_t d = 1; d < 64; d <<= 1) {
-        const uint32_t oa = __shfl_up(xa, d, 64), ob = __shfl_up(xb, d, 64);
-        if (lane >= d) {
-            xa += oa;
-            xb += ob;
-        }
-    }
+    const uint32_t xa = kz_wave_incl_scan(va), xb = kz_wave_incl_scan(vb);
     if (lane == 63) {
         s_wa[wave] = xa;
         s_wb[wave] = xb;
@@ -906,23 +914,31 @@ struct RadixAcc {
 // (and, with acc, adds the pair statistics). With list_mask (keys that
 // carry a sub-tile mask above 16 tile bits) the last pass also writes each
 // entry's mask beside the list.
-__global__ __launch_bounds__(kRadixThreads) void kz_radix_scatter(const uint32_t *keys_in, const uint32_t *vals_in,
+// The waves' counts lie where the regrouped block goes (their places are in
+// registers by then): 37 KB of LDS, four workgroups a CU. Bound by its
+// scattered runs' partial lines (neighbouring blocks on one XCD: 10 M pairs by
+// 9 bits 69 us -> 40) and, in the last pass, by the tiles' atomics (69 -> 65).
+template <uint32_t BITS, bool LAST, bool ACC>
+__global__ __launch_bounds__(kRadixThreads) __attribute__((amdgpu_waves_per_eu(ACC ? 4 : 8))) void kz_radix_scatter(const uint32_t *keys_in, const uint32_t *vals_in,
                                                                   uint32_t *keys_out, uint32_t *vals_out,
                                                                   uint32_t *lists, uint16_t *list_mask,
                                                                   uint32_t *tile_counts,
                                                                   uint32_t *tile_offsets,
                                                                   const uint32_t *ctrl, const uint32_t *table,
                                                                   uint32_t tstride, const uint32_t *totals,
-                                                                  uint32_t shift, uint32_t bits, RadixAcc acc) {
-    __shared__ uint32_t s_wcnt[kRadixWaves * kRadixMaxDigits];
-    __shared__ uint32_t s_lstart[kRadixMaxDigits], s_gbase[kRadixMaxDigits];
-    __shared__ uint32_t s_key[kRadixBlock], s_val[kRadixBlock];
+                                                                  uint32_t shift, RadixAcc acc) {
+    __shared__ uint32_t s_lstart[1u << BITS], s_gbase[1u << BITS];
+    __shared__ uint32_t s_pairs[2 * kRadixBlock];
     __shared__ uint32_t s_wa[kRadixWaves], s_wb[kRadixWaves];
+    static_assert((kRadixWaves << BITS) <= 2 * kRadixBlock, "the counts fit where the pairs go");
+    uint32_t *const s_wcnt = s_pairs, *const s_key = s_pairs, *const s_val = s_pairs + kRadixBlock;
+    constexpr uint32_t nd = 1u << BITS, dmask = nd - 1;
     const uint32_t npairs = ctrl[KZ_BIN_PAIRS];
-    const uint32_t b0 = blockIdx.x * kRadixBlock;
-    if (b0 >= npairs) return;
+    const uint32_t nb = (npairs + kRadixBlock - 1) / kRadixBlock;
+    if (blockIdx.x >= nb) return;
+    const uint32_t blk = xcd_remap(blockIdx.x, nb), b0 = blk * kRadixBlock;
     const uint32_t nitems = min(kRadixBlock, npairs - b0);
-    const uint32_t nd = 1u << bits, dmask = nd - 1, tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
     for (uint32_t i = tid; i < kRadixWaves * nd; i += kRadixThreads) s_wcnt[i] = 0;
     __syncthreads();
 
@@ -941,7 +957,7 @@ __global__ __launch_bounds__(kRadixThreads) void kz_radix_scatter(const uint32_t
     for (uint32_t r = 0; r < kRadixRounds; ++r) {
         const bool ok = key[r] != kNone;
         const uint32_t d = (key[r] >> shift) & dmask;
-        const uint64_t m = digit_match(d, bits, __ballot(ok));
+        const uint64_t m = digit_match<BITS>(d, __ballot(ok));
         const uint32_t lead = ok ? (uint32_t)__builtin_ctzll(m) : lane;
         uint32_t old = 0;
         if (ok && lead == lane) {
@@ -966,20 +982,23 @@ __global__ __launch_bounds__(kRadixThreads) void kz_radix_scatter(const uint32_t
     }
     __syncthreads();
     radix_scan2(s_lstart, s_gbase, nd, s_wa, s_wb);
-    for (uint32_t d = tid; d < nd; d += kRadixThreads) s_gbase[d] += table[(size_t)d * tstride + blockIdx.x];
+    for (uint32_t d = tid; d < nd; d += kRadixThreads) s_gbase[d] += table[(size_t)d * tstride + blk];
 #pragma unroll
     for (uint32_t r = 0; r < kRadixRounds; ++r) {
-        if (key[r] == kNone) continue;
         const uint32_t d = (key[r] >> shift) & dmask;
-        const uint32_t p = s_lstart[d] + wcnt[d] + rk[r];  // < nitems by construction
-        if (p < nitems) {
-            s_key[p] = key[r];
-            s_val[p] = val[r];
-        }
+        rk[r] = key[r] == kNone ? kNone : s_lstart[d] + wcnt[d] + rk[r];  // < nitems by construction
     }
+    __syncthreads();  // the counts have been read
+#pragma unroll
+    for (uint32_t r = 0; r < kRadixRounds; ++r)
+        if (rk[r] < nitems) {
+            s_key[rk[r]] = key[r];
+            s_val[rk[r]] = val[r];
+        }
     __syncthreads();
 
     // out, digit run by digit run
+#pragma unroll(ACC ? 1 : 4)
     for (uint32_t j0 = 0; j0 < nitems; j0 += kRadixThreads) {
         const uint32_t j = j0 + tid;
         const bool ok = j < nitems;
@@ -989,7 +1008,7 @@ __global__ __launch_bounds__(kRadixThreads) void kz_radix_scatter(const uint32_t
             const uint32_t d = (kk >> shift) & dmask;
             g = s_gbase[d] + (j - s_lstart[d]);  // < npairs by construction
             if (g < npairs) {
-                if (lists) {
+                if (LAST) {
                     lists[g] = v;
                     if (list_mask) list_mask[g] = (uint16_t)(kk >> 16);
                 } else {
@@ -998,7 +1017,7 @@ __global__ __launch_bounds__(kRadixThreads) void kz_radix_scatter(const uint32_t
                 }
             }
         }
-        if (!lists) continue;
+        if (!LAST) continue;
         const uint32_t k = ok && list_mask ? kk & 0xFFFFu : kk;  // the tile
         // the last pass's block is sorted by tile: one update per run of a tile
         const Run run = run_of(k, lane);
@@ -1006,7 +1025,7 @@ __global__ __launch_bounds__(kRadixThreads) void kz_radix_scatter(const uint32_t
             atomicAdd(&tile_counts[k], run.len);
             atomicMin(&tile_offsets[k], g);
         }
-        if (!acc.acc) continue;
+        if (!ACC) continue;
         uint32_t area = 0, lo = 0, hi = 0, zinv = 0, zmax = 0;
         if (ok) {
             uint32_t x0, y0, x1, y1;
@@ -1410,7 +1429,7 @@ __device__ __forceinline__ uint32_t cost_bucket(float cost) {
 __device__ __forceinline__ uint32_t bucket_reserve(uint32_t *s, uint32_t bucket, uint32_t items, bool active) {
     const uint32_t lane = lane_id();
     const bool single = active && items == 1;
-    const uint64_t m = digit_match(bucket, 5, __ballot(single));
+    const uint64_t m = digit_match<5>(bucket, __ballot(single));
     uint32_t base = 0;
     if (single && rank_in(m) == 0) base = atomicAdd(&s[bucket], (uint32_t)__popcll(m));
     const uint32_t lead = single ? (uint32_t)__builtin_ctzll(m) : lane;
@@ -2465,25 +2484,59 @@ hipError_t kz_launch_gather_lists(hipStream_t st, const KzFrame &f) {
     return hipGetLastError();
 }
 
+namespace {
+template <uint32_t BITS>
+hipError_t radix_scatter_bits(hipStream_t st, const KzFrame &f, const KzRadixScratch &s, uint32_t in, uint32_t shift,
+                              bool last) {
+    const uint32_t out = in ^ 1u;
+    const RadixAcc none{nullptr, nullptr, nullptr, 0, 0, 0};
+    const RadixAcc acc{f.tri_rect, f.tri_z, f.tile_acc, f.tile_shift, f.tiles_x, f.total_tris};
+    if (!last)
+        kz_radix_scatter<BITS, false, false><<<s.tstride, kRadixThreads, 0, st>>>(
+            s.keys[in], s.vals[in], s.keys[out], s.vals[out], nullptr, nullptr, nullptr, nullptr, s.ctrl, s.table,
+            s.tstride, s.totals, shift, none);
+    else if (!f.tile_acc)
+        kz_radix_scatter<BITS, true, false><<<s.tstride, kRadixThreads, 0, st>>>(
+            s.keys[in], s.vals[in], nullptr, nullptr, f.tile_lists, (uint16_t *)f.list_mask, f.tile_counts,
+            f.tile_offsets, s.ctrl, s.table, s.tstride, s.totals, shift, none);
+    else
+        kz_radix_scatter<BITS, true, true><<<s.tstride, kRadixThreads, 0, st>>>(
+            s.keys[in], s.vals[in], nullptr, nullptr, f.tile_lists, (uint16_t *)f.list_mask, f.tile_counts,
+            f.tile_offsets, s.ctrl, s.table, s.tstride, s.totals, shift, acc);
+    return hipGetLastError();
+}
+
+hipError_t radix_scatter(hipStream_t st, const KzFrame &f, const KzRadixScratch &s, uint32_t in, uint32_t shift,
+                         uint32_t bits, bool last) {
+    switch (bits) {
+    case 1: return radix_scatter_bits<1>(st, f, s, in, shift, last);
+    case 2: return radix_scatter_bits<2>(st, f, s, in, shift, last);
+    case 3: return radix_scatter_bits<3>(st, f, s, in, shift, last);
+    case 4: return radix_scatter_bits<4>(st, f, s, in, shift, last);
+    case 5: return radix_scatter_bits<5>(st, f, s, in, shift, last);
+    case 6: return radix_scatter_bits<6>(st, f, s, in, shift, last);
+    case 7: return radix_scatter_bits<7>(st, f, s, in, shift, last);
+    case 8: return radix_scatter_bits<8>(st, f, s, in, shift, last);
+    case 9: return radix_scatter_bits<9>(st, f, s, in, shift, last);
+    default: return hipErrorInvalidValue;  // (digits are at most kRadixMaxBits)
+    }
+}
+}  // namespace
+
 hipError_t kz_launch_bin_radix(hipStream_t st, const KzFrame &f, const KzRadixScratch &s, uint32_t ntiles) {
     if (f.total_tris == 0) return hipSuccess;
     uint32_t bits = 1;
     while (bits < 32 && (1ull << bits) < ntiles) ++bits;
     const uint32_t passes = kz_radix_passes(ntiles);
     const uint32_t d = (bits + passes - 1) / passes;
-    RadixAcc acc{f.tri_rect, f.tri_z, f.tile_acc, f.tile_shift, f.tiles_x, f.total_tris};
     for (uint32_t p = 0; p < passes; ++p) {
-        const uint32_t in = p & 1u, out = in ^ 1u;
+        const uint32_t in = p & 1u;
         const uint32_t shift = p * d, pb = std::min(d, bits - shift);
         const bool last = p + 1 == passes;
         kz_radix_hist<<<s.tstride, kRadixThreads, 0, st>>>(s.keys[in], s.ctrl, shift, pb, s.table, s.tstride);
         kz_radix_scan<<<1u << pb, kScanThreads, 0, st>>>(s.table, s.tstride, s.ctrl, s.totals);
-        kz_radix_scatter<<<s.tstride, kRadixThreads, 0, st>>>(
-            s.keys[in], s.vals[in], last ? nullptr : s.keys[out], last ? nullptr : s.vals[out],
-            last ? f.tile_lists : nullptr, last ? (uint16_t *)f.list_mask : nullptr, last ? f.tile_counts : nullptr,
-            last ? f.tile_offsets : nullptr, s.ctrl,
-            s.table, s.tstride, s.totals,
-            shift, pb, last ? acc : RadixAcc{nullptr, nullptr, nullptr, 0, 0, 0});
+        const hipError_t e = radix_scatter(st, f, s, in, shift, pb, last);
+        if (e != hipSuccess) return e;
     }
     return hipGetLastError();
 }
