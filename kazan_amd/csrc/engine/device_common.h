@@ -175,6 +175,10 @@ struct KzFrame {
     uint32_t clear_mask;
     uint32_t clear_color;       // packed RGBA8
     float clear_depth;
+    // The render pass's resolve of the colour attachment over the whole
+    // framebuffer, folded into its last batch (4 samples, colour clear
+    // folded: every tile is written), or null
+    uint32_t *resolve;
 };
 
 // Per-tile pair statistics (tile_acc) over the (triangle, tile) pairs; the

@@ -1348,6 +1348,18 @@ VKAPI_ATTR void VKAPI_CALL vkCmdEndRenderPass(VkCommandBuffer commandBuffer) {
         op.y0 = st.render_area.offset.y;
         op.w = std::min<uint32_t>(st.render_area.extent.width, dst->width - (uint32_t)op.x0);
         op.h = std::min<uint32_t>(st.render_area.extent.height, dst->height - (uint32_t)op.y0);
+        // A batch just before, whose raster writes every pixel of the source
+        // (its clear is folded in), resolves it as it writes it.
+        if (!cb->ops.empty() && cb->ops.back().kind == Op::Batch) {
+            Op &last = cb->ops.back();
+            KzFrame &f = last.frame;
+            if (last.variants->fixed.samples == 4 && (f.clear_mask & 1u) && f.color == src->address() && !f.resolve &&
+                f.total_tris > 0 && op.x0 == 0 && op.y0 == 0 && op.w == f.width && op.h == f.height &&
+                op.rwidth == f.width) {
+                f.resolve = op.rdst;
+                continue;
+            }
+        }
         cb->ops.push_back(op);
     }
     st.render_pass = nullptr;
