@@ -524,17 +524,6 @@ __device__ __forceinline__ uint32_t kz_walk_mask(const KzWalk &w) {
     return m;
 }
 
-// whether any sample of the current pixel is inside: a sample is outside iff
-// its OR is negative, all are iff the AND of those is
-__device__ __forceinline__ bool kz_walk_any(const KzWalk &w) {
-    int32_t m = -1;
-#pragma unroll
-    for (int s = 0; s < KZ_SAMPLES; ++s)
-        m &= (int32_t)(((uint32_t)w.e[0] + (uint32_t)w.o[0][s]) | ((uint32_t)w.e[1] + (uint32_t)w.o[1][s]) |
-                       ((uint32_t)w.e[2] + (uint32_t)w.o[2][s]));
-    return m >= 0;
-}
-
 // to the next pixel; `wrap`: the current one ends its row
 __device__ __forceinline__ void kz_walk_step(KzWalk &w, bool wrap) {
 #pragma unroll
@@ -750,7 +739,7 @@ extern "C" __global__ __launch_bounds__(KZ_BIN_BLOCK) void kz_bin_count(KzFrame 
                     int32_t px = t.px0, py = t.py0;
                     const int32_t nc = (t.px1 - t.px0 + 1) * (t.py1 - t.py0 + 1);
                     for (int32_t j = 0; j < nc; ++j) {
-                        if (kz_walk_any(wk)) {
+                        if (kz_walk_mask(wk)) {
                             cx0 = min(cx0, px);
                             cx1 = max(cx1, px);
                             cy0 = min(cy0, py);
