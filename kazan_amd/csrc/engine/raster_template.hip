@@ -1315,7 +1315,8 @@ __device__ __forceinline__ void kz_resolve(const KzFrame &f, const KzLaneTri &L,
 // leaves lanes idle where a candidate is not covered, so it is for batches
 // of larger triangles (the rule is in kz_raster_rect): raster of 1,024 large
 // triangles at 256^2 128 us -> 69; a frame of 40,400 triangles around a
-// camera 645 -> 267.
+// camera 645 -> 267, and with the triangle's constants read once per triangle
+// instead of once per 64 candidates a later 242 -> 222.
 __device__ __forceinline__ void kz_direct(const KzFrame &f, const KzLaneTri &L, const KzTileCov &lc, bool narrow,
                                           int32_t X0, int32_t Y0, uint64_t m, uint32_t lane, uint32_t *s_color,
                                           float *s_depth, unsigned long long &nfrag,
@@ -1327,6 +1328,14 @@ __device__ __forceinline__ void kz_direct(const KzFrame &f, const KzLaneTri &L, 
         const int32_t bx0 = kz_readlane_i(L.cx0, b) - X0, by0 = kz_readlane_i(L.cy0, b) - Y0;
         const int32_t bw = kz_readlane_i(L.cx1, b) - X0 - bx0 + 1;
         const int32_t bc = bw * (kz_readlane_i(L.cy1, b) - Y0 - by0 + 1);
+        const int32_t x0 = kz_readlane_i(L.t.x0, b), y0 = kz_readlane_i(L.t.y0, b);
+        const int32_t d1x = kz_readlane_i(L.t.d1x, b), d1y = kz_readlane_i(L.t.d1y, b);
+        const int32_t d2x = kz_readlane_i(L.t.d2x, b), d2y = kz_readlane_i(L.t.d2y, b);
+        const int32_t s_lo = kz_readlane_i((int32_t)(uint32_t)(uint64_t)L.t.S, b);
+        const int32_t s_hi = kz_readlane_i((int32_t)((uint64_t)L.t.S >> 32), b);
+        const int64_t S = (int64_t)(((uint64_t)(uint32_t)s_lo) | ((uint64_t)(uint32_t)s_hi << 32));
+        const float invS = kz_readlane_f(L.t.invS, b);
+        const float z0 = kz_readlane_f(L.t.z0, b), dz1 = kz_readlane_f(L.t.dz1, b), dz2 = kz_readlane_f(L.t.dz2, b);
         // (candidate i's row as in phase 1 of kz_raster_rect)
         const float rbw = __builtin_amdgcn_rcpf((float)bw);
         for (int32_t i0 = 0; i0 < bc; i0 += 64) {
@@ -1338,14 +1347,6 @@ __device__ __forceinline__ void kz_direct(const KzFrame &f, const KzLaneTri &L, 
             nfrag += kz_wave_samples(mask);
             const uint32_t pix = mask ? (uint32_t)(ly * KZ_TS + lx) : 0u;
             const int32_t px = X0 + lx, py = Y0 + ly;
-            const int32_t x0 = kz_readlane_i(L.t.x0, b), y0 = kz_readlane_i(L.t.y0, b);
-            const int32_t d1x = kz_readlane_i(L.t.d1x, b), d1y = kz_readlane_i(L.t.d1y, b);
-            const int32_t d2x = kz_readlane_i(L.t.d2x, b), d2y = kz_readlane_i(L.t.d2y, b);
-            const int32_t s_lo = kz_readlane_i((int32_t)(uint32_t)(uint64_t)L.t.S, b);
-            const int32_t s_hi = kz_readlane_i((int32_t)((uint64_t)L.t.S >> 32), b);
-            const int64_t S = (int64_t)(((uint64_t)(uint32_t)s_lo) | ((uint64_t)(uint32_t)s_hi << 32));
-            const float invS = kz_readlane_f(L.t.invS, b);
-            const float z0 = kz_readlane_f(L.t.z0, b), dz1 = kz_readlane_f(L.t.dz1, b), dz2 = kz_readlane_f(L.t.dz2, b);
             float zs[KZ_SAMPLES], c01 = 0.0f, c20 = 0.0f, c12 = 0.0f;
             uint32_t maybe = 0;
 #pragma unroll
