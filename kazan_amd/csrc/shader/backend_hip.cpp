@@ -767,7 +767,7 @@ bool generate_pipeline_source(const PipelineCodegenInput &in, PipelineCodegenOut
 
 namespace {
 // threads of a block that takes several workgroups
-constexpr uint64_t kComputeBlock = 256;
+constexpr uint64_t kComputeBlock = 512;
 }  // namespace
 
 bool generate_compute_source(const ir::Module &cs, const PipelineCodegenInput &in, std::string &out,
@@ -792,7 +792,8 @@ bool generate_compute_source(const ir::Module &cs, const PipelineCodegenInput &i
     // barriers a block takes up to `per_block` consecutive workgroups along x
     // (f.per_block of them; the last block may have fewer): a dispatch of
     // one-wave workgroups is bound by starting its blocks, 16.8 M saxpy
-    // elements in workgroups of 64 took 62 us, in blocks of four of them 45.
+    // elements in workgroups of 64 took 62 us, in blocks of four of them 47, of
+    // eight 44.5.
     const bool alone = !cs.workgroup_variables.empty() || g.os.str().find("__syncthreads") != std::string::npos;
     per_block = alone ? 1u : (uint32_t)std::max<uint64_t>(1, kComputeBlock / n);
     os << "extern \"C\" __global__ __launch_bounds__(" << n * per_block << ") void kz_compute(KzComputeFrame f) {\n";
