@@ -796,9 +796,9 @@ hipError_t Engine::execute(std::vector<Op> &ops, GraphCache *cache) {
     if (!graphable || !draws || (cache->eager_runs == 0 && !cache->exec)) {
         // a command buffer recorded for every frame would run its first trial
         // in all of them, and never learn from it
-        const bool tune = !cache || !cache->recorded_per_frame || cache->eager_runs > 0;
+        const bool first = cache && cache->eager_runs == 0;
         if (cache) ++cache->eager_runs;
-        return execute_eager(ops, tune);
+        return execute_eager(ops, !first || !cache->recorded_per_frame, !first);
     }
     // every allocation before the capture
     for (Op &op : ops)
@@ -859,37 +859,42 @@ hipError_t Engine::warm_raster(const PipelineKernels *kern) {
 // in one: a kernel of a replayed graph takes at least 4.5 us, launched by
 // itself half of that, so that trials of single launches favour plans of ten
 // small kernels. The device waits first until the host has queued the rest.
+// Not so (`graph`) in a recording's first submission, which may be its only
+// one: the graph would cost it 0.2 ms.
 // (With the plain raster tried at smaller tiles too, 131,072 Phong triangles
 // at 720p and four samples 167 us a frame -> 130.)
-hipError_t Engine::run_trial(const Op &op, const BatchConfig &cfg) {
+hipError_t Engine::run_trial(const Op &op, const BatchConfig &cfg, bool graph) {
     BatchTuning &t = *op.tuning;
     if (t.trial) hipGraphExecDestroy(t.trial);  // (the trial before has ended: its events were read)
     t.trial = nullptr;
-    if (graphs_ && !kernel_timing_) {
+    if (graph && graphs_ && !kernel_timing_) {
         const uint32_t b0 = pending_batches_, l0 = pending_launches_;
         const uint64_t gen = generation_;
-        hipGraph_t graph = nullptr;
+        hipGraph_t captured = nullptr;
         KZ_TRY(hipStreamBeginCapture(stream_, hipStreamCaptureModeRelaxed));
         const hipError_t e = run_batch(op, cfg);
-        const hipError_t e2 = hipStreamEndCapture(stream_, &graph);
-        const bool ok = e == hipSuccess && e2 == hipSuccess && gen == generation_ &&
-                        hipGraphInstantiate(&t.trial, graph, nullptr, nullptr, 0) == hipSuccess &&
-                        hipGraphUpload(t.trial, stream_) == hipSuccess;
-        if (graph) hipGraphDestroy(graph);
-        if (!ok) {
+        const hipError_t e2 = hipStreamEndCapture(stream_, &captured);
+        if (e != hipSuccess || e2 != hipSuccess || gen != generation_ ||
+            hipGraphInstantiate(&t.trial, captured, nullptr, nullptr, 0) != hipSuccess)
             t.trial = nullptr;
+        else if (hipGraphUpload(t.trial, stream_) != hipSuccess) {
+            hipGraphExecDestroy(t.trial);
+            t.trial = nullptr;
+        }
+        if (captured) hipGraphDestroy(captured);
+        if (!t.trial) {  // launched by itself instead
             pending_batches_ = b0;
             pending_launches_ = l0;
             if (e != hipSuccess) return e;
         }
     }
-    KZ_TRY(kz_launch_wait(stream_));
+    if (graph) KZ_TRY(kz_launch_wait(stream_));
     KZ_TRY(hipEventRecord(t.ev[0], stream_));
     KZ_TRY(t.trial ? hipGraphLaunch(t.trial, stream_) : run_batch(op, cfg));
     return hipEventRecord(t.ev[1], stream_);
 }
 
-hipError_t Engine::execute_eager(std::vector<Op> &ops, bool tune) {
+hipError_t Engine::execute_eager(std::vector<Op> &ops, bool tune, bool graph_trials) {
     for (Op &op : ops)
         if (op.kind == Op::Batch) {
             BatchConfig cfg;
@@ -902,7 +907,7 @@ hipError_t Engine::execute_eager(std::vector<Op> &ops, bool tune) {
                     KZ_TRY(prepare_batch(op, cfg.shift));
                     if (!cfg.persistent) KZ_TRY(warm_raster(kern));
                 }
-                KZ_TRY(run_trial(op, cfg));
+                KZ_TRY(run_trial(op, cfg, graph_trials));
             } else {
                 KZ_TRY(run_batch(op, cfg));
             }

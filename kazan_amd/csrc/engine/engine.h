@@ -298,9 +298,9 @@ class Engine {
     BatchConfig default_config(const Op &op) const;
     hipError_t prepare_batch(const Op &op, uint32_t shift);
     hipError_t run_batch(const Op &op, const BatchConfig &cfg);
-    hipError_t execute_eager(std::vector<Op> &ops, bool tune = true);
+    hipError_t execute_eager(std::vector<Op> &ops, bool tune = true, bool graph_trials = true);
     hipError_t warm_raster(const PipelineKernels *kern);
-    hipError_t run_trial(const Op &op, const BatchConfig &cfg);
+    hipError_t run_trial(const Op &op, const BatchConfig &cfg, bool graph);
     uint32_t *zero_word_ = nullptr;
     hipError_t launch_ops(std::vector<Op> &ops);  // tuned configurations, no tuning events
     hipError_t launch_ops_one(const Op &op);      // a non-batch op

@@ -1032,6 +1032,7 @@ static void reset_cb(CommandBuffer *cb) {
         hipEventSynchronize(cb->done);
         // recorded anew after one submission: likely again
         cb->graph.recorded_per_frame = cb->submissions == 1;
+        cb->recorded_before = true;
     }
     cb->graph.reset();
     cb->graph.eager_runs = 0;
@@ -1057,19 +1058,21 @@ static void destroy_cb(CommandBuffer *cb) {
 // The next draw records of cb's recording, at least `bytes` long.
 static DrawRecords *next_records(CommandBuffer *cb, size_t bytes) {
     if (cb->records_used == cb->records.size()) cb->records.emplace_back();
-    DrawRecords &r = cb->records[cb->records_used];
-    if (r.cap < bytes) {  // (not in use: the recording before has finished)
+    DrawRecords &r = cb->records[cb->records_used];  // (not in use: the recording before has finished)
+    const size_t cap = cb->recorded_before ? bytes + bytes / 2 : bytes;
+    if (r.cap < bytes) {
         hipFree(r.dev);
-        hipHostFree(r.host);
-        r = DrawRecords();
-        const size_t cap = bytes + bytes / 2;
+        r.dev = nullptr;
+        r.cap = 0;
         if (hipMalloc((void **)&r.dev, cap) != hipSuccess) return nullptr;
-        if (hipHostMalloc((void **)&r.host, cap, hipHostMallocDefault) != hipSuccess) {
-            hipFree(r.dev);
-            r = DrawRecords();
-            return nullptr;
-        }
         r.cap = cap;
+    }
+    if (cb->recorded_before && r.host_cap < bytes) {
+        hipHostFree(r.host);
+        r.host = nullptr;
+        r.host_cap = 0;
+        if (hipHostMalloc((void **)&r.host, cap, hipHostMallocDefault) != hipSuccess) return nullptr;
+        r.host_cap = cap;
     }
     if (!cb->done && hipEventCreateWithFlags(&cb->done, hipEventDisableTiming) != hipSuccess) {
         cb->done = nullptr;
@@ -1131,7 +1134,7 @@ VKAPI_ATTR VkResult VKAPI_CALL vkEndCommandBuffer(VkCommandBuffer commandBuffer)
     CommandBuffer *cb = from<CommandBuffer>(commandBuffer);
     if (!cb->recording) return VK_ERROR_INITIALIZATION_FAILED;
     set_device(cb->device);
-    // each batch's draw records, copied to the device by the recording's first
+    // each batch's draw records, copied here or by the recording's first
     // submission; every submission reuses them
     for (Op &op : cb->ops) {
         if (op.kind != Op::Batch || op.draws.empty()) continue;
@@ -1142,8 +1145,10 @@ VKAPI_ATTR VkResult VKAPI_CALL vkEndCommandBuffer(VkCommandBuffer commandBuffer)
         const size_t nblk = ((size_t)op.frame.total_tris + KZ_BIN_BLOCK - 1) / KZ_BIN_BLOCK + 1;
         DrawRecords *r = next_records(cb, rec_bytes + (n + nblk) * sizeof(uint32_t));
         if (!r) return VK_ERROR_OUT_OF_DEVICE_MEMORY;
-        std::memcpy(r->host, op.draws.data(), rec_bytes);
-        uint32_t *begin = (uint32_t *)(r->host + rec_bytes);
+        std::vector<char> first(cb->recorded_before ? 0 : r->bytes);
+        char *host = cb->recorded_before ? r->host : first.data();
+        std::memcpy(host, op.draws.data(), rec_bytes);
+        uint32_t *begin = (uint32_t *)(host + rec_bytes);
         for (size_t i = 0; i < n; ++i) begin[i] = op.draws[i].tri_begin;
         uint32_t *block_draw = begin + n;
         for (size_t b = 0, d = 0; b < nblk; ++b) {
@@ -1151,7 +1156,10 @@ VKAPI_ATTR VkResult VKAPI_CALL vkEndCommandBuffer(VkCommandBuffer commandBuffer)
             while (d + 1 < n && op.draws[d + 1].tri_begin <= g) ++d;
             block_draw[b] = (uint32_t)d;
         }
-        cb->records_pending = true;
+        if (cb->recorded_before)
+            cb->records_pending = true;
+        else if (hipMemcpy(r->dev, host, r->bytes, hipMemcpyHostToDevice) != hipSuccess)
+            return VK_ERROR_DEVICE_LOST;
         op.d_draws = (KzDraw *)r->dev;
         op.d_draw_begin = (uint32_t *)(r->dev + rec_bytes);
         op.d_block_draw = op.d_draw_begin + n;

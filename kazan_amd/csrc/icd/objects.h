@@ -201,11 +201,13 @@ struct RecordState {
     bool batch_open = false;  // the last op is a batch that may take more draws
 };
 
-// A batch's draw records: in pinned memory as recorded, and on the device,
-// where the first submission after the recording copies them.
+// A batch's draw records on the device, and from a command buffer's second
+// recording on in pinned memory, from where the first submission after the
+// recording copies them (a first recording, often the only one, copies them
+// itself: pinning memory would cost it more).
 struct DrawRecords {
     char *host = nullptr, *dev = nullptr;
-    size_t cap = 0, bytes = 0;
+    size_t cap = 0, host_cap = 0, bytes = 0;
 };
 
 struct CommandBuffer : Dispatchable {
@@ -216,6 +218,7 @@ struct CommandBuffer : Dispatchable {
     std::vector<DrawRecords> records;
     size_t records_used = 0;
     bool records_pending = false;  // recorded, not copied to the device yet
+    bool recorded_before = false;
     hipEvent_t done = nullptr;     // after this recording's last submission
     uint32_t submissions = 0;      // of this recording
     GraphCache graph;  // the ops as a hipGraph, once captured

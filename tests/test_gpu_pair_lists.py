@@ -3,9 +3,11 @@ triangles, by their lanes when the chunk has at most two pairs a triangle,
 else 1,024 pairs at a time on workgroups of their own. Triangle counts at the
 edges of binning blocks and chunks, large triangles (hundreds of tiles each)
 alone, among small ones and after a chunk of small ones, and a list storage
-that ends within a chunk of large ones, against the oracle through the Vulkan
-C ABI at every tile size the tuner tries. The bar is the parity suite's:
-counts equal, coverage and depth bit-exact, colour within 1 LSB.
+that ends within a chunk of large ones; clipped triangles, whose pieces are
+entries of their own, at one and four samples and past the storage, against
+the oracle through the Vulkan C ABI at every tile size the tuner tries. The
+bar is the parity suite's: counts equal, coverage and depth bit-exact,
+colour within 1 LSB.
 """
 import numpy as np
 import pytest
@@ -61,4 +63,18 @@ def test_cut_within_large_triangles(driver, monkeypatch, oracle, form):
     monkeypatch.setenv("KAZAN_BINNING", "radix")
     monkeypatch.setenv("KAZAN_LIST_CAPACITY_LIMIT", "30000")
     st, _, _ = check_parity(Context(driver), oracle, _scene(6000, range(2000, 3500)), frames=2)
+    assert st["list_overflow"] >= 1
+
+
+@pytest.mark.parametrize("form", ["balanced", "plain"])
+def test_clip_pieces_with_radix_binning(driver, monkeypatch, oracle, form):
+    from kazan_amd.scenes.renderer import Context
+    monkeypatch.setenv("KAZAN_PIPELINE", form)
+    monkeypatch.setenv("KAZAN_BINNING", "radix")
+    ctx = Context(driver)
+    for s in (g.camera_inside(4000, 400, 256, 192), g.camera_inside(1000, 100, 128, 96, samples=4)):
+        for frames in (1, 4):
+            check_parity(ctx, oracle, s, frames=frames)
+    monkeypatch.setenv("KAZAN_LIST_CAPACITY_LIMIT", "3000")
+    st, _, _ = check_parity(Context(driver), oracle, g.camera_inside(600, 600, 256, 256), frames=2)
     assert st["list_overflow"] >= 1

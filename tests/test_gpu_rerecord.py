@@ -1,0 +1,38 @@
+"""A command buffer recorded anew for every frame, as a game does: its draw
+records' memory is kept over recordings (of more draws than before, and of
+fewer), each frame has the draws of its recording, and a recording that is
+submitted again after all is tuned and replayed as any other. The bar is the
+parity suite's: counts equal, depth bit-exact, colour within 1 LSB.
+"""
+import numpy as np
+import pytest
+
+from kazan_amd.scenes import generators as g
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(r, oracle, st, frames):
+    oc, od, _, ost = oracle.render(r.s)
+    assert st["fragments"] == frames * ost["fragments"]
+    c, d, _ = r.read_back()
+    np.testing.assert_array_equal(d.view(np.uint32), od.view(np.uint32))
+    assert np.abs(c.astype(np.int16) - oc.astype(np.int16)).max() <= 1
+
+
+@pytest.mark.parametrize("form", ["balanced", "plain"])
+def test_recorded_for_every_frame(driver, monkeypatch, oracle, form):
+    from kazan_amd.scenes.renderer import Context, SceneRenderer
+    monkeypatch.setenv("KAZAN_PIPELINE", form)
+    ctx = Context(driver)
+    s = g.zipf_draws(200, 20_000, 320, 180)
+    draws = s.draws
+    r = SceneRenderer(ctx, s)
+    cb = r.cb
+    for k in (2, 5, 60, 200, 3):
+        s.draws = draws[:k]
+        with monkeypatch.context() as m:
+            m.setattr(ctx, "command_buffer", lambda: cb)
+            r._record()
+        _check(r, oracle, r.render(1), 1)
+    _check(r, oracle, r.render(40), 40)
