@@ -673,8 +673,9 @@ int final_choice(const BatchTuning &t) {
 
 // Candidates, one HIP-event-timed trial per submission: every tile size
 // whose kernels fit (full grid, the plan with the cost model when there is
-// one); at the fastest size, a half grid and the plain raster (one workgroup
-// per tile, no plan); at the fastest of those, the plan without the model and
+// one); at the fastest size, the model's plan with its fragment weight times
+// 16 (without a model a half grid) and the plain raster (one workgroup per
+// tile, no plan); at the fastest of those, the plan without the model and
 // the plain raster of the next smaller tiles (the plain raster's neighbours
 // when it is the fastest); at the fastest planned one, splits of at most 4
 // sub-tiles and none (many small triangles are set up once per sub-tile they
@@ -722,7 +723,12 @@ hipError_t Engine::pick_config(Op &op, BatchConfig &cfg, bool &timed, bool tune)
         if (best >= 0) {
             const BatchConfig b = t.cand[best];
             if (t.phase == 0) {
-                t.cand.push_back({b.shift, 2u, b.model, true, 2u, 1u});
+                // (fragments weighted 16 times: where a frame has few tiles, of
+                // many fragments each, its splits are what a plan is for, and
+                // it has to be seen before the plain raster ends the search:
+                // 256 triangles in 64^2 83 us a frame, plain 89)
+                if (b.model) t.cand.push_back({b.shift, 1u, true, true, 2u, 16u});
+                else t.cand.push_back({b.shift, 2u, false, true, 2u, 1u});
                 t.cand.push_back({b.shift, 1u, false, false, 2u, 1u});
             } else if (t.phase == 1) {
                 // the plain raster has only its tiles to fill the chip with:
