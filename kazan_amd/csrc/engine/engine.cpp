@@ -629,8 +629,7 @@ hipError_t Engine::regrow(T *&p, uint64_t count) {
     return grow(p, count);
 }
 
-// Tuning candidates of a batch: every tile size whose kernels fit (full
-// grid) first; then, at the fastest tile size, a half and a quarter grid.
+// The untuned configuration of a batch.
 BatchConfig Engine::default_config(const Op &op) const {
     BatchConfig c;
     c.shift = op.tile_shift;

@@ -143,7 +143,7 @@ struct BatchTuning {
     BatchTuning &operator=(const BatchTuning &) = delete;
     ~BatchTuning();
     bool done = false;
-    int phase = 0;  // 0: tile sizes, 1: grid sizes, 2: plan and raster forms, 3: split depth, 4: fragment weight,
+    int phase = 0;  // 0: tile sizes, 1, 2: plan and raster forms, 3: split depth, 4: fragment weight,
                     // 5: every tile size x grid size again, 6: the three fastest twice more each
     std::vector<BatchConfig> cand;
     std::vector<float> ms;           // per candidate, -1 = not timed
