@@ -1311,6 +1311,7 @@ VKAPI_ATTR void VKAPI_CALL vkCmdBeginRenderPass(VkCommandBuffer commandBuffer, c
     st.render_area = bi->renderArea;
     st.subpass = 0;
     st.batch_open = false;
+    st.pass_draws = false;
     const VkRect2D &a = bi->renderArea;
     for (uint32_t i = 0; i < st.render_pass->attachments.size(); ++i) {
         const VkAttachmentDescription &ad = st.render_pass->attachments[i];
@@ -1356,9 +1357,11 @@ VKAPI_ATTR void VKAPI_CALL vkCmdEndRenderPass(VkCommandBuffer commandBuffer) {
         op.y0 = st.render_area.offset.y;
         op.w = std::min<uint32_t>(st.render_area.extent.width, dst->width - (uint32_t)op.x0);
         op.h = std::min<uint32_t>(st.render_area.extent.height, dst->height - (uint32_t)op.y0);
-        // A batch just before, whose raster writes every pixel of the source
-        // (its clear is folded in), resolves it as it writes it.
-        if (!cb->ops.empty() && cb->ops.back().kind == Op::Batch) {
+        // A batch of this render pass just before, whose raster writes every
+        // pixel of the source (its clear is folded in), resolves it as it
+        // writes it. (A batch of an earlier pass may sample or fetch from the
+        // image that this one resolves into: its raster must not write it.)
+        if (st.pass_draws && cb->ops.back().kind == Op::Batch) {
             Op &last = cb->ops.back();
             KzFrame &f = last.frame;
             if (last.variants->fixed.samples == 4 && (f.clear_mask & 1u) && f.color == src->address() && !f.resolve &&
@@ -1480,6 +1483,7 @@ static void record_draw(CommandBuffer *cb, uint32_t count, uint32_t instances, u
         cb->ops.push_back(std::move(op));
         batch = &cb->ops.back();
         st.batch_open = true;
+        st.pass_draws = true;
     }
     const uint32_t tris = count / 3;
     for (uint32_t inst = 0; inst < instances; ++inst) {

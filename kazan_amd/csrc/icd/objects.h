@@ -199,6 +199,7 @@ struct RecordState {
     VkRect2D render_area{};
     uint32_t subpass = 0;
     bool batch_open = false;  // the last op is a batch that may take more draws
+    bool pass_draws = false;  // the render pass has recorded a batch
 };
 
 // A batch's draw records on the device, and from a command buffer's second
