@@ -127,6 +127,7 @@ struct KzFrame {
     uint32_t *gather_list;    // (2 words each)
     uint32_t *super_state;    // [squares * KZ_SUPER_WORDS], zeroed by kz_bin_count
     unsigned long long *stats;  // KZ_STAT_* counters
+    uint32_t *need;             // KZ_NEED_* words in host memory
 
     // Load-balanced mode. A work item is a square sub-tile of a screen
     // tile: level L splits the tile into 4^L squares of side TS >> L (L = 0
@@ -319,6 +320,14 @@ enum {
 // workgroup's atomics; kz_stats_reduce folds them when the host waits.
 #define KZ_STAT_STRIPES 256
 
+// What outgrew its storage since the host last looked, in host memory that it
+// reads without waiting for the queue. Written only when something did.
+enum {
+    KZ_NEED_PAIRS = 0,  // the largest batch's (triangle, tile) pairs past the list capacity, or 0
+    KZ_NEED_SPLIT = 1,  // nonzero: the sub-tile lists (KZ_CTRL_SPLIT_MAX has the largest total)
+    KZ_NEED_WORDS = 2
+};
+
 // Per-triangle pixel bounding box (inclusive, clipped to the scissor),
 // packed as px0 | py0 << 16 | px1 << 32 | py1 << 48; ~0 = no pixels.
 #define KZ_RECT_EMPTY (~0ULL)
@@ -437,6 +446,14 @@ __device__ __forceinline__ uint32_t kz_wave_incl_scan(uint32_t v) {
     KZ_DPP_ADD(0x143, 0xC);  // row_bcast:31 into rows 2 and 3
 #undef KZ_DPP_ADD
     return v;
+}
+
+// A batch's `pairs` did not fit the lists (one thread of a batch calls it, and
+// the batches follow each other: nothing else writes the word meanwhile).
+__device__ __forceinline__ void kz_need_pairs(uint32_t *need, unsigned long long pairs) {
+    const uint32_t p = pairs < 0xFFFFFFFFull ? (uint32_t)pairs : 0xFFFFFFFFu;
+    if (p > __hip_atomic_load(&need[KZ_NEED_PAIRS], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))
+        __hip_atomic_store(&need[KZ_NEED_PAIRS], p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Tile t's list: its offset and count. A tile flagged by a cut (binning

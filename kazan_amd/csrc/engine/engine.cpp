@@ -75,6 +75,7 @@ Engine::~Engine() {
     hipFree(cost_model_d_);
     hipFree(stats_d_);
     if (stats_h_) hipHostFree(stats_h_);
+    if (need_h_) hipHostFree(need_h_);
     for (hipEvent_t e : event_pool_) hipEventDestroy(e);
     if (ev_start_) hipEventDestroy(ev_start_);
     if (ev_end_) hipEventDestroy(ev_end_);
@@ -87,11 +88,13 @@ bool Engine::init(int hip_device, std::string &err) {
     if ((e = hipSetDevice(device_)) != hipSuccess || (e = hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking)) ||
         (e = hipEventCreate(&ev_start_)) || (e = hipEventCreate(&ev_end_)) ||
         (e = hipMalloc((void **)&stats_d_, kStatWords * sizeof(unsigned long long))) ||
-        (e = hipHostMalloc((void **)&stats_h_, KZ_STAT_COUNT * sizeof(unsigned long long), hipHostMallocDefault))) {
+        (e = hipHostMalloc((void **)&stats_h_, KZ_STAT_COUNT * sizeof(unsigned long long), hipHostMallocDefault)) ||
+        (e = hipHostMalloc((void **)&need_h_, KZ_NEED_WORDS * sizeof(uint32_t), hipHostMallocCoherent))) {
         err = hipGetErrorString(e);
         return false;
     }
     std::memset(stats_h_, 0, KZ_STAT_COUNT * sizeof(unsigned long long));
+    std::memset(need_h_, 0, KZ_NEED_WORDS * sizeof(uint32_t));
     // KAZAN_LIST_CAPACITY_LIMIT caps the per-tile list storage (entries);
     // tiles whose lists do not fit render through the in-order scan path
     if (const char *e = std::getenv("KAZAN_LIST_CAPACITY_LIMIT")) list_limit_ = std::strtoull(e, nullptr, 10);
@@ -431,6 +434,7 @@ hipError_t Engine::run_batch(const Op &op, const BatchConfig &cfg) {
     f.tri_draw = f.ndraws > 1 ? tri_draw_ : nullptr;
     f.tri_rec = setup_records_ ? tri_rec_ : nullptr;
     f.stats = stats_d_;
+    f.need = need_h_;
     f.tile_shift = shift;
     if (persistent) {
         f.balanced = 1;
@@ -543,7 +547,8 @@ hipError_t Engine::run_batch(const Op &op, const BatchConfig &cfg) {
         KZ_TRY(acc ? kz_launch_bin_hist_acc(stream_, f) : kz_launch_bin_hist(stream_, f));
         KZ_TRY(mark(KS_BIN_HIST, true));
         KZ_TRY(mark(KS_BIN_SCAN, false));
-        KZ_TRY(kz_launch_scan(stream_, tile_counts_, tile_offsets_, tile_cursor_, ntiles, list_capacity_, stats_d_));
+        KZ_TRY(kz_launch_scan(stream_, tile_counts_, tile_offsets_, tile_cursor_, ntiles, list_capacity_, stats_d_,
+                              need_h_));
         KZ_TRY(mark(KS_BIN_SCAN, true));
         KZ_TRY(mark(KS_BIN_SCATTER, false));
         KZ_TRY(kz_launch_bin_scatter(stream_, f));
@@ -976,6 +981,11 @@ hipError_t Engine::end_submit(hipEvent_t fence_event) {
     return hipSuccess;
 }
 
+bool Engine::outgrown() const {
+    const volatile uint32_t *need = need_h_;
+    return need[KZ_NEED_PAIRS] || need[KZ_NEED_SPLIT];
+}
+
 void Engine::collect_stats() {
     if (!submit_open_) return;
     // the striped counters are folded and read once per wait, not once per
@@ -1006,10 +1016,14 @@ void Engine::collect_stats() {
     timing_events_.clear();
     events_used_ = 0;
     submit_open_ = false;
-    // A submission whose lists overflowed rendered correctly through the
-    // in-order scan fallback; size the lists for the next one.
-    if (last_.counters[KZ_STAT_LIST_OVERFLOW]) {
-        uint64_t need = last_.counters[KZ_STAT_LIST_ENTRIES] + last_.counters[KZ_STAT_LIST_ENTRIES] / 4;
+    // A batch whose lists overflowed rendered correctly through the in-order
+    // scan fallback; size the lists for the largest such batch (the counters
+    // hold the pairs of every batch since the last collection).
+    const uint32_t pairs = need_h_[KZ_NEED_PAIRS];
+    const bool split = need_h_[KZ_NEED_SPLIT] != 0;
+    std::memset(need_h_, 0, KZ_NEED_WORDS * sizeof(uint32_t));
+    if (pairs) {
+        uint64_t need = (uint64_t)pairs + pairs / 4;
         if (list_limit_) need = std::min<uint64_t>(need, list_limit_);
         if (need > list_capacity_ && need < 0xFFFFFFF0ull) {
             hipStreamSynchronize(stream_);
@@ -1018,7 +1032,7 @@ void Engine::collect_stats() {
     }
     // Likewise for sub-tile lists (their overflow fallback filters the
     // parent tile's list): the device keeps the largest batch total.
-    if (ctrl_ && last_.counters[KZ_STAT_SPLIT_ENTRIES] > split_capacity_) {
+    if (ctrl_ && split) {
         uint32_t mx = 0;
         if (hipMemcpy(&mx, ctrl_ + KZ_CTRL_SPLIT_MAX, sizeof mx, hipMemcpyDeviceToHost) == hipSuccess &&
             mx > split_capacity_) {

@@ -10,6 +10,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <atomic>
 #include <cstdint>
 #include <memory>
 #include <string>
@@ -248,6 +249,9 @@ class Engine {
     const BatchConfig &last_tuned() const { return last_tuned_; }
     // After the submission's work is complete: read stats, adapt capacity.
     void collect_stats();
+    // whether a batch outgrew its list storage (it was drawn by a slower
+    // path); collect_stats makes room
+    bool outgrown() const;
     const SubmitStats &last_stats() const { return last_; }
 
     uint32_t list_capacity() const { return list_capacity_; }
@@ -316,7 +320,7 @@ class Engine {
     // (KAZAN_GRID_DIVISOR, KAZAN_SPLIT_LEVEL)
     uint32_t default_grid_div_ = 1, default_max_level_ = 2;
     uint64_t generation_ = 1;  // bumped whenever captured graphs go stale
-    uint64_t submissions_ = 0;
+    std::atomic<uint64_t> submissions_{0};  // (read by threads that wait on fences)
     uint32_t graph_launches_ = 0, graph_captures_ = 0;
     BatchConfig last_tuned_{0, 0, false, false, 0, 0};
     uint64_t list_limit_ = 0;
@@ -379,6 +383,7 @@ class Engine {
     uint32_t *tri_rec_ = nullptr;
     uint64_t cap_rec_words_ = 0;
     unsigned long long *stats_d_ = nullptr, *stats_h_ = nullptr;
+    uint32_t *need_h_ = nullptr;  // KZ_NEED_* words, pinned
     uint32_t cap_tiles_ = 0, cap_tris_ = 0, list_capacity_ = 0;
     uint32_t pending_batches_ = 0, pending_launches_ = 0;
     bool submit_open_ = false;

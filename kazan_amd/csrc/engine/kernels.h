@@ -15,7 +15,7 @@ hipError_t kz_launch_fill_rect_u32(hipStream_t st, uint32_t *dst, uint32_t width
 // beyond `capacity` (sort binning; radix binning's last pass writes the
 // offsets itself).
 hipError_t kz_launch_scan(hipStream_t st, uint32_t *counts, uint32_t *offsets, uint32_t *cursor, uint32_t n,
-                          uint32_t capacity, unsigned long long *stats);
+                          uint32_t capacity, unsigned long long *stats, uint32_t *need);
 // Radix binning, after kz_bin_count and kz_pair_scan (the pipeline's) wrote
 // f.tri_rect and the pair offsets.
 struct KzRadixScratch {

@@ -158,15 +158,19 @@ __global__ void kz_fill_rect_u32(uint32_t *dst, uint32_t width, int32_t x0, int3
 
 // Exclusive prefix sum of counts[0, n) into offsets and cursor. With stats,
 // adds the total to the list-entry statistic and, when `capacity` is
-// exceeded, counts an overflow.
+// exceeded, counts an overflow and tells the host (need).
 __global__ __launch_bounds__(kScanThreads) void kz_scan(uint32_t *counts, uint32_t *offsets, uint32_t *cursor,
-                                                        uint32_t n, uint32_t capacity, unsigned long long *stats) {
+                                                        uint32_t n, uint32_t capacity, unsigned long long *stats,
+                                                        uint32_t *need) {
     __shared__ uint32_t s_wave[kScanThreads / 64];
     __shared__ uint32_t s_carry;
     const uint32_t total = block_exclusive_scan(counts, offsets, cursor, n, s_wave, &s_carry);
     if (threadIdx.x == 0 && stats) {
         atomicAdd(&stats[KZ_STAT_LIST_ENTRIES], (unsigned long long)total);
-        if (total > capacity) atomicAdd(&stats[KZ_STAT_LIST_OVERFLOW], 1ull);
+        if (total > capacity) {
+            atomicAdd(&stats[KZ_STAT_LIST_OVERFLOW], 1ull);
+            kz_need_pairs(need, total);
+        }
     }
 }
 
@@ -1348,7 +1352,10 @@ __global__ __launch_bounds__(kGatherThreads) void kz_gather_lists(KzFrame f, uin
         f.bin_ctrl[KZ_BIN_PIECES] = 0;  // for the next batch
         f.bin_ctrl[KZ_BIN_CLIPPED] = 0;
         atomicAdd(&f.stats[KZ_STAT_LIST_ENTRIES], all);
-        if (all > cap) atomicAdd(&f.stats[KZ_STAT_LIST_OVERFLOW], 1ull);
+        if (all > cap) {
+            atomicAdd(&f.stats[KZ_STAT_LIST_OVERFLOW], 1ull);
+            kz_need_pairs(f.need, all);
+        }
     }
     GatherAcc acc = {};
     const uint32_t want = tile ? (1u << col) | (0x10000u << row) : 0u;
@@ -1791,6 +1798,8 @@ __global__ __launch_bounds__(kSplitThreads) void kz_split_offsets(KzFrame f) {
     if (lane == 63 && total) {
         base = atomicAdd(&f.ctrl[KZ_CTRL_SPLIT_CURSOR], total);
         atomicMax(&f.ctrl[KZ_CTRL_SPLIT_MAX], base + total);
+        if (base + total > f.split_capacity)
+            __hip_atomic_store(&f.need[KZ_NEED_SPLIT], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         atomicAdd(&kz_stats_stripe_of(f)[KZ_STAT_SPLIT_ENTRIES], (unsigned long long)total);
     }
     uint32_t run = readlane(base, 63) + x - v;
@@ -2445,8 +2454,8 @@ hipError_t kz_launch_fill_rect_u32(hipStream_t st, uint32_t *dst, uint32_t width
 }
 
 hipError_t kz_launch_scan(hipStream_t st, uint32_t *counts, uint32_t *offsets, uint32_t *cursor, uint32_t n,
-                          uint32_t capacity, unsigned long long *stats) {
-    kz_scan<<<1, kScanThreads, 0, st>>>(counts, offsets, cursor, n, capacity, stats);
+                          uint32_t capacity, unsigned long long *stats, uint32_t *need) {
+    kz_scan<<<1, kScanThreads, 0, st>>>(counts, offsets, cursor, n, capacity, stats, need);
     return hipGetLastError();
 }
 

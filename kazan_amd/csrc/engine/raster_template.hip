@@ -1575,7 +1575,10 @@ extern "C" __global__ __launch_bounds__(KZ_PAIR_SCAN_THREADS) void kz_pair_scan(
         f.bin_ctrl[KZ_BIN_OVER] = over ? 1u : 0u;
         f.bin_ctrl[KZ_BIN_EXTRA] = ecarry;
         atomicAdd(&f.stats[KZ_STAT_LIST_ENTRIES], carry);
-        if (over) atomicAdd(&f.stats[KZ_STAT_LIST_OVERFLOW], 1ull);
+        if (over) {
+            atomicAdd(&f.stats[KZ_STAT_LIST_OVERFLOW], 1ull);
+            kz_need_pairs(f.need, carry);
+        }
     }
 }
 

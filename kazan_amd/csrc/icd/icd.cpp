@@ -1672,12 +1672,13 @@ VKAPI_ATTR VkResult VKAPI_CALL vkWaitForFences(VkDevice device, uint32_t n, cons
         std::this_thread::sleep_for(std::chrono::microseconds(20));
     }
     // The statistics fold waits for the whole queue: only when that costs
-    // nothing more than the wait itself, or (list capacities grow from the
-    // counters it reads) after a number of waits with later frames in flight.
+    // nothing more than the wait itself, when a batch outgrew its lists (the
+    // fold makes room for the next frames), or after a number of waits with
+    // later frames in flight.
     uint64_t last = 0;
     for (uint32_t i = 0; i < n && waitAll; ++i) last = std::max(last, from<Fence>(fences[i])->submission);
     if (last == d->engine->submissions() || hipStreamQuery(d->engine->stream()) == hipSuccess ||
-        (waitAll && ++d->waits_behind >= 16)) {
+        (waitAll && (d->engine->outgrown() || ++d->waits_behind >= 16))) {
         d->waits_behind = 0;
         d->engine->collect_stats();
     }

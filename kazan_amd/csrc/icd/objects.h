@@ -10,6 +10,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <atomic>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -50,7 +51,7 @@ struct Device : Dispatchable {
     PhysicalDevice *physical = nullptr;
     std::unique_ptr<Queue> queue;
     std::unique_ptr<Engine> engine;
-    uint32_t waits_behind = 0;  // fence waits since the statistics were read, frames after them in flight
+    std::atomic<uint32_t> waits_behind{0};  // fence waits since the statistics were read, frames after them in flight
 };
 
 struct DeviceMemory {
