@@ -126,9 +126,16 @@ KAZAN_EXPORT int kazan_compile_pipeline_spirv(const KazanPipelineDesc *desc, uin
 /* A GLCompute entry point; storage and uniform buffers take kernel slots in
  * (set, binding) order. what: 0 = generated kernel body, 1 = full kernel
  * source, 2 = compile to a code object and report its size, whether the
- * cache held it and the workgroup size */
+ * cache held it, the workgroup size and the workgroups that a block of its
+ * launches may take (per_block) */
 KAZAN_EXPORT int kazan_compile_compute_spirv(const uint32_t *words, size_t nwords, const char *entry, uint32_t what,
                                              char *out, size_t cap, size_t *out_len);
+
+/* The launch vkCmdDispatch makes of groups[] workgroups of local[] invocations
+ * whose kernel takes up to per_block of them a block: the blocks and their
+ * threads. Returns the workgroups (along x) of a block. */
+KAZAN_EXPORT int kazan_compute_launch(const uint32_t local[3], uint32_t per_block, const uint32_t groups[3],
+                                      uint32_t grid[3], uint32_t block[3]);
 
 #ifdef __cplusplus
 }

@@ -22,6 +22,7 @@
 
 #include "kazan/kazan_icd.h"
 #include "kernels.h"
+#include "../shader/backend_hip.h"
 #include "objects.h"
 
 namespace kz {
@@ -1240,23 +1241,16 @@ static void record_dispatch(CommandBuffer *cb, uint32_t bx, uint32_t by, uint32_
     Op op;
     op.kind = Op::Dispatch;
     op.cs_kernel = p->cs_kernel;
-    op.groups[0] = x;
-    op.groups[1] = y;
-    op.groups[2] = z;
-    for (int k = 0; k < 3; ++k) op.block[k] = p->local_size[k];
+    const ComputeLaunch c = compute_launch(p->local_size, p->cs_per_block, x, y, z);
+    for (int k = 0; k < 3; ++k) {
+        op.groups[k] = c.grid[k];
+        op.block[k] = c.block[k];
+    }
     KzComputeFrame &f = op.cframe;
     f.groups[0] = x;
     f.groups[1] = y;
     f.groups[2] = z;
-    f.per_block = 1;
-    if (p->cs_per_block > 1) {  // its kernel takes linear blocks
-        // several workgroups a block, unless the last block of a row would
-        // leave more than a fifth of the row's threads without one
-        f.per_block = x >= 4 * p->cs_per_block ? p->cs_per_block : 1u;
-        op.block[0] *= op.block[1] * op.block[2] * f.per_block;
-        op.block[1] = op.block[2] = 1;
-        op.groups[0] = (x + f.per_block - 1) / f.per_block;
-    }
+    f.per_block = c.per_block;
     f.base[0] = bx;
     f.base[1] = by;
     f.base[2] = bz;

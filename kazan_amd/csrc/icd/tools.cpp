@@ -167,8 +167,19 @@ extern "C" int kazan_compile_compute_spirv(const uint32_t *words, size_t nwords,
     if (!kz::compile_compute_code(source, true, code, log, &hit)) return put(log, out, cap, out_len, -1);
     return put("code_object_bytes=" + std::to_string(code.size()) + " cache_hit=" + (hit ? "1" : "0") +
                    " local_size=" + std::to_string(m.local_size[0]) + "x" + std::to_string(m.local_size[1]) + "x" +
-                   std::to_string(m.local_size[2]),
+                   std::to_string(m.local_size[2]) + " per_block=" + std::to_string(per_block),
                out, cap, out_len, 0);
+}
+
+extern "C" int kazan_compute_launch(const uint32_t local[3], uint32_t per_block, const uint32_t groups[3],
+                                    uint32_t grid[3], uint32_t block[3]) {
+    if (!local || !groups || !grid || !block || per_block == 0) return -1;
+    const kz::ComputeLaunch c = kz::compute_launch(local, per_block, groups[0], groups[1], groups[2]);
+    for (int k = 0; k < 3; ++k) {
+        grid[k] = c.grid[k];
+        block[k] = c.block[k];
+    }
+    return (int)c.per_block;
 }
 
 // --- the learned tile-cost model's kernels, outside a Vulkan device ------

@@ -770,6 +770,21 @@ namespace {
 constexpr uint64_t kComputeBlock = 512;
 }  // namespace
 
+ComputeLaunch compute_launch(const uint32_t local[3], uint32_t most, uint32_t x, uint32_t y, uint32_t z) {
+    ComputeLaunch c{{x, y, z}, {local[0], local[1], local[2]}, 1u};
+    // several workgroups a block, unless the last block of a row would leave
+    // more than a fifth of the row's threads without one, or the row (all of
+    // a workgroup's invocations along x) has more threads than a launch takes
+    const uint64_t n = (uint64_t)local[0] * local[1] * local[2], blocks = ((uint64_t)x + most - 1) / most;
+    if (most > 1 && x >= 4ull * most && blocks * most * n <= 0xFFFFFFFFull) {
+        c.per_block = most;
+        c.grid[0] = (uint32_t)blocks;
+        c.block[0] = (uint32_t)(n * most);
+        c.block[1] = c.block[2] = 1;
+    }
+    return c;
+}
+
 bool generate_compute_source(const ir::Module &cs, const PipelineCodegenInput &in, std::string &out,
                              uint32_t &per_block, std::string &err) {
     const uint32_t lx = cs.local_size[0], ly = cs.local_size[1], lz = cs.local_size[2];
@@ -802,7 +817,13 @@ bool generate_compute_source(const ir::Module &cs, const PipelineCodegenInput &i
         os << "    const uint32_t li = threadIdx.x % " << n << "u;\n";
         os << "    const uint32_t gx = blockIdx.x * f.per_block + threadIdx.x / " << n << "u;\n";
         os << "    if (gx >= f.groups[0]) return;\n";
-        os << "    const uint32_t lid[3] = {li % L[0], li / L[0] % L[1], li / (L[0] * L[1])};\n";
+        if (ly * lz == 1) {
+            os << "    const uint32_t lid[3] = {li, 0u, 0u};\n";
+        } else {  // (a workgroup alone has its block's shape; threadIdx.x < L[0] <= n then)
+            os << "    const bool one = f.per_block == 1u;\n";
+            os << "    const uint32_t lid[3] = {one ? threadIdx.x : li % L[0], one ? threadIdx.y : li / L[0] % L[1],\n";
+            os << "                             one ? threadIdx.z : li / (L[0] * L[1])};\n";
+        }
     } else {
         os << "    const uint32_t gx = blockIdx.x;\n";
         os << "    const uint32_t lid[3] = {threadIdx.x, threadIdx.y, threadIdx.z};\n";

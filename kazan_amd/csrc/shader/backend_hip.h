@@ -52,12 +52,20 @@ struct PipelineCodegenOutput {
 bool generate_pipeline_source(const PipelineCodegenInput &in, PipelineCodegenOutput &out, std::string &err);
 
 // A compute pipeline's source: the shader as device function kz_cs_main,
-// its workgroup memory, and the kernel kz_compute(KzComputeFrame) that runs
-// one workgroup per dispatched group (the module's local size as its block).
-// Uses in.ubo_slot and in.ssbo_slot for the descriptor bindings.
-// per_block: the workgroups along x that a block of the launch may take.
+// its workgroup memory, and the kernel kz_compute(KzComputeFrame), launched as
+// compute_launch says. Uses in.ubo_slot and in.ssbo_slot for the descriptor
+// bindings. per_block: the workgroups along x that a block of the launch may
+// take.
 bool generate_compute_source(const ir::Module &cs, const PipelineCodegenInput &in, std::string &out,
-                             uint32_t &per_block,
-                             std::string &err);
+                             uint32_t &per_block, std::string &err);
+
+// The launch of a dispatch of x * y * z workgroups of `local` invocations:
+// one workgroup a block, in its own shape, or (per_block > 1, KzComputeFrame's
+// too) up to `most` consecutive ones along x in a linear block.
+struct ComputeLaunch {
+    uint32_t grid[3], block[3];
+    uint32_t per_block;
+};
+ComputeLaunch compute_launch(const uint32_t local[3], uint32_t most, uint32_t x, uint32_t y, uint32_t z);
 
 }  // namespace kz
