@@ -126,8 +126,8 @@ KAZAN_EXPORT int kazan_compile_pipeline_spirv(const KazanPipelineDesc *desc, uin
 /* A GLCompute entry point; storage and uniform buffers take kernel slots in
  * (set, binding) order. what: 0 = generated kernel body, 1 = full kernel
  * source, 2 = compile to a code object and report its size, whether the
- * cache held it, the workgroup size and the workgroups that a block of its
- * launches may take (per_block) */
+ * cache held it, the workgroup size, the workgroups that a block of its
+ * launches may take (per_block), vgprs and scratch (bytes per lane) */
 KAZAN_EXPORT int kazan_compile_compute_spirv(const uint32_t *words, size_t nwords, const char *entry, uint32_t what,
                                              char *out, size_t cap, size_t *out_len);
 

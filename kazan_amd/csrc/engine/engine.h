@@ -78,6 +78,9 @@ bool kernel_resources(const std::vector<char> &elf, const char *kernel, KernelRe
 std::string compute_full_source(const std::string &compute_source);
 bool compile_compute_code(const std::string &compute_source, bool optimize, std::vector<char> &code, std::string &log,
                           bool *cache_hit);
+// The workgroups (up to `most`, of n invocations) a block of a kernel with
+// these resources takes: 0 when its registers are at the limit of such blocks.
+uint32_t compute_per_block(const KernelResources &r, uint32_t n, uint32_t most);
 // Loads the code object on the current device.
 bool load_pipeline_kernels(const std::vector<char> &code, PipelineKernels &out, std::string &err);
 

@@ -338,6 +338,25 @@ bool compile_compute_code(const std::string &compute_source, bool optimize, std:
     return compile_cached(compute_full_source(compute_source), optimize ? "-O3" : "-O0", code, log, cache_hit, true);
 }
 
+// A block of 512 threads leaves a thread 256 registers at most, where a wave
+// that is a block of its own may have 512: at the limit the kernel is compiled
+// for workgroups alone. Below it a block takes no more workgroups than leaves
+// the waves resident that its registers allow (at 3 waves per SIMD one block
+// of 8 waves, or three of 4). Shaders in workgroups of 64 that read and write
+// 268 MB each, 48, 100 and 200 values per invocation (152 registers, 320, and
+// 512 with some scratch): 117, 196 and 435 us in blocks of 8 workgroups, 109,
+// 109 and 214 as chosen here (4, 1 and 1).
+uint32_t compute_per_block(const KernelResources &r, uint32_t n, uint32_t most) {
+    if (most > 1 && r.vgprs >= 256u) return 0;
+    const uint32_t slots = 4u * std::min(512u / std::max(r.vgprs, 8u), 8u);  // waves of a CU
+    auto resident = [&](uint32_t k) {
+        const uint32_t waves = (n * k + 63u) / 64u;
+        return slots / waves * (n * k);
+    };
+    while (most > 1 && resident(most) < resident(1)) most /= 2;
+    return most;
+}
+
 bool load_pipeline_kernels(const std::vector<char> &code, PipelineKernels &out, std::string &err) {
     hipError_t e = hipModuleLoadData(&out.module, code.data());
     if (e != hipSuccess) {

@@ -211,6 +211,24 @@ bool create_graphics_pipeline(Device *dev, const VkGraphicsPipelineCreateInfo *c
 // vkCreateComputePipelines: reference ComputePipeline::create
 // (vulkan-driver/src/pipeline.rs:122-154: the one compute stage, the
 // layout, the optimisation mode), continued here to a HIP kernel.
+bool compile_compute(const ir::Module &cs, const PipelineCodegenInput &in, bool optimize, std::string &source,
+                     std::vector<char> &code, uint32_t &per_block, bool *cache_hit, std::string &err) {
+    for (const bool several : {true, false}) {
+        std::string log;
+        source.clear();
+        if (!generate_compute_source(cs, in, several, source, per_block, err)) return false;
+        if (!compile_compute_code(source, optimize, code, log, cache_hit)) {
+            err = "kernel compilation failed:\n" + log;
+            return false;
+        }
+        KernelResources r;
+        if (per_block == 1 || !kernel_resources(code, "kz_compute", r)) break;
+        per_block = compute_per_block(r, cs.local_size[0] * cs.local_size[1] * cs.local_size[2], per_block);
+        if (per_block) break;
+    }
+    return true;
+}
+
 bool create_compute_pipeline(Device *dev, const VkComputePipelineCreateInfo *ci, Pipeline **out, std::string &err) {
     (void)dev;
     const VkPipelineShaderStageCreateInfo &st = ci->stage;
@@ -233,13 +251,8 @@ bool create_compute_pipeline(Device *dev, const VkComputePipelineCreateInfo *ci,
     cg.ubo_slot = p->ubo_slot;
     cg.ssbo_slot = p->ssbo_slot;
     std::string source;
-    if (!generate_compute_source(cmod, cg, source, p->cs_per_block, err)) return false;
     std::vector<char> code;
-    std::string log;
-    if (!compile_compute_code(source, (ci->flags & 0x1u) == 0, code, log, nullptr)) {
-        err = "kernel compilation failed:\n" + log;
-        return false;
-    }
+    if (!compile_compute(cmod, cg, (ci->flags & 0x1u) == 0, source, code, p->cs_per_block, nullptr, err)) return false;
     hipError_t e = hipModuleLoadData(&p->cs_module, code.data());
     if (e == hipSuccess) e = hipModuleGetFunction(&p->cs_kernel, p->cs_module, "kz_compute");
     if (e != hipSuccess) {

@@ -15,6 +15,11 @@
 #include "../shader/spirv_reader.h"
 #include "../shader/translate.h"
 
+namespace kz {
+bool compile_compute(const ir::Module &cs, const PipelineCodegenInput &in, bool optimize, std::string &source,
+                     std::vector<char> &code, uint32_t &per_block, bool *cache_hit, std::string &err);
+}
+
 namespace {
 
 int put(const std::string &s, char *out, size_t cap, size_t *out_len, int rc) {
@@ -158,16 +163,19 @@ extern "C" int kazan_compile_compute_spirv(const uint32_t *words, size_t nwords,
     for (size_t i = 0; i < ubos.size() && i < KZ_MAX_UBOS; ++i) cg.ubo_slot[ubos[i]] = (uint32_t)i;
     std::string source;
     uint32_t per_block = 1;
-    if (!kz::generate_compute_source(m, cg, source, per_block, err)) return put(err, out, cap, out_len, -1);
-    if (what == 0) return put(source, out, cap, out_len, 0);
-    if (what == 1) return put(kz::compute_full_source(source), out, cap, out_len, 0);
+    if (what < 2) {
+        if (!kz::generate_compute_source(m, cg, true, source, per_block, err)) return put(err, out, cap, out_len, -1);
+        return put(what == 0 ? source : kz::compute_full_source(source), out, cap, out_len, 0);
+    }
     std::vector<char> code;
-    std::string log;
     bool hit = false;
-    if (!kz::compile_compute_code(source, true, code, log, &hit)) return put(log, out, cap, out_len, -1);
+    if (!kz::compile_compute(m, cg, true, source, code, per_block, &hit, err)) return put(err, out, cap, out_len, -1);
+    kz::KernelResources r;
+    kz::kernel_resources(code, "kz_compute", r);
     return put("code_object_bytes=" + std::to_string(code.size()) + " cache_hit=" + (hit ? "1" : "0") +
                    " local_size=" + std::to_string(m.local_size[0]) + "x" + std::to_string(m.local_size[1]) + "x" +
-                   std::to_string(m.local_size[2]) + " per_block=" + std::to_string(per_block),
+                   std::to_string(m.local_size[2]) + " per_block=" + std::to_string(per_block) +
+                   " vgprs=" + std::to_string(r.vgprs) + " scratch=" + std::to_string(r.scratch),
                out, cap, out_len, 0);
 }
 

@@ -785,7 +785,7 @@ ComputeLaunch compute_launch(const uint32_t local[3], uint32_t most, uint32_t x,
     return c;
 }
 
-bool generate_compute_source(const ir::Module &cs, const PipelineCodegenInput &in, std::string &out,
+bool generate_compute_source(const ir::Module &cs, const PipelineCodegenInput &in, bool several, std::string &out,
                              uint32_t &per_block, std::string &err) {
     const uint32_t lx = cs.local_size[0], ly = cs.local_size[1], lz = cs.local_size[2];
     const uint64_t n = (uint64_t)lx * ly * lz;
@@ -809,7 +809,7 @@ bool generate_compute_source(const ir::Module &cs, const PipelineCodegenInput &i
     // one-wave workgroups is bound by starting its blocks, 16.8 M saxpy
     // elements in workgroups of 64 took 62 us, in blocks of four of them 47, of
     // eight 44.5.
-    const bool alone = !cs.workgroup_variables.empty() || g.os.str().find("__syncthreads") != std::string::npos;
+    const bool alone = !several || !cs.workgroup_variables.empty() || g.os.str().find("__syncthreads") != std::string::npos;
     per_block = alone ? 1u : (uint32_t)std::max<uint64_t>(1, kComputeBlock / n);
     os << "extern \"C\" __global__ __launch_bounds__(" << n * per_block << ") void kz_compute(KzComputeFrame f) {\n";
     os << "    const uint32_t L[3] = {" << lx << "u, " << ly << "u, " << lz << "u};\n";

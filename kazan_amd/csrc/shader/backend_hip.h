@@ -55,8 +55,8 @@ bool generate_pipeline_source(const PipelineCodegenInput &in, PipelineCodegenOut
 // its workgroup memory, and the kernel kz_compute(KzComputeFrame), launched as
 // compute_launch says. Uses in.ubo_slot and in.ssbo_slot for the descriptor
 // bindings. per_block: the workgroups along x that a block of the launch may
-// take.
-bool generate_compute_source(const ir::Module &cs, const PipelineCodegenInput &in, std::string &out,
+// take, 1 unless `several`.
+bool generate_compute_source(const ir::Module &cs, const PipelineCodegenInput &in, bool several, std::string &out,
                              uint32_t &per_block, std::string &err);
 
 // The launch of a dispatch of x * y * z workgroups of `local` invocations:

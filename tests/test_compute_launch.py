@@ -1,9 +1,17 @@
 """The launch of a dispatch (kazan_compute_launch, what vkCmdDispatch records):
 every workgroup is in exactly one block, and no dimension has more threads than
-a launch takes (2^32 - 1) where the workgroups' own shape has fewer."""
+a launch takes (2^32 - 1) where the workgroups' own shape has fewer. And the
+workgroups a block takes of a shader that needs many registers: no more than
+the waves its registers leave resident, and one where blocks of several would
+make it spill."""
 import ctypes
 
+import numpy as np
 import pytest
+
+from kazan_amd import vk
+from kazan_amd.scenes import compute_shaders as cs
+from kazan_amd.scenes import spirv as sp
 
 U3 = ctypes.c_uint32 * 3
 MOST_THREADS = 2**32 - 1
@@ -31,3 +39,46 @@ def test_blocks_cover_the_groups(driver, local, x):
     # several a block wherever the rule allows it
     fits = x >= 4 * most and -(-x // most) * most * n <= MOST_THREADS
     assert per == (most if fits else 1)
+
+
+def held_values_shader(held):
+    """o[g + n i] = v[g + n i] * (v[g] + v[g + n] + ...), i < held, n a push
+    constant: an invocation holds all its values until its first store."""
+
+    def body(m, builtin):
+        u, fl = m.t_int(False), m.t_float()
+        gid = builtin(sp.BuiltInGlobalInvocationId, "g")
+        v, o = cs._ssbo(m, fl, 4, 0, "v"), cs._ssbo(m, fl, 4, 1, "o")
+        pc = cs._push_block(m, [u])
+        f = sp.Function(m)
+        g = cs._gid_x(f, m, gid)
+        n = f.load(u, f.access_chain(m.t_ptr(sp.StoragePushConstant, u), pc, m.c_int(0)))
+        at = [f.binop(sp.OpIAdd, u, g, f.binop(sp.OpIMul, u, n, m.c_int(i, signed=False))) for i in range(held)]
+        x = [f.load(fl, cs._elem(f, m, v, fl, a)) for a in at]
+        s = x[0]
+        for y in x[1:]:
+            s = f.fadd(fl, s, y)
+        for a, y in zip(at, x):
+            f.store(cs._elem(f, m, o, fl, a), f.fmul(fl, y, s))
+        f.ret()
+        return f
+
+    return cs._compute_module((64, 1, 1), body).to_bytes()
+
+
+@pytest.mark.parametrize("held", [4, 48, 100])
+def test_block_of_a_shader_with_many_registers(driver, tmp_path, monkeypatch, held):
+    monkeypatch.setenv("KAZAN_PIPELINE_CACHE", str(tmp_path))
+    w = np.frombuffer(held_values_shader(held), np.uint32).copy()
+    rc, msg = vk.tool_call(driver, "kazan_compile_compute_spirv", w.ctypes.data_as(ctypes.c_void_p),
+                           ctypes.c_size_t(w.size), b"main", ctypes.c_uint32(2))
+    assert rc == 0, msg
+    kv = {k: v for k, v in (t.split("=") for t in msg.split())}
+    vgprs, per = int(kv["vgprs"]), int(kv["per_block"])
+    assert int(kv["scratch"]) == 0  # (as a workgroup alone has it)
+    waves = min(512 // vgprs, 8) * 4
+    assert waves // per * per == waves or per == 1
+    if held == 4:
+        assert per == 8
+    elif held == 100:
+        assert vgprs > 256 and per == 1

@@ -2,6 +2,7 @@
 block takes one workgroup and where it takes several (around the rule's line:
 four blocks' worth of them along x), with and without a base workgroup: every
 invocation sees its own ids and the dispatch's size, as it writes them itself.
+Shaders that need many registers, whose blocks take fewer workgroups or one.
 And a dispatch whose rows have more threads in all than a launch takes along x
 in linear blocks."""
 import numpy as np
@@ -10,6 +11,7 @@ import pytest
 from kazan_amd.scenes import compute_shaders as cs
 from kazan_amd.scenes import spirv as sp
 from kazan_amd.scenes.compute import ComputeKernel, read_buffer
+from test_compute_launch import held_values_shader
 
 pytestmark = pytest.mark.gpu
 
@@ -99,6 +101,26 @@ def test_ids(ctx, local):
                 assert (got[want.size:] == 0xDEADBEEF).all()
     finally:
         k.destroy()
+
+
+@pytest.mark.parametrize("held", [4, 48, 100])
+def test_many_registers(ctx, held):
+    for groups in (1, 31, 33, 70):
+        n = 64 * groups
+        x = np.random.default_rng(groups).random((held, n), np.float32)
+        s = x[0].copy()
+        for y in x[1:]:
+            s += y
+        vb, ob = ctx.device_buffer_with(x), ctx.device_buffer_with(np.zeros(x.size + 64, np.float32))
+        k = ComputeKernel(ctx, held_values_shader(held), 2, push_bytes=4)
+        k.bind([(vb[0], x.nbytes), (ob[0], x.nbytes)])
+        k.run((groups,), push=np.array([n], np.uint32))
+        got = read_buffer(ctx, ob[0], x.nbytes + 256, np.float32)
+        k.destroy()
+        ctx.destroy_buffer(vb)
+        ctx.destroy_buffer(ob)
+        np.testing.assert_array_equal(got[:x.size].reshape(x.shape), x * s)
+        assert (got[x.size:] == 0).all()
 
 
 def test_long_rows_of_tall_workgroups(ctx):
