@@ -137,6 +137,11 @@ KAZAN_EXPORT int kazan_compile_compute_spirv(const uint32_t *words, size_t nword
 KAZAN_EXPORT int kazan_compute_launch(const uint32_t local[3], uint32_t per_block, const uint32_t groups[3],
                                       uint32_t grid[3], uint32_t block[3]);
 
+/* 1 if a batch of `triangles` over a width x height framebuffer is binned by
+ * gathering at tiles of tile_size px (8, 16, 32 or 64), 0 if by the radix
+ * sort, -1 for another tile size. */
+KAZAN_EXPORT int kazan_gather_binning(uint32_t triangles, uint32_t width, uint32_t height, uint32_t tile_size);
+
 #ifdef __cplusplus
 }
 #endif

@@ -105,6 +105,7 @@ bool Engine::init(int hip_device, std::string &err) {
     if (const char *e = std::getenv("KAZAN_BINNING")) {
         radix_ = std::strcmp(e, "sort") != 0;
         gather_ = radix_ && std::strcmp(e, "radix") != 0;
+        gather_always_ = std::strcmp(e, "gather") == 0;
     }
     if (const char *e = std::getenv("KAZAN_GRID_DIVISOR")) {
         const int d = std::atoi(e);
@@ -310,15 +311,41 @@ uint32_t gather_square_cap(uint32_t tris, uint32_t supers) {
 }
 }  // namespace
 
-// Gather binning is for batches whose squares' triangle lists are short: the
-// tiles of a square all read its list, so the work grows with the square of
-// the triangles' density, where radix binning's grows with the pairs. At
-// 65,536 triangles and 720p its two launches took 37 us against the radix
-// chain's 45 (a cluster), 34 against 46 (64 meshes) and 25 against 52 (a
-// grid); at 131,072 in 64 meshes, most of them in a few squares, 150 against
-// 62. (squares: their totals are summed by every workgroup.)
-bool Engine::use_gather(const KzFrame &f) const {
-    return gather_ && f.total_tris <= kGatherTris && (uint64_t)squares(f.width) * squares(f.height) <= kGatherSquares;
+// Gather binning's work, where radix binning's grows with the pairs only:
+// - every segment is tested against every square (2.1 ns each);
+// - a square's blocks of 8 tiles each read its list: ns per square by tile
+//   size, as a grid's tiles cost them (a cluster's empty squares less);
+// - they do so the longer the denser the triangles, and at larger tiles a
+//   wave walks more of them alone.
+// The line is where it stays ahead of the radix chain (42 to 52 us, or 62 with
+// the model's statistics) in all of a grid, a cluster, 64 meshes and large
+// triangles. Frames, radix us / gather us (grid, cluster, meshes), one
+// configuration each:
+//   16 px tiles: 65,536 triangles at 720p 119/96, 97/94, 97/83 and at 1080p
+//   138/127, 96/91, 109/101; 49,152 at 1440p 169/169, 96/93, 111/104; past the
+//   line 65,536 at 1440p 174/179, 100/102, 117/119, at 4K 261/309, 113/145,
+//   129/150, and in 640x480 (3,277 a square) 101/79, 120/144, 92/74;
+//   8 px: 16,384 in 640x480 99/89, 80/58, 74/57; past it 8,192 at 720p
+//   125/150, 82/71, 85/70 and at 4K 405/644, 149/191, 169/216;
+//   32 px: 32,768 at 720p 132/107, 116/112, 110/92; past it 65,536 146/138,
+//   121/151, 126/116, and 16,384 in 640x480 126/114, 92/103, 75/66;
+//   64 px: 16,384 at 1080p 360/346, 137/134, 127/123; past it 32,768 399/388,
+//   145/159, 143/148.
+bool gather_pays(uint32_t tris, uint32_t width, uint32_t height, uint32_t shift) {
+    const uint64_t supers = (uint64_t)squares(width) * squares(height);
+    const uint64_t segs = (tris + KZ_GATHER_SEG - 1) / KZ_GATHER_SEG;
+    static constexpr uint32_t kSquareNs[] = {1400, 96, 24, 8};  // 8 px tiles on
+    static_assert(sizeof kSquareNs / sizeof *kSquareNs == kMaxTileShift - kMinTileShift + 1, "a cost per tile size");
+    const uint32_t most = shift <= 4 ? kGatherTris : shift == 5 ? kGatherTris / 2 : kGatherTris / 4;
+    return tris <= most && tris <= supers * (shift <= 4 ? 2048 : 640) &&
+           supers * (10 * kSquareNs[shift - kMinTileShift] + 21 * segs) <= 360000;
+}
+
+// (squares: their totals are summed by every workgroup)
+bool Engine::use_gather(const KzFrame &f, uint32_t shift) const {
+    if (!gather_ || f.total_tris > kGatherTris || (uint64_t)squares(f.width) * squares(f.height) > kGatherSquares)
+        return false;
+    return gather_always_ || gather_pays(f.total_tris, f.width, f.height, shift);
 }
 
 hipError_t Engine::ensure_gather(const KzFrame &f) {
@@ -390,7 +417,7 @@ hipError_t Engine::prepare_batch(const Op &op, uint32_t shift) {
             cap_rec_words_ = w;
         }
     }
-    if (use_gather(f)) KZ_TRY(ensure_gather(f));
+    if (use_gather(f, shift)) KZ_TRY(ensure_gather(f));
     const uint64_t clip_words = (uint64_t)cap_clip_ * KZ_REC_WORDS_FOR(op.variants->fixed.num_varyings);
     if (clip_words > cap_clip_words_) {
         KZ_TRY(hipStreamSynchronize(stream_));
@@ -485,7 +512,7 @@ hipError_t Engine::run_batch(const Op &op, const BatchConfig &cfg) {
     uint32_t launches = 0;
 
     // binning: pixel boxes, then the per-tile lists in primitive order
-    if (use_gather(f)) {
+    if (use_gather(f, shift)) {
         const uint32_t supers_x = squares(f.width), supers_y = squares(f.height);
         f.super_shift = KZ_SUPER_PX_SHIFT - shift;
         f.supers_x = supers_x;

@@ -230,6 +230,10 @@ struct GraphCache {
     bool recorded_per_frame = false;
 };
 
+// Whether gather binning is the faster one for a batch of `tris` triangles
+// over a width x height framebuffer at tiles of 1 << shift px.
+bool gather_pays(uint32_t tris, uint32_t width, uint32_t height, uint32_t shift);
+
 class Engine {
   public:
     ~Engine();
@@ -361,12 +365,13 @@ class Engine {
     uint32_t cap_clip_ = 0;
     uint64_t cap_clip_words_ = 0;
     uint32_t *tri_draw_ = nullptr;  // draw of each triangle, for batches of several draws
-    // Binning: for batches of few triangles every tile gathers its list; else
-    // radix (pairs in primitive order, stable radix sort by tile). With
-    // KAZAN_BINNING=radix always radix, with =sort per-tile counts, an
-    // unordered scatter and a sort of every list.
-    bool radix_ = true, gather_ = true;
-    bool use_gather(const KzFrame &f) const;
+    // Binning: for batches of few triangles on few tiles every tile gathers
+    // its list (gather_pays); else radix (pairs in primitive order, stable
+    // radix sort by tile). With KAZAN_BINNING=gather wherever its tables fit,
+    // with =radix always radix, with =sort per-tile counts, an unordered
+    // scatter and a sort of every list.
+    bool radix_ = true, gather_ = true, gather_always_ = false;
+    bool use_gather(const KzFrame &f, uint32_t shift) const;
     hipError_t ensure_gather(const KzFrame &f);
     uint32_t *gather_seg_ = nullptr, *gather_list_ = nullptr, *super_state_ = nullptr;
     uint64_t cap_gather_ = 0;

@@ -190,6 +190,12 @@ extern "C" int kazan_compute_launch(const uint32_t local[3], uint32_t per_block,
     return (int)c.per_block;
 }
 
+extern "C" int kazan_gather_binning(uint32_t triangles, uint32_t width, uint32_t height, uint32_t tile_size) {
+    for (uint32_t s = kz::kMinTileShift; s <= kz::kMaxTileShift; ++s)
+        if (tile_size == 1u << s) return kz::gather_pays(triangles, width, height, s) ? 1 : 0;
+    return -1;
+}
+
 // --- the learned tile-cost model's kernels, outside a Vulkan device ------
 
 static_assert(KAZAN_COST_PARAMS == KZ_PARAMS, "parameter count of kazan_tools.h");

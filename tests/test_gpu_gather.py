@@ -1,5 +1,6 @@
-"""Gather binning (batches of up to 65,536 triangles): every tile collects its
-list from its 128 px square's triangles. Triangle counts at the edges of a
+"""Gather binning: every tile collects its list from its 128 px square's
+triangles. On devices that use it wherever its tables fit (also where the rule
+would sort), but for one test of the rule itself. Triangle counts at the edges of a
 2,048-triangle segment, a block of tiles with more candidates than its
 workgroup holds (6,144), a square with more triangles than its coarse list
 takes (its segments are then tested one by one), the largest batch it takes
@@ -13,9 +14,22 @@ import pytest
 
 from kazan_amd.scenes import generators as g
 from scene_kit import scene_from_pixels
-from test_gpu_parity import check_parity, mctx  # noqa: F401  (the per-form device fixture)
+from test_gpu_parity import check_parity
 
 pytestmark = pytest.mark.gpu
+
+_CTX = {}
+
+
+@pytest.fixture(params=["balanced", "plain"])
+def mctx(request, driver, monkeypatch):
+    """A device of each pipeline form that gathers."""
+    from kazan_amd.scenes.renderer import Context
+    if request.param not in _CTX:
+        monkeypatch.setenv("KAZAN_PIPELINE", request.param)
+        monkeypatch.setenv("KAZAN_BINNING", "gather")
+        _CTX[request.param] = Context(driver)
+    return _CTX[request.param]
 
 
 def _scene(n, w, h, box, size=1.0, large=()):
@@ -56,8 +70,28 @@ def test_largest_batch(mctx, oracle, n):
 def test_storage_too_small(driver, monkeypatch, oracle, form):
     from kazan_amd.scenes.renderer import Context
     monkeypatch.setenv("KAZAN_PIPELINE", form)
+    monkeypatch.setenv("KAZAN_BINNING", "gather")
     monkeypatch.setenv("KAZAN_LIST_CAPACITY_LIMIT", "1000")
     ctx = Context(driver)
     for s in (_scene(5000, 256, 128, (0, 0, 256, 128), large=range(0, 5000, 50)), g.camera_inside(300, 300, 256, 192)):
         st, _, _ = check_parity(ctx, oracle, s, frames=2)
         assert st["list_overflow"] >= 1
+
+
+def test_rule(driver, monkeypatch, oracle):
+    """Either side of the rule's lines, at one tile size: the launches are those of the binning it names."""
+    from kazan_amd.scenes.renderer import Context
+    monkeypatch.setenv("KAZAN_AUTOTUNE", "0")
+    monkeypatch.setenv("KAZAN_TILE_SHIFT", "4")
+    ctxs = {}
+    for binning in (None, "radix", "gather"):
+        with monkeypatch.context() as m:
+            if binning:
+                m.setenv("KAZAN_BINNING", binning)
+            ctxs[binning] = Context(driver)
+    for n, w, h in ((2048, 128, 128), (2049, 128, 128), (3000, 2048, 2048), (3000, 3840, 2160)):
+        s = _scene(n, w, h, (0, 0, w, h), size=4.0)
+        launches = {b: check_parity(c, oracle, s)[0]["launches"] for b, c in ctxs.items()}
+        named = "gather" if driver.lib.kazan_gather_binning(n, w, h, 16) else "radix"
+        assert launches["gather"] != launches["radix"]
+        assert launches[None] == launches[named], (n, w, h)
