@@ -702,9 +702,10 @@ int final_choice(const BatchTuning &t) {
 }
 }  // namespace
 
-// Candidates, one HIP-event-timed trial per submission: every tile size
-// whose kernels fit (full grid, the plan with the cost model when there is
-// one); at the fastest size, the model's plan with its fragment weight times
+// Candidates, one HIP-event-timed trial per submission from a recording's
+// second on: every tile size whose kernels fit (full grid, the plan with the
+// cost model when there is one; the pipeline's own size, which the first
+// submission ran untimed, last); at the fastest size, the model's plan with its fragment weight times
 // 16 (without a model a half grid) and the plain raster (one workgroup per
 // tile, no plan); at the fastest of those, the plan without the model and
 // the plain raster of the next smaller tiles (the plain raster's neighbours
@@ -716,31 +717,21 @@ int final_choice(const BatchTuning &t) {
 // (both were chosen with the deepest splits and the model; with fewer splits
 // smaller tiles on a larger grid may pay); then the three fastest twice more
 // each. The finalist with the lowest median of its three runs is kept.
-hipError_t Engine::pick_config(Op &op, BatchConfig &cfg, bool &timed, bool tune) {
-    cfg = default_config(op);
-    timed = false;
+hipError_t Engine::advance_tuning(Op &op) {
     if (!autotune()) return hipSuccess;
-    if (!tune) {
-        // (without the model: its statistics and predictions cost more than
-        // its plan saves unless a trial has shown otherwise)
-        cfg.model = false;
-        return hipSuccess;
-    }
     const bool model = cost_model_d_ != nullptr;
     if (!op.tuning) {
         op.tuning = std::make_shared<BatchTuning>();
         BatchTuning &t = *op.tuning;
         for (uint32_t s = kMinTileShift; s <= kMaxTileShift; ++s)
-            if (op.variants->fits(s)) t.cand.push_back({s, 1u, model, true, 2u});
+            if (s != op.tile_shift && op.variants->fits(s)) t.cand.push_back({s, 1u, model, true, 2u});
+        t.cand.push_back({op.tile_shift, 1u, model, true, 2u});
         t.ms.assign(t.cand.size(), -1.0f);
         KZ_TRY(hipEventCreate(&t.ev[0]));
         KZ_TRY(hipEventCreate(&t.ev[1]));
     }
     BatchTuning &t = *op.tuning;
-    if (t.done) {
-        cfg = t.choice;
-        return hipSuccess;
-    }
+    if (t.done) return hipSuccess;
     if (t.pending >= 0) {  // the previous submission's trial
         KZ_TRY(hipEventSynchronize(t.ev[1]));
         float ms = -1.0f;
@@ -803,46 +794,66 @@ hipError_t Engine::pick_config(Op &op, BatchConfig &cfg, bool &timed, bool tune)
         }
         ++t.phase;
     }
-    if (t.next < t.cand.size()) {
-        cfg = t.cand[t.next];
-        t.pending = (int)t.next++;
-        timed = true;
-        return hipSuccess;
-    }
+    if (t.next < t.cand.size()) return hipSuccess;
     const int best = final_choice(t);
     t.done = true;
     if (t.trial) hipGraphExecDestroy(t.trial);
     t.trial = nullptr;
     if (best >= 0) t.choice = t.cand[best];
     else t.choice = default_config(op);
-    cfg = t.choice;
-    last_tuned_ = cfg;
+    last_tuned_ = t.choice;
     return hipSuccess;
+}
+
+// What a submission runs the batch with: the choice, the next trial, or (the
+// recording's first submission, `tune` false) the untuned configuration, with
+// the model if `model`.
+void Engine::pick_config(Op &op, BatchConfig &cfg, bool &timed, bool tune, bool model) {
+    cfg = default_config(op);
+    timed = false;
+    if (!autotune()) return;
+    if (!tune) {
+        cfg.model = model;
+        return;
+    }
+    BatchTuning &t = *op.tuning;
+    if (t.done) {
+        cfg = t.choice;
+    } else if (t.next < t.cand.size()) {
+        cfg = t.cand[t.next];
+        t.pending = (int)t.next++;
+        timed = true;
+    }
 }
 
 hipError_t Engine::execute(std::vector<Op> &ops, GraphCache *cache) {
     // Graphs pay off for command buffers that draw and are submitted again:
-    // the first submission (and every tuning trial) runs eagerly.
+    // the first submission (and every tuning trial) runs eagerly. The first
+    // is no trial: a command buffer recorded (or allocated) for every frame
+    // would run the same one in all of them and never learn from it, and it
+    // would load another tile size's kernels than the pipeline's creation did.
     bool graphable = cache != nullptr && graphs_ && !kernel_timing_;
+    const bool first = cache && cache->eager_runs == 0;
     bool draws = false;
     for (Op &op : ops)
         if (op.kind == Op::Batch) {
             draws = true;
+            if (!first) KZ_TRY(advance_tuning(op));
             if (autotune() && !(op.tuning && op.tuning->done)) graphable = false;
         }
-    if (!graphable || !draws || (cache->eager_runs == 0 && !cache->exec)) {
-        // a command buffer recorded for every frame would run its first trial
-        // in all of them, and never learn from it
-        const bool first = cache && cache->eager_runs == 0;
+    if (!graphable || !draws || first) {
         if (cache) ++cache->eager_runs;
-        return execute_eager(ops, !first || !cache->recorded_per_frame, !first);
+        // (without the model in a recording for every frame: its statistics
+        // and predictions cost more than its plan saves unless a trial has
+        // shown otherwise)
+        return execute_eager(ops, !first, !first || !cache->recorded_per_frame);
     }
     // every allocation before the capture
     for (Op &op : ops)
         if (op.kind == Op::Batch) {
             BatchConfig cfg;
             bool timed;
-            KZ_TRY(pick_config(op, cfg, timed));
+            pick_config(op, cfg, timed);
             if (!op.variants->get(cfg.shift)) return execute_eager(ops);
             KZ_TRY(prepare_batch(op, cfg.shift));
         }
@@ -896,15 +907,13 @@ hipError_t Engine::warm_raster(const PipelineKernels *kern) {
 // in one: a kernel of a replayed graph takes at least 4.5 us, launched by
 // itself half of that, so that trials of single launches favour plans of ten
 // small kernels. The device waits first until the host has queued the rest.
-// Not so (`graph`) in a recording's first submission, which may be its only
-// one: the graph would cost it 0.2 ms.
 // (With the plain raster tried at smaller tiles too, 131,072 Phong triangles
 // at 720p and four samples 167 us a frame -> 130.)
-hipError_t Engine::run_trial(const Op &op, const BatchConfig &cfg, bool graph) {
+hipError_t Engine::run_trial(const Op &op, const BatchConfig &cfg) {
     BatchTuning &t = *op.tuning;
     if (t.trial) hipGraphExecDestroy(t.trial);  // (the trial before has ended: its events were read)
     t.trial = nullptr;
-    if (graph && graphs_ && !kernel_timing_) {
+    if (graphs_ && !kernel_timing_) {
         const uint32_t b0 = pending_batches_, l0 = pending_launches_;
         const uint64_t gen = generation_;
         hipGraph_t captured = nullptr;
@@ -925,18 +934,18 @@ hipError_t Engine::run_trial(const Op &op, const BatchConfig &cfg, bool graph) {
             if (e != hipSuccess) return e;
         }
     }
-    if (graph) KZ_TRY(kz_launch_wait(stream_));
+    KZ_TRY(kz_launch_wait(stream_));
     KZ_TRY(hipEventRecord(t.ev[0], stream_));
     KZ_TRY(t.trial ? hipGraphLaunch(t.trial, stream_) : run_batch(op, cfg));
     return hipEventRecord(t.ev[1], stream_);
 }
 
-hipError_t Engine::execute_eager(std::vector<Op> &ops, bool tune, bool graph_trials) {
+hipError_t Engine::execute_eager(std::vector<Op> &ops, bool tune, bool model) {
     for (Op &op : ops)
         if (op.kind == Op::Batch) {
             BatchConfig cfg;
             bool timed;
-            KZ_TRY(pick_config(op, cfg, timed, tune));
+            pick_config(op, cfg, timed, tune, model);
             if (timed) {
                 // a trial times the batch, not the loading of a tile size's
                 // kernels or the growth of its scratch (host work and syncs)
@@ -944,7 +953,7 @@ hipError_t Engine::execute_eager(std::vector<Op> &ops, bool tune, bool graph_tri
                     KZ_TRY(prepare_batch(op, cfg.shift));
                     if (!cfg.persistent) KZ_TRY(warm_raster(kern));
                 }
-                KZ_TRY(run_trial(op, cfg, graph_trials));
+                KZ_TRY(run_trial(op, cfg));
             } else {
                 KZ_TRY(run_batch(op, cfg));
             }

@@ -226,7 +226,7 @@ struct GraphCache {
     uint32_t batches = 0, launches = 0;
     uint32_t eager_runs = 0;  // a command buffer is captured from its second submission on
     // the command buffer was recorded anew after a single submission: its
-    // first submission takes the untuned configuration
+    // first submission goes without the cost model
     bool recorded_per_frame = false;
 };
 
@@ -303,15 +303,18 @@ class Engine {
 
   private:
     hipError_t ensure_scratch(uint32_t tiles, uint32_t tris);
-    // the configuration a batch runs with this submission (tuning trial or
-    // the tuned choice), and its scratch allocated for it
-    hipError_t pick_config(Op &op, BatchConfig &cfg, bool &timed, bool tune = true);
+    // reads the last trial's time, adds the candidates it leads to, and
+    // concludes when none is left
+    hipError_t advance_tuning(Op &op);
+    // the configuration a batch runs with this submission (untuned, tuning
+    // trial or the tuned choice)
+    void pick_config(Op &op, BatchConfig &cfg, bool &timed, bool tune = true, bool model = true);
     BatchConfig default_config(const Op &op) const;
     hipError_t prepare_batch(const Op &op, uint32_t shift);
     hipError_t run_batch(const Op &op, const BatchConfig &cfg);
-    hipError_t execute_eager(std::vector<Op> &ops, bool tune = true, bool graph_trials = true);
+    hipError_t execute_eager(std::vector<Op> &ops, bool tune = true, bool model = true);
     hipError_t warm_raster(const PipelineKernels *kern);
-    hipError_t run_trial(const Op &op, const BatchConfig &cfg, bool graph);
+    hipError_t run_trial(const Op &op, const BatchConfig &cfg);
     uint32_t *zero_word_ = nullptr;
     hipError_t launch_ops(std::vector<Op> &ops);  // tuned configurations, no tuning events
     hipError_t launch_ops_one(const Op &op);      // a non-batch op

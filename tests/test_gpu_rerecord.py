@@ -36,3 +36,24 @@ def test_recorded_for_every_frame(driver, monkeypatch, oracle, form):
             r._record()
         _check(r, oracle, r.render(1), 1)
     _check(r, oracle, r.render(40), 40)
+
+
+def test_first_submission_loads_no_other_kernels(driver, monkeypatch, tmp_path):
+    """A recording's first submission, often its only one, draws with the tile
+    size its pipeline was created with: a new pipeline's other sizes are
+    compiled (and loaded) by the submissions after it."""
+    import os
+    from kazan_amd.scenes.renderer import Context, SceneRenderer
+    monkeypatch.setenv("KAZAN_PIPELINE", "balanced")
+    monkeypatch.setenv("KAZAN_PIPELINE_CACHE", str(tmp_path))
+    ctx = Context(driver)
+    s = g.zipf_draws(20, 2000, 320, 180)
+    r = SceneRenderer(ctx, s)
+    created = sorted(os.listdir(tmp_path))
+    assert len(created) == 1
+    for _ in range(3):  # command buffers allocated, submitted once and freed
+        r.render(1)
+        assert sorted(os.listdir(tmp_path)) == created
+        r._record()
+    r.render(2)
+    assert len(os.listdir(tmp_path)) == 2
