@@ -142,6 +142,14 @@ KAZAN_EXPORT int kazan_compute_launch(const uint32_t local[3], uint32_t per_bloc
  * sort, -1 for another tile size. */
 KAZAN_EXPORT int kazan_gather_binning(uint32_t triangles, uint32_t width, uint32_t height, uint32_t tile_size);
 
+/* The search for a batch's configuration, over times that ms() gives instead
+ * of the device. A configuration is {tile size in px, grid divisor, cost model,
+ * persistent raster, deepest split, fragment weight scale}. own_tile: the
+ * pipeline's tile size; largest_tile: the largest that fits. Writes up to cap
+ * trials in order and the choice; returns the number of trials, or -1. */
+KAZAN_EXPORT int kazan_tune(uint32_t own_tile, uint32_t largest_tile, uint32_t model, float (*ms)(const uint32_t *),
+                            uint32_t *trials, uint32_t cap, uint32_t *choice);
+
 #ifdef __cplusplus
 }
 #endif

@@ -702,33 +702,102 @@ int final_choice(const BatchTuning &t) {
 }
 }  // namespace
 
+// The first candidates: every tile size, the pipeline's own (which the first
+// submission ran untimed) last.
+void BatchTuning::begin(uint32_t own_shift, bool model) {
+    for (uint32_t s = kMinTileShift; s <= kMaxTileShift; ++s)
+        if (s != own_shift) cand.push_back({s, 1u, model, true, 2u});
+    cand.push_back({own_shift, 1u, model, true, 2u});
+    ms.assign(cand.size(), -1.0f);
+}
+
 // Candidates, one HIP-event-timed trial per submission from a recording's
-// second on: every tile size whose kernels fit (full grid, the plan with the
-// cost model when there is one; the pipeline's own size, which the first
-// submission ran untimed, last); at the fastest size, the model's plan with its fragment weight times
-// 16 (without a model a half grid) and the plain raster (one workgroup per
-// tile, no plan); at the fastest of those, the plan without the model and
-// the plain raster of the next smaller tiles (the plain raster's neighbours
-// when it is the fastest); at the fastest planned one, splits of at most 4
-// sub-tiles and none (many small triangles are set up once per sub-tile they
-// touch); with a cost model, the model's plan with its fragment weight times 4
-// and 16 (a pipeline whose fragments cost more than the training pipelines');
-// at the fastest planned one, every other pair of tile size and grid size
-// (both were chosen with the deepest splits and the model; with fewer splits
-// smaller tiles on a larger grid may pay); then the three fastest twice more
-// each. The finalist with the lowest median of its three runs is kept.
+// second on: every tile size (full grid, the plan with the cost model when
+// there is one); at the fastest size, the model's plan with its fragment
+// weight times 16 (without a model a half grid) and the plain raster (one
+// workgroup per tile, no plan); at the fastest of those, the plan without the
+// model and the plain raster of the next smaller tiles (the plain raster's
+// neighbours when it is the fastest); at the fastest planned one, splits of at
+// most 4 sub-tiles and none (many small triangles are set up once per sub-tile
+// they touch); with a cost model, the model's plan with its fragment weight
+// times 4 and 16 (a pipeline whose fragments cost more than the training
+// pipelines'); at the fastest planned one, every other pair of tile size and grid size (both were chosen with the deepest
+// splits and the model; with fewer splits smaller tiles on a larger grid may
+// pay); then the three fastest twice more each. The finalist with the lowest median of its three runs is kept.
+// Candidates whose kernels do not build (tiles that do not fit LDS among
+// them) are passed over. False when no trial is left: choice is then set, or
+// left as it was if none could be timed.
+bool BatchTuning::more(bool model, const std::function<bool(uint32_t shift)> &builds) {
+    for (;; ++phase) {
+        while (next < cand.size() && !builds(cand[next].shift)) ++next;
+        if (next < cand.size()) return true;
+        if (phase == 6) break;
+        const int best = fastest(*this);
+        if (best < 0) continue;
+        const BatchConfig b = cand[best];
+        if (phase == 0) {
+            // (fragments weighted 16 times: where a frame has few tiles, of
+            // many fragments each, its splits are what a plan is for, and it
+            // has to be seen before the plain raster ends the search: 256
+            // triangles in 64^2 83 us a frame, plain 89)
+            if (b.model) cand.push_back({b.shift, 1u, true, true, 2u, 16u});
+            else cand.push_back({b.shift, 2u, false, true, 2u, 1u});
+            cand.push_back({b.shift, 1u, false, false, 2u, 1u});
+        } else if (phase == 1) {
+            // the plain raster has only its tiles to fill the chip with:
+            // smaller ones often suit it better than the plan's best
+            const uint32_t s = b.shift > kMinTileShift ? b.shift - 1 : b.shift + 1;
+            if (b.persistent && b.model) cand.push_back({b.shift, b.grid_div, false, true, 2u, 1u});
+            if (!b.persistent) cand.push_back({s > b.shift ? s + 1 : b.shift + 1, 1u, false, false, 2u, 1u});
+            cand.push_back({s, 1u, false, false, 2u, 1u});
+        } else if (phase == 2) {
+            if (b.persistent) {
+                cand.push_back({b.shift, b.grid_div, b.model, true, 1u, 1u});
+                cand.push_back({b.shift, b.grid_div, b.model, true, 0u, 1u});
+            }
+        } else if (phase == 3) {
+            if (b.persistent && model) {
+                // (splitting by triangle counts may not have paid; by weighted
+                // fragments it may)
+                cand.push_back({b.shift, b.grid_div, true, true, 2u, 4u});
+                cand.push_back({b.shift, b.grid_div, true, true, 2u, 16u});
+            }
+        } else if (phase == 4) {
+            if (b.persistent)
+                for (uint32_t s = kMinTileShift; s <= kMaxTileShift; ++s)
+                    for (uint32_t d : {1u, 2u, 4u})
+                        if (s != b.shift || d != b.grid_div)
+                            cand.push_back({s, d, b.model, true, b.max_level, b.frag_scale});
+        } else {
+            // the three fastest twice more each (a near tie is decided by the
+            // median of three runs, not by one run's noise)
+            std::vector<size_t> order;
+            for (size_t i = 0; i < cand.size(); ++i)
+                if (ms[i] >= 0) order.push_back(i);
+            std::sort(order.begin(), order.end(), [&](size_t x, size_t y) { return ms[x] < ms[y]; });
+            for (size_t k = 0; k < order.size() && k < 3; ++k) {
+                const BatchConfig c = cand[order[k]];
+                finals.push_back({order[k], cand.size(), cand.size() + 1});
+                cand.push_back(c);
+                cand.push_back(c);
+            }
+        }
+        ms.resize(cand.size(), -1.0f);
+    }
+    const int best = final_choice(*this);
+    if (best >= 0) choice = cand[best];
+    return false;
+}
+
 hipError_t Engine::advance_tuning(Op &op) {
     if (!autotune()) return hipSuccess;
     const bool model = cost_model_d_ != nullptr;
     if (!op.tuning) {
         op.tuning = std::make_shared<BatchTuning>();
-        BatchTuning &t = *op.tuning;
-        for (uint32_t s = kMinTileShift; s <= kMaxTileShift; ++s)
-            if (s != op.tile_shift && op.variants->fits(s)) t.cand.push_back({s, 1u, model, true, 2u});
-        t.cand.push_back({op.tile_shift, 1u, model, true, 2u});
-        t.ms.assign(t.cand.size(), -1.0f);
-        KZ_TRY(hipEventCreate(&t.ev[0]));
-        KZ_TRY(hipEventCreate(&t.ev[1]));
+        op.tuning->begin(op.tile_shift, model);
+        op.tuning->choice = default_config(op);
+        KZ_TRY(hipEventCreate(&op.tuning->ev[0]));
+        KZ_TRY(hipEventCreate(&op.tuning->ev[1]));
     }
     BatchTuning &t = *op.tuning;
     if (t.done) return hipSuccess;
@@ -738,69 +807,10 @@ hipError_t Engine::advance_tuning(Op &op) {
         if (hipEventElapsedTime(&ms, t.ev[0], t.ev[1]) == hipSuccess) t.ms[t.pending] = ms;
         t.pending = -1;
     }
-    // skip candidates whose kernels do not build
-    while (t.next < t.cand.size() && !op.variants->get(t.cand[t.next].shift)) ++t.next;
-    while (t.next == t.cand.size() && t.phase < 6) {
-        const int best = fastest(t);
-        if (best >= 0) {
-            const BatchConfig b = t.cand[best];
-            if (t.phase == 0) {
-                // (fragments weighted 16 times: where a frame has few tiles, of
-                // many fragments each, its splits are what a plan is for, and
-                // it has to be seen before the plain raster ends the search:
-                // 256 triangles in 64^2 83 us a frame, plain 89)
-                if (b.model) t.cand.push_back({b.shift, 1u, true, true, 2u, 16u});
-                else t.cand.push_back({b.shift, 2u, false, true, 2u, 1u});
-                t.cand.push_back({b.shift, 1u, false, false, 2u, 1u});
-            } else if (t.phase == 1) {
-                // the plain raster has only its tiles to fill the chip with:
-                // smaller ones often suit it better than the plan's best
-                const uint32_t s = b.shift > kMinTileShift ? b.shift - 1 : b.shift + 1;
-                if (b.persistent && b.model) t.cand.push_back({b.shift, b.grid_div, false, true, 2u, 1u});
-                if (!b.persistent) t.cand.push_back({s > b.shift ? s + 1 : b.shift + 1, 1u, false, false, 2u, 1u});
-                t.cand.push_back({s, 1u, false, false, 2u, 1u});
-            } else if (t.phase == 2) {
-                if (b.persistent) {
-                    t.cand.push_back({b.shift, b.grid_div, b.model, true, 1u, 1u});
-                    t.cand.push_back({b.shift, b.grid_div, b.model, true, 0u, 1u});
-                }
-            } else if (t.phase == 3) {
-                if (b.persistent && model) {
-                    // (splitting by triangle counts may not have paid; by
-                    // weighted fragments it may)
-                    t.cand.push_back({b.shift, b.grid_div, true, true, 2u, 4u});
-                    t.cand.push_back({b.shift, b.grid_div, true, true, 2u, 16u});
-                }
-            } else if (t.phase == 4) {
-                if (b.persistent)
-                    for (uint32_t s = kMinTileShift; s <= kMaxTileShift; ++s)
-                        for (uint32_t d : {1u, 2u, 4u})
-                            if ((s != b.shift || d != b.grid_div) && op.variants->fits(s))
-                                t.cand.push_back({s, d, b.model, true, b.max_level, b.frag_scale});
-            } else {
-                // the three fastest twice more each (a near tie is decided
-                // by the median of three runs, not by one run's noise)
-                std::vector<size_t> order;
-                for (size_t i = 0; i < t.cand.size(); ++i)
-                    if (t.ms[i] >= 0) order.push_back(i);
-                std::sort(order.begin(), order.end(), [&](size_t x, size_t y) { return t.ms[x] < t.ms[y]; });
-                for (size_t k = 0; k < order.size() && k < 3; ++k) {
-                    t.finals.push_back({order[k], t.cand.size(), t.cand.size() + 1});
-                    t.cand.push_back(t.cand[order[k]]);
-                    t.cand.push_back(t.cand[order[k]]);
-                }
-            }
-            t.ms.resize(t.cand.size(), -1.0f);
-        }
-        ++t.phase;
-    }
-    if (t.next < t.cand.size()) return hipSuccess;
-    const int best = final_choice(t);
+    if (t.more(model, [&](uint32_t shift) { return op.variants->get(shift) != nullptr; })) return hipSuccess;
     t.done = true;
     if (t.trial) hipGraphExecDestroy(t.trial);
     t.trial = nullptr;
-    if (best >= 0) t.choice = t.cand[best];
-    else t.choice = default_config(op);
     last_tuned_ = t.choice;
     return hipSuccess;
 }

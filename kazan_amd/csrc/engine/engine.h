@@ -12,6 +12,7 @@
 
 #include <atomic>
 #include <cstdint>
+#include <functional>
 #include <memory>
 #include <string>
 #include <vector>
@@ -146,6 +147,8 @@ struct BatchTuning {
     BatchTuning(const BatchTuning &) = delete;
     BatchTuning &operator=(const BatchTuning &) = delete;
     ~BatchTuning();
+    void begin(uint32_t own_shift, bool model);
+    bool more(bool model, const std::function<bool(uint32_t shift)> &builds);
     bool done = false;
     int phase = 0;  // 0: tile sizes, 1, 2: plan and raster forms, 3: split depth, 4: fragment weight,
                     // 5: every tile size x grid size again, 6: the three fastest twice more each

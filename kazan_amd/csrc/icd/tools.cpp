@@ -196,6 +196,29 @@ extern "C" int kazan_gather_binning(uint32_t triangles, uint32_t width, uint32_t
     return -1;
 }
 
+extern "C" int kazan_tune(uint32_t own_tile, uint32_t largest_tile, uint32_t model, float (*ms)(const uint32_t *),
+                          uint32_t *trials, uint32_t cap, uint32_t *choice) {
+    uint32_t own = kz::kMinTileShift;
+    while (own < kz::kMaxTileShift && 1u << own != own_tile) ++own;
+    if (!ms || !trials || !choice || 1u << own != own_tile) return -1;
+    kz::BatchTuning t;
+    t.begin(own, model != 0);
+    auto put_config = [](uint32_t *p, const kz::BatchConfig &c) {
+        const uint32_t v[6] = {1u << c.shift, c.grid_div, c.model, c.persistent, c.max_level, c.frag_scale};
+        std::memcpy(p, v, sizeof v);
+    };
+    uint32_t n = 0;
+    while (t.more(model != 0, [&](uint32_t s) { return s <= kz::kMaxTileShift && 1u << s <= largest_tile; })) {
+        uint32_t c[6];
+        put_config(c, t.cand[t.next]);
+        if (n < cap) std::memcpy(trials + 6 * n, c, sizeof c);
+        t.ms[t.next++] = ms(c);
+        ++n;
+    }
+    put_config(choice, t.choice);
+    return (int)n;
+}
+
 // --- the learned tile-cost model's kernels, outside a Vulkan device ------
 
 static_assert(KAZAN_COST_PARAMS == KZ_PARAMS, "parameter count of kazan_tools.h");
