@@ -720,10 +720,12 @@ void BatchTuning::begin(uint32_t own_shift, bool model) {
 // neighbours when it is the fastest); at the fastest planned one, splits of at
 // most 4 sub-tiles and none (many small triangles are set up once per sub-tile
 // they touch); with a cost model, the model's plan with its fragment weight
-// times 4 and 16 (a pipeline whose fragments cost more than the training
-// pipelines'); at the fastest planned one, every other pair of tile size and grid size (both were chosen with the deepest
+// times 4, and times 16 with splits of at most 4 (a pipeline whose fragments
+// cost more than the training pipelines'); at the fastest planned one, every
+// other pair of tile size and grid size (both were chosen with the deepest
 // splits and the model; with fewer splits smaller tiles on a larger grid may
-// pay); then the three fastest twice more each. The finalist with the lowest median of its three runs is kept.
+// pay); then the three fastest, no two of them the same configuration, twice
+// more each. The finalist with the lowest median of its three runs is kept.
 // Candidates whose kernels do not build (tiles that do not fit LDS among
 // them) are passed over. False when no trial is left: choice is then set, or
 // left as it was if none could be timed.
@@ -760,7 +762,7 @@ bool BatchTuning::more(bool model, const std::function<bool(uint32_t shift)> &bu
                 // (splitting by triangle counts may not have paid; by weighted
                 // fragments it may)
                 cand.push_back({b.shift, b.grid_div, true, true, 2u, 4u});
-                cand.push_back({b.shift, b.grid_div, true, true, 2u, 16u});
+                cand.push_back({b.shift, b.grid_div, true, true, 1u, 16u});
             }
         } else if (phase == 4) {
             if (b.persistent)
@@ -775,9 +777,12 @@ bool BatchTuning::more(bool model, const std::function<bool(uint32_t shift)> &bu
             for (size_t i = 0; i < cand.size(); ++i)
                 if (ms[i] >= 0) order.push_back(i);
             std::sort(order.begin(), order.end(), [&](size_t x, size_t y) { return ms[x] < ms[y]; });
-            for (size_t k = 0; k < order.size() && k < 3; ++k) {
-                const BatchConfig c = cand[order[k]];
-                finals.push_back({order[k], cand.size(), cand.size() + 1});
+            for (size_t i : order) {
+                const BatchConfig c = cand[i];
+                const bool again = std::any_of(finals.begin(), finals.end(),
+                                               [&](const std::vector<size_t> &f) { return cand[f[0]] == c; });
+                if (again || finals.size() == 3) continue;
+                finals.push_back({i, cand.size(), cand.size() + 1});
                 cand.push_back(c);
                 cand.push_back(c);
             }

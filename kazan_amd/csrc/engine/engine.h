@@ -137,6 +137,10 @@ struct BatchConfig {
     // training pipelines' fragment cost, and a pipeline whose fragments cost
     // more (a heavier fragment shader, more samples) needs a larger one
     uint32_t frag_scale = 1;
+    bool operator==(const BatchConfig &o) const {
+        return shift == o.shift && grid_div == o.grid_div && model == o.model && persistent == o.persistent &&
+               max_level == o.max_level && frag_scale == o.frag_scale;
+    }
 };
 
 // Autotuning of one batch (balanced form): its first submissions time

@@ -1,5 +1,6 @@
 """The search for a batch's configuration (kazan_tune: the tuner over given
-times): what it tries, and that it never tries what does not build."""
+times): what it tries, that it never tries what does not build, and that the
+runs that decide are of different configurations."""
 import ctypes
 import itertools
 
@@ -33,6 +34,20 @@ def _random_times(seed, favour=None):
     if favour:
         t = {c: (v - 0.9 if favour(c) else v) for c, v in t.items()}
     return t
+
+
+@pytest.mark.parametrize("seed", range(20))
+@pytest.mark.parametrize("favour", [None, lambda c: c[3] == 0, lambda c: c[3] == 1, lambda c: c[5] == 16])
+def test_finalists_differ(driver, seed, favour):
+    times = _random_times(seed, favour)
+    for model in (0, 1):
+        trials, choice = _tune(driver, times, model=model)
+        finals = trials[-6:]
+        assert finals[0] == finals[1] and finals[2] == finals[3] and finals[4] == finals[5]
+        assert len({finals[0], finals[2], finals[4]}) == 3, finals
+        # noise-free times: the three fastest of all that was tried, the fastest kept
+        assert [finals[0], finals[2], finals[4]] == sorted(set(trials[:-6]), key=times.get)[:3]
+        assert choice == min(trials, key=times.get)
 
 
 @pytest.mark.parametrize("own", [8, 16, 32])
