@@ -25,9 +25,6 @@ hipError_t grow(T *&p, uint64_t count) {
     return hipMalloc((void **)&p, std::max<uint64_t>(count, 1) * sizeof(T));
 }
 
-// clip pieces kept per batch: their records take 64 B and 12 B per varying
-constexpr uint32_t kMaxClipPieces = 65536;
-
 // gather binning: the most triangles and squares of a batch
 constexpr uint32_t kGatherTris = 65536, kGatherSquares = 1024;
 static_assert(kGatherTris <= KZ_GATHER_SEG * KZ_GATHER_SEGS, "segments of a batch");
@@ -98,6 +95,10 @@ bool Engine::init(int hip_device, std::string &err) {
     // KAZAN_LIST_CAPACITY_LIMIT caps the per-tile list storage (entries);
     // tiles whose lists do not fit render through the in-order scan path
     if (const char *e = std::getenv("KAZAN_LIST_CAPACITY_LIMIT")) list_limit_ = std::strtoull(e, nullptr, 10);
+    // KAZAN_CLIP_PIECES_LIMIT lowers the clip pieces kept per batch; triangles
+    // past them are clipped again in every tile
+    if (const char *e = std::getenv("KAZAN_CLIP_PIECES_LIMIT"))
+        clip_limit_ = (uint32_t)std::min<uint64_t>(std::strtoull(e, nullptr, 10), clip_limit_);
     if (const char *e = std::getenv("KAZAN_PIPELINE")) balanced_ = std::strcmp(e, "plain") != 0;
     if (const char *e = std::getenv("KAZAN_AUTOTUNE")) autotune_ = std::strcmp(e, "0") != 0;
     if (const char *e = std::getenv("KAZAN_GRAPHS")) graphs_ = std::strcmp(e, "0") != 0;
@@ -277,8 +278,8 @@ hipError_t Engine::ensure_scratch(uint32_t tiles, uint32_t tris) {
     if (tris > cap_tris_) {
         const uint32_t t = std::max(tris, cap_tris_ + cap_tris_ / 2);
         // (clip pieces: as many as there are triangles in a small batch; past
-        // kMaxClipPieces the raster clips what is left tile by tile)
-        cap_clip_ = radix_ && !setup_records_ ? std::min(std::max(t, 1024u), kMaxClipPieces) : 0u;
+        // the limit the raster clips what is left tile by tile)
+        cap_clip_ = radix_ && !setup_records_ ? std::min(std::max(t, 1024u), clip_limit_) : 0u;
         KZ_TRY(regrow(tri_rect_, (uint64_t)t + cap_clip_));
         KZ_TRY(regrow(tri_draw_, t));
         if (cap_clip_) {

@@ -372,7 +372,7 @@ class Engine {
     uint64_t *tri_rect_ = nullptr;
     // clip pieces (radix binning without setup records)
     uint32_t *clip_of_ = nullptr, *clip_tris_ = nullptr, *clip_rec_ = nullptr;
-    uint32_t cap_clip_ = 0;
+    uint32_t cap_clip_ = 0, clip_limit_ = 65536;  // pieces: their records take 64 B and 12 B per varying
     uint64_t cap_clip_words_ = 0;
     uint32_t *tri_draw_ = nullptr;  // draw of each triangle, for batches of several draws
     // Binning: for batches of few triangles on few tiles every tile gathers

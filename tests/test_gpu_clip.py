@@ -3,12 +3,14 @@ against the oracle's R-CLIP, through the Vulkan C ABI.
 
 Triangles that cross the near or far plane, reach behind the eye or leave
 the guard band are clipped into a fan of pieces drawn in their place: the
-binning kernel bins a clipped triangle by the union of its pieces' boxes,
-and the raster draws the pieces as a batch of their own. Cases: a camera
+binning kernel clips a triangle once and its pieces are list entries of their
+own; past the room for pieces it is binned by the union of their boxes, and
+the raster clips it again and draws them as a batch. Cases: a camera
 inside the geometry (both pipeline forms, 1x and 4x samples), clipped
 triangles interleaved with thousands of small ones in long tile lists,
-the setup-record and sort-binning paths, and the list-overflow path (a
-first frame whose pairs exceed the list storage). The bar is the parity
+the setup-record and sort-binning paths, the list-overflow path (a first
+frame whose pairs exceed the list storage), and room for some of the pieces
+only. The bar is the parity
 suite's: fragment, set-up and clipped counts equal, coverage and depth
 bit-exact, colour within 1 LSB.
 """
@@ -81,3 +83,23 @@ def test_clip_other_paths(driver, monkeypatch, oracle, form, env):
     ctx = Context(driver)
     for s in (g.camera_inside(3000, 300, 192, 128), g.camera_inside(1000, 100, 128, 96, samples=4)):
         check_parity(ctx, oracle, s)
+
+
+@pytest.mark.parametrize("limit", [0, 5, 40])
+@pytest.mark.parametrize("binning", ["gather", "radix"])
+@pytest.mark.parametrize("form", ["balanced", "plain"])
+def test_room_for_some_pieces(driver, monkeypatch, oracle, form, binning, limit):
+    """Lists of pieces' entries, of triangles clipped tile by tile and of
+    small triangles between them, in every tile size the search tries."""
+    from kazan_amd.scenes.renderer import Context
+    monkeypatch.setenv("KAZAN_PIPELINE", form)
+    monkeypatch.setenv("KAZAN_BINNING", binning)
+    monkeypatch.setenv("KAZAN_CLIP_PIECES_LIMIT", str(limit))
+    ctx = Context(driver)
+    for s in (g.camera_inside(3000, 300, 192, 128), g.camera_inside(1000, 100, 128, 96, samples=4)):
+        for frames in (1, 4):
+            _, ost, _ = check_parity(ctx, oracle, s, frames=frames)
+        assert ost["triangles_clipped"] > 20  # (of two pieces and more)
+    monkeypatch.setenv("KAZAN_LIST_CAPACITY_LIMIT", "3000")
+    st, _, _ = check_parity(Context(driver), oracle, g.camera_inside(600, 600, 256, 256), frames=2)
+    assert st["list_overflow"] >= 1
