@@ -454,6 +454,14 @@ typedef enum VkColorComponentFlagBits {
 } VkColorComponentFlagBits;
 typedef VkFlags VkColorComponentFlags;
 
+typedef enum VkCommandPoolResetFlagBits {
+    VK_COMMAND_POOL_RESET_RELEASE_RESOURCES_BIT = 0x1
+} VkCommandPoolResetFlagBits;
+
+typedef enum VkCommandBufferResetFlagBits {
+    VK_COMMAND_BUFFER_RESET_RELEASE_RESOURCES_BIT = 0x1
+} VkCommandBufferResetFlagBits;
+
 typedef enum VkFenceCreateFlagBits {
     VK_FENCE_CREATE_SIGNALED_BIT = 0x1
 } VkFenceCreateFlagBits;

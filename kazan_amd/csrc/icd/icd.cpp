@@ -1045,14 +1045,23 @@ static void reset_cb(CommandBuffer *cb) {
     cb->recording = false;
 }
 
-static void destroy_cb(CommandBuffer *cb) {
-    reset_cb(cb);
-    if (cb->done || !cb->records.empty()) set_device(cb->device);
+// Gives the memory of its recordings back (reset first).
+static void release_records(CommandBuffer *cb) {
+    if (!cb->records.empty()) set_device(cb->device);
     for (DrawRecords &r : cb->records) {
         hipFree(r.dev);
         hipHostFree(r.host);
     }
-    if (cb->done) hipEventDestroy(cb->done);
+    cb->records.clear();
+}
+
+static void destroy_cb(CommandBuffer *cb) {
+    reset_cb(cb);
+    release_records(cb);
+    if (cb->done) {
+        set_device(cb->device);
+        hipEventDestroy(cb->done);
+    }
     delete cb;
 }
 
@@ -1093,8 +1102,11 @@ VKAPI_ATTR void VKAPI_CALL vkDestroyCommandPool(VkDevice, VkCommandPool pool, co
     delete p;
 }
 
-VKAPI_ATTR VkResult VKAPI_CALL vkResetCommandPool(VkDevice, VkCommandPool pool, VkCommandPoolResetFlags) {
-    for (CommandBuffer *cb : from<CommandPool>(pool)->buffers) reset_cb(cb);
+VKAPI_ATTR VkResult VKAPI_CALL vkResetCommandPool(VkDevice, VkCommandPool pool, VkCommandPoolResetFlags flags) {
+    for (CommandBuffer *cb : from<CommandPool>(pool)->buffers) {
+        reset_cb(cb);
+        if (flags & VK_COMMAND_POOL_RESET_RELEASE_RESOURCES_BIT) release_records(cb);
+    }
     return VK_SUCCESS;
 }
 
@@ -1170,8 +1182,10 @@ VKAPI_ATTR VkResult VKAPI_CALL vkEndCommandBuffer(VkCommandBuffer commandBuffer)
     return VK_SUCCESS;
 }
 
-VKAPI_ATTR VkResult VKAPI_CALL vkResetCommandBuffer(VkCommandBuffer commandBuffer, VkCommandBufferResetFlags) {
-    reset_cb(from<CommandBuffer>(commandBuffer));
+VKAPI_ATTR VkResult VKAPI_CALL vkResetCommandBuffer(VkCommandBuffer commandBuffer, VkCommandBufferResetFlags flags) {
+    CommandBuffer *cb = from<CommandBuffer>(commandBuffer);
+    reset_cb(cb);
+    if (flags & VK_COMMAND_BUFFER_RESET_RELEASE_RESOURCES_BIT) release_records(cb);
     return VK_SUCCESS;
 }
 

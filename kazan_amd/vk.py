@@ -582,6 +582,8 @@ _SIGS = {
     "vkDestroyCommandPool": (None, [Handle, Handle, c_void_p]),
     "vkAllocateCommandBuffers": (c_int32, [Handle, P(VkCommandBufferAllocateInfo), P(Handle)]),
     "vkFreeCommandBuffers": (None, [Handle, Handle, c_uint32, P(Handle)]),
+    "vkResetCommandPool": (c_int32, [Handle, Handle, c_uint32]),
+    "vkResetCommandBuffer": (c_int32, [Handle, c_uint32]),
     "vkBeginCommandBuffer": (c_int32, [Handle, P(VkCommandBufferBeginInfo)]),
     "vkEndCommandBuffer": (c_int32, [Handle]),
     "vkCmdBindPipeline": (None, [Handle, c_int32, Handle]),
