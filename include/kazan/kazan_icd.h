@@ -88,7 +88,7 @@ typedef VkResult(VKAPI_PTR *PFN_vkGetDrawStatsKAZAN)(VkDevice device, uint64_t *
 
 /* Kernels of one draw batch, in launch order, for per-kernel timing. */
 enum KazanKernel {
-    KAZAN_KERNEL_CLEAR_COUNTS = 0, /* counter resets */
+    KAZAN_KERNEL_CLEAR_COUNTS = 0, /* reads 0: part of BIN_COUNT */
     KAZAN_KERNEL_BIN_COUNT = 1,    /* vertex shader + setup: pixel boxes */
     KAZAN_KERNEL_BIN_HIST = 2,     /* (triangle, tile) pairs per tile */
     KAZAN_KERNEL_BIN_SCAN = 3,     /* list offsets */

@@ -304,8 +304,10 @@ enum {
 };
 #define KZ_PAIR_PIECE 1024u  // pairs of a chunk that one workgroup writes
 enum {
-    KZ_BIN_PAIRS = 0,  // pairs generated and sorted this batch (<= list capacity)
-    KZ_BIN_CUT = 1,    // first pair chunk whose pairs did not fit (chunks when all fit)
+    // (triangle, tile) pairs of the batch: those sorted (<= list capacity), or
+    // of gather binning all, for the plan's share of a workgroup only
+    KZ_BIN_PAIRS = 0,
+    KZ_BIN_CUT = 1,    // first pair chunk whose pairs did not fit (chunks when all fit); gather binning: 0
     KZ_BIN_OVER = 2,   // 1 when chunks were cut
     KZ_BIN_EXTRA = 3,  // pieces of chunks' pairs after their first
     // clip pieces reserved (past clip_cap: not kept) and triangles with

@@ -143,8 +143,8 @@ struct BatchConfig {
     }
 };
 
-// Autotuning of one batch (balanced form): its first submissions time
-// candidate configurations with HIP events, one candidate per submission;
+// Autotuning of one batch (balanced form): its submissions from the second on
+// time candidate configurations with HIP events, one candidate per submission;
 // then the fastest is kept. Pixels never depend on the choice.
 struct BatchTuning {
     BatchTuning() = default;
@@ -183,7 +183,7 @@ struct Op {
     uint32_t tile_shift = 4;                // the pipeline's default tile size
     std::shared_ptr<BatchTuning> tuning;    // created at the first submission
     KzFrame frame{};                // draws/scratch pointers filled at submit
-    std::vector<KzDraw> draws;      // host copy, uploaded at end of recording
+    std::vector<KzDraw> draws;      // host copy, uploaded at the end of recording or by its first submission
     KzDraw *d_draws = nullptr;      // device copy owned by the command buffer
     uint32_t *d_draw_begin = nullptr;  // the draws' first triangles, in the same allocation
     uint32_t *d_block_draw = nullptr;  // then the draw of each 256-triangle block's first triangle
@@ -200,7 +200,7 @@ struct Op {
 
 // Kernels of a batch, in launch order, for per-kernel timing.
 enum KernelSlot {
-    KS_CLEAR_COUNTS = 0,
+    KS_CLEAR_COUNTS = 0,  // (no launch of its own any more: part of KS_BIN_COUNT; reads 0)
     KS_BIN_COUNT,
     KS_BIN_HIST,
     KS_BIN_SCAN,

@@ -139,12 +139,13 @@ __global__ void kz_fill_u32(uint32_t *dst, uint64_t n, uint32_t value) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = value;
 }
 
-// Fills a rectangle of a W-wide attachment with `spp` 32-bit values per pixel.
-// (a sleep of 127 is 8,128 cycles, about 3.4 us)
+// Keeps the stream busy for about 0.1 ms, in which the host queues what is
+// timed after it (a sleep of 127 is 8,128 cycles, about 3.4 us).
 __global__ void kz_wait() {
     for (int i = 0; i < 30; ++i) __builtin_amdgcn_s_sleep(127);
 }
 
+// Fills a rectangle of a W-wide attachment with `spp` 32-bit values per pixel.
 __global__ void kz_fill_rect_u32(uint32_t *dst, uint32_t width, int32_t x0, int32_t y0, uint32_t w, uint32_t h,
                                  uint32_t spp, uint32_t value) {
     const uint64_t n = (uint64_t)w * h * spp;

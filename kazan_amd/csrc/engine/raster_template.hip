@@ -1403,9 +1403,8 @@ __device__ __forceinline__ void kz_direct(const KzFrame &f, const KzLaneTri &L, 
 
 // The pieces ks + lane of the clip polygon of triangle g0 (one that needs
 // clipping), set up, with their varyings' base and deltas; ok: the lane's
-// piece exists and set up. The whole wave calls it, and only for a batch
-// that starts with such a triangle, so it stays out of line: its
-// temporaries do not weigh on the raster's registers.
+// piece exists and set up. The whole wave calls it: in the raster only for a
+// batch that starts with such a triangle, in a branch of its own.
 struct KzClipBatch {
     KzTri t;
     float a0[KZ_NVA], da1[KZ_NVA], da2[KZ_NVA];
@@ -1781,7 +1780,7 @@ __device__ unsigned long long kz_raster_rect(const KzFrame &f, int32_t X0, int32
         }
         // A triangle that needs clipping (and has no pieces) is drawn as its own batch of
         // pieces (lane j: piece ks + j), in its place: a batch whose first
-        // triangle needs it draws that triangle's pieces (out of line), any
+        // triangle needs it draws that triangle's pieces, any
         // other batch ends before its first such triangle.
         const uint64_t clipm = kz_ballot(clip);
         const bool clip_batch = (clipm & 1ull) != 0;
