@@ -139,10 +139,12 @@ __global__ void kz_fill_u32(uint32_t *dst, uint64_t n, uint32_t value) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = value;
 }
 
-// Keeps the stream busy for about 0.1 ms, in which the host queues what is
-// timed after it (a sleep of 127 is 8,128 cycles, about 3.4 us).
+// Keeps the stream busy for about 34 us (a sleep of 127 is 8,128 cycles, about
+// 3.4 us), in which the host queues what is timed after it: an event and a
+// graph, about 15 us. (At 100 us the trials of a small frame took 13.4 ms, at
+// 34 us 10.5; the same configurations are chosen.)
 __global__ void kz_wait() {
-    for (int i = 0; i < 30; ++i) __builtin_amdgcn_s_sleep(127);
+    for (int i = 0; i < 10; ++i) __builtin_amdgcn_s_sleep(127);
 }
 
 // Fills a rectangle of a W-wide attachment with `spp` 32-bit values per pixel.
