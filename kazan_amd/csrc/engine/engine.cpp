@@ -318,28 +318,33 @@ uint32_t gather_square_cap(uint32_t tris, uint32_t supers) {
 //   size, as a grid's tiles cost them (a cluster's empty squares less);
 // - they do so the longer the denser the triangles, and at larger tiles a
 //   wave walks more of them alone.
-// The line is where it stays ahead of the radix chain (42 to 52 us, or 62 with
-// the model's statistics) in all of a grid, a cluster, 64 meshes and large
-// triangles. Frames, radix us / gather us (grid, cluster, meshes), one
-// configuration each:
-//   16 px tiles: 65,536 triangles at 720p 119/96, 97/94, 97/83 and at 1080p
-//   138/127, 96/91, 109/101; 49,152 at 1440p 169/169, 96/93, 111/104; past the
-//   line 65,536 at 1440p 174/179, 100/102, 117/119, at 4K 261/309, 113/145,
-//   129/150, and in 640x480 (3,277 a square) 101/79, 120/144, 92/74;
-//   8 px: 16,384 in 640x480 99/89, 80/58, 74/57; past it 8,192 at 720p
-//   125/150, 82/71, 85/70 and at 4K 405/644, 149/191, 169/216;
+// The line is about where the radix chain (42 to 52 us) has caught up over a
+// grid, a cluster and 64 meshes. Frames at one tile size, radix us / gather us
+// of the three:
+//   16 px tiles: 65,536 triangles at 720p 119/96, 97/94, 97/83, at 1080p
+//   138/127, 96/91, 109/101, at 1440p 174/179, 100/102, 117/119 and in 640x480
+//   101/79, 120/144, 92/74; past the line at 4K 261/309, 113/145, 129/150 and in
+//   256^2 79/85, 95/121, 68/64;
+//   8 px: 16,384 in 128^2 64/61, 83/81, 56/48 and in 640x480 99/89, 80/58, 74/57;
+//   past it 8,192 at 720p 125/150, 82/71, 85/70 and at 4K 405/644, 149/191,
+//   169/216;
 //   32 px: 32,768 at 720p 132/107, 116/112, 110/92; past it 65,536 146/138,
 //   121/151, 126/116, and 16,384 in 640x480 126/114, 92/103, 75/66;
 //   64 px: 16,384 at 1080p 360/346, 137/134, 127/123; past it 32,768 399/388,
 //   145/159, 143/148.
+// With the tuner's choice of tiles and of the raster, gathering wherever the
+// tables fit against this (grid, cluster, meshes): 65,536 triangles at 4K
+// 275/231, 123/110, 132/126, in 256^2 59/67, 113/96, 42/56 (radix alone up to
+// 73, 100 and 60); the same at 1440p, 1080p, 720p and in 640x480 and below.
 bool gather_pays(uint32_t tris, uint32_t width, uint32_t height, uint32_t shift) {
     const uint64_t supers = (uint64_t)squares(width) * squares(height);
     const uint64_t segs = (tris + KZ_GATHER_SEG - 1) / KZ_GATHER_SEG;
-    static constexpr uint32_t kSquareNs[] = {1400, 96, 24, 8};  // 8 px tiles on
+    static constexpr uint32_t kSquareNs[] = {1560, 96, 24, 8};  // 8 px tiles on
     static_assert(sizeof kSquareNs / sizeof *kSquareNs == kMaxTileShift - kMinTileShift + 1, "a cost per tile size");
     const uint32_t most = shift <= 4 ? kGatherTris : shift == 5 ? kGatherTris / 2 : kGatherTris / 4;
-    return tris <= most && tris <= supers * (shift <= 4 ? 2048 : 640) &&
-           supers * (10 * kSquareNs[shift - kMinTileShift] + 21 * segs) <= 360000;
+    const uint32_t density = shift > 4 ? 640u : shift == 3 && tris <= kGatherTris / 4 ? 16384u : 4096u;
+    return tris <= most && tris <= supers * density &&
+           supers * (10 * kSquareNs[shift - kMinTileShift] + 21 * segs) <= 400000;
 }
 
 // (squares: their totals are summed by every workgroup)
