@@ -2081,9 +2081,10 @@ extern "C" __global__ __launch_bounds__(64) KZ_RASTER_ATTR void kz_raster(KzFram
     // cut chunk on were dropped) draws its list, then the triangles from
     // the cut on by an in-order scan of their pixel boxes; a list past the
     // capacity without a flag (sort binning) is a scan of every triangle.
-    // (An empty tile returns at once unless clears are folded.)
+    // (An empty tile returns at once unless clears are folded; its offset is
+    // any value, radix binning's all ones.)
     const bool cut = f.tile_flag && f.tile_flag[tile];
-    const bool scan = cut || (uint64_t)off + n > (uint64_t)f.list_capacity;
+    const bool scan = cut || (n && (uint64_t)off + n > (uint64_t)f.list_capacity);
     uint32_t lcnt = scan ? 0u : n;
     const uint32_t *lids = f.tile_lists + off;
     if (cut) {
