@@ -313,38 +313,39 @@ uint32_t gather_square_cap(uint32_t tris, uint32_t supers) {
 }  // namespace
 
 // Gather binning's work, where radix binning's grows with the pairs only:
-// - every segment is tested against every square (2.1 ns each);
+// - every segment is tested against every square (3 ns each);
 // - a square's blocks of 8 tiles each read its list: ns per square by tile
-//   size, as a grid's tiles cost them (a cluster's empty squares less);
+//   size, between a grid's (all tiles busy) and a cluster's;
 // - they do so the longer the denser the triangles, and at larger tiles a
 //   wave walks more of them alone.
-// The line is about where the radix chain (42 to 52 us) has caught up over a
-// grid, a cluster and 64 meshes. Frames at one tile size, radix us / gather us
-// of the three:
-//   16 px tiles: 65,536 triangles at 720p 119/96, 97/94, 97/83, at 1080p
-//   138/127, 96/91, 109/101, at 1440p 174/179, 100/102, 117/119 and in 640x480
-//   101/79, 120/144, 92/74; past the line at 4K 261/309, 113/145, 129/150 and in
-//   256^2 79/85, 95/121, 68/64;
-//   8 px: 16,384 in 128^2 64/61, 83/81, 56/48 and in 640x480 99/89, 80/58, 74/57;
-//   past it 8,192 at 720p 125/150, 82/71, 85/70 and at 4K 405/644, 149/191,
-//   169/216;
-//   32 px: 32,768 at 720p 132/107, 116/112, 110/92; past it 65,536 146/138,
-//   121/151, 126/116, and 16,384 in 640x480 126/114, 92/103, 75/66;
-//   64 px: 16,384 at 1080p 360/346, 137/134, 127/123; past it 32,768 399/388,
-//   145/159, 143/148.
-// With the tuner's choice of tiles and of the raster, gathering wherever the
-// tables fit against this (grid, cluster, meshes): 65,536 triangles at 4K
-// 275/231, 123/110, 132/126, in 256^2 59/67, 113/96, 42/56 (radix alone up to
-// 73, 100 and 60); the same at 1440p, 1080p, 720p and in 640x480 and below.
+// The line is where the radix chain (eight launches, 40 to 50 us) has caught up
+// over a grid, a cluster and 64 meshes drawn as one batch and as 64. Frames at
+// one tile size and the plain raster, radix us / gather us of the four:
+//   16 px tiles: 65,536 triangles at 720p 100/77, 81/73, 97/83, 2500/1442, at
+//   1440p 153/158, 81/86, 117/119, 3047/1993, in 640x480 85/64, 112/124, 92/74,
+//   2369/1378, and 8,192 at 4K 199/213, 86/77, 116/105, 3192/2445; past the
+//   line at 4K 65,536 235/280, 95/126, 129/150 (as 64 batches each is within),
+//   and in 256^2 67/71, 199/217, 68/64;
+//   8 px: 8,192 in 640x480 83/76, 61/40, 74/57, 2241/1250, at 720p 104/129,
+//   65/55, 85/70, 2445/1519 (a grid is 15 to 60 us faster at 16 px), 65,536 in
+//   256^2 66/59, 114/116, 70/55, 2197/1226; past it at 1080p 139/213, 75/77,
+//   103/97, at 4K 311/572, 128/163, 169/215, and 65,536 in 128^2 61/62, 92/138;
+//   32 px: 32,768 at 720p 116/92, 93/83, 110/92; past it 65,536 129/122,
+//   126/140, 126/116 and 32,768 in 640x480 126/117, 136/167;
+//   64 px: 8,192 at 1080p 317/304, 91/83; past it 32,768 372/362, 144/150.
+// With the tuner's choice of tiles and raster, gathering wherever the tables
+// fit against this (grid, cluster, meshes): 65,536 triangles at 4K 274/237,
+// 123/96, 132/112, in 256^2 59/59, 114/96, 42/41, in 128^2 50/50, 139/94, 38/45;
+// within 4 % at 1440p, 1080p, 720p and in 640x480 and below.
 bool gather_pays(uint32_t tris, uint32_t width, uint32_t height, uint32_t shift) {
     const uint64_t supers = (uint64_t)squares(width) * squares(height);
     const uint64_t segs = (tris + KZ_GATHER_SEG - 1) / KZ_GATHER_SEG;
-    static constexpr uint32_t kSquareNs[] = {1560, 96, 24, 8};  // 8 px tiles on
+    static constexpr uint32_t kSquareNs[] = {900, 96, 24, 8};  // 8 px tiles on
     static_assert(sizeof kSquareNs / sizeof *kSquareNs == kMaxTileShift - kMinTileShift + 1, "a cost per tile size");
     const uint32_t most = shift <= 4 ? kGatherTris : shift == 5 ? kGatherTris / 2 : kGatherTris / 4;
-    const uint32_t density = shift > 4 ? 640u : shift == 3 && tris <= kGatherTris / 4 ? 16384u : 4096u;
-    return tris <= most && tris <= supers * density &&
-           supers * (10 * kSquareNs[shift - kMinTileShift] + 21 * segs) <= 400000;
+    const uint32_t density = shift > 4 ? 640u : shift == 3 ? 16384u : 4096u;
+    return tris <= most && tris <= std::max<uint64_t>(supers * density, 2048) &&
+           supers * (kSquareNs[shift - kMinTileShift] + 3 * segs) <= 56000;
 }
 
 // (squares: their totals are summed by every workgroup)

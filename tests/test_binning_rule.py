@@ -5,13 +5,14 @@ import pytest
 
 GATHER = [  # triangles, width, height, tile size
     (256, 64, 64, 8), (256, 64, 64, 64), (1024, 256, 256, 8), (1024, 256, 256, 16), (11834, 1023, 575, 16),
-    (65536, 1280, 720, 16), (65536, 1920, 1080, 16), (65536, 2560, 1440, 16), (8192, 3440, 1440, 16),
-    (65536, 640, 480, 16), (65536, 640, 480, 8), (16384, 640, 480, 8), (16384, 128, 128, 8), (32768, 1280, 720, 32), (8192, 3840, 2160, 32), (16384, 1920, 1080, 64),
+    (65536, 1280, 720, 16), (65536, 1920, 1080, 16), (65536, 2560, 1440, 16), (8192, 3840, 2160, 16),
+    (65536, 640, 480, 16), (65536, 640, 480, 8), (65536, 256, 256, 8), (16384, 128, 128, 8), (8192, 1280, 720, 8),
+    (32768, 1280, 720, 32), (8192, 3840, 2160, 32), (2048, 64, 64, 32), (16384, 1920, 1080, 64),
 ]
 RADIX = [
-    (65537, 1280, 720, 16), (65536, 3440, 1440, 16), (8192, 3840, 2160, 16), (65536, 3840, 2160, 16),
-    (8192, 1280, 720, 8), (8192, 3840, 2160, 8), (65536, 256, 256, 16), (65536, 256, 256, 8), (16384, 64, 64, 16),
-    (65536, 1280, 720, 32), (16384, 640, 480, 32), (32768, 1920, 1080, 64), (65536, 4096, 4096, 32),
+    (65537, 1280, 720, 16), (65536, 3440, 1440, 16), (16384, 3840, 2160, 16), (65536, 3840, 2160, 16),
+    (65536, 1280, 720, 8), (8192, 1920, 1080, 8), (65536, 256, 256, 16), (65536, 128, 128, 8), (16384, 64, 64, 16),
+    (65536, 1280, 720, 32), (16384, 640, 480, 32), (32768, 1920, 1080, 64), (1, 16384, 16384, 16),
 ]
 
 

@@ -89,7 +89,7 @@ def test_rule(driver, monkeypatch, oracle):
             if binning:
                 m.setenv("KAZAN_BINNING", binning)
             ctxs[binning] = Context(driver)
-    for n, w, h in ((4096, 128, 128), (4097, 128, 128), (3000, 2048, 2048), (3000, 3840, 2160)):
+    for n, w, h in ((4096, 128, 128), (4097, 128, 128), (3000, 2048, 2048), (3000, 4096, 4096)):
         s = _scene(n, w, h, (0, 0, w, h), size=4.0)
         launches = {b: check_parity(c, oracle, s)[0]["launches"] for b, c in ctxs.items()}
         named = "gather" if driver.lib.kazan_gather_binning(n, w, h, 16) else "radix"
