@@ -4,8 +4,8 @@
 // The cache is the counterpart of the pipeline cache the reference leaves as
 // a stub (vkCreatePipelineCache, vulkan-driver/src/api_impl.rs:3979; nil
 // pipelineCacheUUID :1489-1492): code objects are keyed by a 64-bit FNV-1a
-// hash of all parts of the kernel source and the compile options, stored as
-// <dir>/<hash>.hsaco. The directory is $KAZAN_PIPELINE_CACHE, else
+// hash of all parts of the kernel source, the compile options and the
+// compiler, stored as <dir>/<hash>.hsaco. The directory is $KAZAN_PIPELINE_CACHE, else
 // _pipeline_cache/ beside the driver library.
 #include <dlfcn.h>
 #include <hip/hiprtc.h>
@@ -190,16 +190,30 @@ std::string pipeline_code_dir() { return cache_dir(); }
 
 namespace {
 
+// The compiler of this process. A process that has loaded another ROCm's
+// libraries (PyTorch brings its own) compiles with that one's: its version may
+// read the same, its code is not (the eight-light raster at four samples: 144
+// registers and 3 waves a SIMD from PyTorch's, 128 and 4 from ROCm 7.2's; a 4K
+// frame of it 1600 us and 1410).
+std::string compiler_id() {
+    int major = 0, minor = 0;
+    hiprtcVersion(&major, &minor);
+    std::string id = "hiprtc " + std::to_string(major) + "." + std::to_string(minor);
+    Dl_info info;
+    struct stat st;
+    if (dladdr((void *)&hiprtcCompileProgram, &info) && info.dli_fname && stat(info.dli_fname, &st) == 0)
+        id += std::string(" ") + info.dli_fname + " " + std::to_string((long long)st.st_size);
+    return id;
+}
+
 // The hash of what every source of a kind has in it (`text` and the shared
-// structs) and of the compile options: once per process. (With the whole
+// structs), of the compile options and of the compiler: once per process. (With the whole
 // source hashed and the code object read byte by byte each time, creating a
 // cached pipeline took 0.81 to 1.08 ms, now 0.62 to 0.83.)
 uint64_t fixed_hash(const char *text) {
     std::string s = text;
     for (int i = 0; i < kNumOptions; ++i) s += std::string("\n") + kCompileOptions[i];
-    int rtc_major = 0, rtc_minor = 0;
-    hiprtcVersion(&rtc_major, &rtc_minor);
-    s += "\nhiprtc " + std::to_string(rtc_major) + "." + std::to_string(rtc_minor) + "\n";
+    s += "\n" + compiler_id() + "\n";
     return fnv1a64(kz_src_device_common, sizeof kz_src_device_common, fnv1a64(s.data(), s.size()));
 }
 

@@ -6,6 +6,10 @@ the reference, where it is a stub) for every shader pair and fixed-function
 combination the scene workloads use; the code objects land in the on-disk
 cache that the device path loads from.
 """
+import os
+import subprocess
+import sys
+
 import pytest
 
 from kazan_amd.scenes import generators as g
@@ -89,3 +93,38 @@ def test_occupancy_step_raises_only_without_spills(driver):
     r = _resources(driver, _scenes()["grid_textured_blend"], 4)
     assert r["kz_raster_waves"] >= 5 and r["kz_raster_scratch"] == 0
     assert r["kz_raster_persistent_scratch"] == 0
+
+
+_COMPILE = """
+import sys
+sys.path.insert(0, %r)
+if %r:
+    import torch
+from kazan_amd import vk
+from kazan_amd.scenes import generators as g
+from kazan_amd.scenes.renderer import compile_offline
+rc, msg = compile_offline(vk.Driver(), g.random_triangles(8, 32, 32), 2)
+lib = sorted({ln.split()[-1] for ln in open("/proc/self/maps") if "libhiprtc" in ln})
+print(rc, "cache_hit=1" in msg, lib[0])
+"""
+
+
+def test_cache_tells_compilers_apart(driver, tmp_path):
+    """A process that has loaded PyTorch compiles with PyTorch's ROCm: its code
+    objects are not those of a process without it, nor the other way round."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, KAZAN_PIPELINE_CACHE=str(tmp_path))
+
+    def run(torch):
+        out = subprocess.run([sys.executable, "-c", _COMPILE % (root, torch)], env=env, capture_output=True, text=True,
+                             timeout=300)
+        assert out.returncode == 0, out.stderr
+        rc, hit, lib = out.stdout.split()
+        assert rc == "0"
+        return hit == "True", lib
+
+    hit, lib = run(False)
+    assert not hit
+    torch_hit, torch_lib = run(True)
+    assert torch_hit == (torch_lib == lib)
+    assert run(False) == (True, lib) and run(True) == (True, torch_lib)
