@@ -188,10 +188,9 @@ def main():
                     help="pipeline forms to measure, first = the reported one (%s)" % ",".join(FORMS))
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=50)
-    # the balanced form autotunes over its first (at most) 12 submissions
-    # (one timed candidate each), runs the choice eagerly on the next and
-    # captures the command buffer into a hipGraph on the one after: warm up
-    # past that
+    # the balanced form autotunes over its submissions from the second on (at
+    # most 29, one timed candidate each) and then captures the command buffer
+    # into a hipGraph: measure() submits until it has, then warms up
     ap.add_argument("--warmup", type=int, default=30)
     ap.add_argument("--workload", default="grid_1080p")
     ap.add_argument("--skewed", default="cluster_4m_1080p",

@@ -23,6 +23,9 @@
  *                                vkCreateComputePipelines does (reference
  *                                ComputePipeline::create, vulkan-driver/src/
  *                                pipeline.rs:122-154)
+ *   kazan_compute_launch,        the driver's own rules over given sizes: a
+ *   kazan_gather_binning,        dispatch's launch, a batch's binning, the
+ *   kazan_tune                   search for its configuration
  *
  * All return 0 on success and a negative value on failure, with a message in
  * `out`. Output longer than `cap` is truncated; *out_len receives the full

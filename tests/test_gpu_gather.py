@@ -48,7 +48,7 @@ def _scene(n, w, h, box, size=1.0, large=()):
 @pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 4100])
 def test_segment_edges(mctx, oracle, n):
     s = _scene(n, 256, 128, (0, 0, 256, 128), large=range(0, n, 97))
-    for frames in (1, 2, 3, 4):  # (the balanced form's k-th frame has its k-th tile size)
+    for frames in (1, 2, 3, 4):  # (the balanced form's first frames have its tile sizes, 16, 8, 32, 64 px)
         check_parity(mctx, oracle, s, frames=frames)
 
 

@@ -52,7 +52,7 @@ def _scene(n, large):
     (2049, range(1020, 1030)), (5000, range(1024, 2048)), (5000, range(0, 5000, 40)),
 ])
 def test_pairs_of_large_and_small(rctx, oracle, n, large):
-    for frames in (1, 4):  # (the balanced form's k-th frame has its k-th tile size)
+    for frames in (1, 4):  # (the balanced form's first frames have its tile sizes, 16, 8, 32, 64 px)
         check_parity(rctx, oracle, _scene(n, large), frames=frames)
 
 

@@ -55,6 +55,6 @@ def test_tile_relative_coverage(mctx, oracle, make, samples):
     s = scene_from_pixels(tris, W, H, colors=rng.random((n, 3, 4)), z=rng.random((n, 3)), samples=samples)
     s.blend = (1, g.BLEND_SRC_ALPHA, g.BLEND_ONE_MINUS_SRC_ALPHA, 0, g.BLEND_ONE, g.BLEND_ONE_MINUS_SRC_ALPHA, 0)
     s.scissor = (3, 5, W - 10, H - 6)
-    # (the balanced form draws its k-th frame with the k-th tile size that fits: 8, 16, 32, 64 px)
+    # (the balanced form draws its first frames with its tile sizes: 16, 8, 32 and, where they fit, 64 px)
     for frames in (1, 2, 3, 4):
         check_parity(mctx, oracle, s, frames=frames)
